@@ -194,56 +194,59 @@ int vxm_launch_rmsnorm(vxm_ctx *ctx, float *h, vxm_parts delta, float res_scale,
 // host-computed (cos, sin) of every (position, pair): [position][hd/2].  qkv: raw projections [M][qd + 2*kvd].
 // Tokens come in segments of S (one per CFG branch); token t has position
 // pos0 + t % S and segment t / S, whose cache starts at seg * seg_stride.
+// One thread per pair of neighbouring projection values (a rotary pair of a q or
+// k head, which are stored pair-interleaved: row 2i is dim i, row 2i + 1 dim
+// i + hd / 2; two neighbouring dims of a v head).  Latency-bound: a thread issues
+// the loads of all K-split slices at once and adds them in slice order, and the
+// pairs of one token are spread over workgroups.  (One workgroup per token that
+// walked its pairs and read the slices one after another took 15.0 us at 5 and
+// at 24 tokens of 16 / 2 x 128 heads with 8 slices.)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_rope_kv(const vxm_parts qkv, int nh, int nkv, int hd,
                                                  int pos0, int S, const float2 *__restrict__ cs,
                                                  int no_rope, float *__restrict__ q_out, uint16_t *__restrict__ kc,
                                                  uint16_t *__restrict__ vc, int cap, int64_t seg_stride,
                                                  int cache_pos0) {
-    const int t = blockIdx.x;
+    const int t = blockIdx.x, half = hd / 2, idx = blockIdx.y * blockDim.x + threadIdx.x;
+    if (idx >= (nh + 2 * nkv) * half) return;
+    const int head = idx / half, i = idx % half;   // q heads, then k heads, then v heads
     const int seg = t / S, ti = t % S;
-    const int pos = pos0 + ti;
-    const int half = hd / 2;
-    const int qd = nh * hd, kvd = nkv * hd;
-    const float *row = qkv.p + (int64_t)t * (qd + 2 * kvd);
-    // the projection: its K-split slices added in order
-    auto at = [&](int i) {
-        float v = row[i];
-        for (int z = 1; z < qkv.n; z++) v = v + row[z * qkv.stride + i];
-        return v;
-    };
-    uint16_t *kseg = kc + seg * seg_stride, *vseg = vc + seg * seg_stride;
-    const int cpos = cache_pos0 + ti;
-    // q and k pairs
-    for (int idx = threadIdx.x; idx < (nh + nkv) * half; idx += blockDim.x) {
-        const int head = idx / half, i = idx % half;
-        const bool isq = head < nh;
-        // q and k rows are stored pair-interleaved: head row 2i is dim i, 2i+1 is dim i + hd/2
-        const int src = isq ? head * hd : qd + (head - nh) * hd;
-        float x0 = vxm_bf16(at(src + 2 * i)), x1 = vxm_bf16(at(src + 2 * i + 1));
-        float y0 = x0, y1 = x1;
-        if (!no_rope) {
-            const float2 r = cs[(int64_t)pos * half + i];
-            const float c = r.x, s = r.y;
-            y0 = vxm_bf16(x0 * c - x1 * s);
-            y1 = vxm_bf16(x0 * s + x1 * c);
+    // (nh + 2 nkv) hd and hd are even: the pair is 8-byte aligned
+    const float *src = qkv.p + ((int64_t)t * (nh + 2 * nkv) + head) * hd + 2 * i;
+    float2 part[VXM_MAX_PARTS];
+#pragma unroll
+    for (int z = 0; z < VXM_MAX_PARTS; z++)
+        if (z < qkv.n) part[z] = *(const float2 *)(src + z * qkv.stride);
+    const bool rot = !no_rope && head < nh + nkv;
+    float2 r = make_float2(1.0f, 0.0f);
+    if (rot) r = cs[(int64_t)(pos0 + ti) * half + i];
+    float2 x = part[0];
+#pragma unroll
+    for (int z = 1; z < VXM_MAX_PARTS; z++)
+        if (z < qkv.n) {
+            x.x = x.x + part[z].x;
+            x.y = x.y + part[z].y;
         }
-        if (isq) {
-            float *qo = q_out + (int64_t)t * qd + head * hd;
-            qo[i] = y0;
-            qo[i + half] = y1;
-        } else {
-            const int kh = head - nh;
-            uint16_t *kd = kseg + ((int64_t)kh * cap + cpos) * hd;
-            kd[i] = vxm_f2h(y0);
-            kd[i + half] = vxm_f2h(y1);
-        }
+    const float x0 = vxm_bf16(x.x), x1 = vxm_bf16(x.y);
+    float y0 = x0, y1 = x1;
+    if (rot) {
+        y0 = vxm_bf16(x0 * r.x - x1 * r.y);
+        y1 = vxm_bf16(x0 * r.y + x1 * r.x);
     }
-    // v
-    for (int idx = threadIdx.x; idx < kvd; idx += blockDim.x) {
-        const int kh = idx / hd, dd = idx % hd;
-        const float val = vxm_bf16(at(qd + kvd + idx));
-        vseg[((int64_t)kh * cap + cpos) * hd + dd] = vxm_f2h(val);
+    if (head < nh) {
+        float *qo = q_out + ((int64_t)t * nh + head) * hd;
+        qo[i] = y0;
+        qo[i + half] = y1;
+        return;
+    }
+    const bool is_k = head < nh + nkv;
+    const int kh = is_k ? head - nh : head - nh - nkv;
+    uint16_t *dst = (is_k ? kc : vc) + seg * seg_stride + ((int64_t)kh * cap + cache_pos0 + ti) * hd;
+    if (is_k) {
+        dst[i] = vxm_f2h(y0);
+        dst[i + half] = vxm_f2h(y1);
+    } else {
+        *(uint32_t *)(dst + 2 * i) = (uint32_t)vxm_f2h(y0) | ((uint32_t)vxm_f2h(y1) << 16);
     }
 }
 
@@ -254,8 +257,9 @@ int vxm_launch_rope_kv(vxm_ctx *ctx, vxm_parts qkv, int64_t M, int nh, int nkv, 
     if (!no_rope && (!cs || pos0 + std::min<int64_t>(M, S) > cs_rows))
         return vxm_fail(ctx, VXM_ERR_BACKEND, "rope: table holds %d positions, %lld needed", cs_rows,
                         (long long)(pos0 + std::min<int64_t>(M, S)));
-    hipLaunchKernelGGL(k_rope_kv, dim3((unsigned)M), dim3(256), 0, ctx->stream, qkv, nh, nkv, hd, pos0, S,
-                       cs, no_rope, q_out, kc, vc, cap, seg_stride, cache_pos0);
+    const int pairs = (nh + 2 * nkv) * (hd / 2);
+    hipLaunchKernelGGL(k_rope_kv, dim3((unsigned)M, (unsigned)((pairs + 255) / 256)), dim3(256), 0, ctx->stream, qkv,
+                       nh, nkv, hd, pos0, S, cs, no_rope, q_out, kc, vc, cap, seg_stride, cache_pos0);
     VXM_CHECK_LAUNCH(ctx);
     return VXM_OK;
 }
@@ -266,12 +270,19 @@ int vxm_launch_rope_kv(vxm_ctx *ctx, vxm_parts qkv, int64_t M, int nh, int nkv, 
 // (float)(1/sum)); out = sum_j p_j v_j.  Query head h reads kv head
 // h / (nh / nkv).  Causal: token t of a segment sees cache rows
 // [0, kv_base + t]; non-causal: rows [0, S).  Scores live in LDS (kv_len <= cap).
+// Latency-bound (few tokens, 16 heads): a thread forms whole scores, so it loads
+// its key row 16 bytes at a time, eight loads in flight (hd % 8 == 0; 2 bytes at a
+// time otherwise), and P V keeps eight V loads in flight; the order of every sum
+// is the scalar loop's.  xq != nullptr (hd % 32 == 0): the head's output goes out
+// as Q8_0 blocks instead of fp32, without a launch of its own.
 // ---------------------------------------------------------------------------
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                    const uint16_t *__restrict__ vc, float *__restrict__ out, int nh,
                                                    int nkv, int hd, int cap, int64_t seg_stride, int S,
-                                                   int kv_base, int causal) {
-    extern __shared__ float lds[];
+                                                   int kv_base, int causal, int8_t *__restrict__ xq,
+                                                   uint16_t *__restrict__ xd, int variant) {
+    extern __shared__ __align__(16) float lds[];
     __shared__ float red[8];
     __shared__ double redd[4];
     const int h = blockIdx.x, t = blockIdx.y;
@@ -281,8 +292,8 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
     const uint16_t *kb = kc + seg * seg_stride + (int64_t)kvh * cap * hd;
     const uint16_t *vb = vc + seg * seg_stride + (int64_t)kvh * cap * hd;
     float *sq = lds;              // [hd]
-    float *sc = lds + hd;         // [kv_len]
-    float *part = sc + cap;       // [256]
+    float *part = lds + hd;       // [256]
+    float *sc = part + 256;       // [kv_len]
     const float *qr = q + (int64_t)t * nh * hd + h * hd;
     for (int d = threadIdx.x; d < hd; d += blockDim.x) sq[d] = qr[d];
     __syncthreads();
@@ -291,7 +302,26 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
     for (int j = threadIdx.x; j < kv_len; j += blockDim.x) {
         const uint16_t *kr = kb + (int64_t)j * hd;
         float s = 0.0f;
-        for (int d = 0; d < hd; d++) s += vxm_h2f(kr[d]) * sq[d];
+        if (VEC) {
+            for (int d0 = 0; d0 < hd; d0 += 64) {
+                uint4 kv[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (d0 + 8 * u < hd) kv[u] = *(const uint4 *)(kr + d0 + 8 * u);
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    if (d0 + 8 * u >= hd) break;
+                    const uint32_t w[4] = {kv[u].x, kv[u].y, kv[u].z, kv[u].w};
+                    const float4 qa = *(const float4 *)(sq + d0 + 8 * u), qb = *(const float4 *)(sq + d0 + 8 * u + 4);
+                    const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        s += vxm_h2f((uint16_t)(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu)) * qv[e];
+                }
+            }
+        } else {
+            for (int d = 0; d < hd; d++) s += vxm_h2f(kr[d]) * sq[d];
+        }
         s = s * scale;
         sc[j] = s;
         mx = fmaxf(mx, s);
@@ -315,14 +345,31 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
     if (sl < slices) {
         const int jper = (kv_len + slices - 1) / slices;
         const int j0 = sl * jper, j1 = min(kv_len, j0 + jper);
-        for (int j = j0; j < j1; j++) acc += vxm_h2f(vb[(int64_t)j * hd + d]) * sc[j];
+        int j = j0;
+        for (; j + 8 <= j1; j += 8) {
+            uint16_t v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = vb[(int64_t)(j + u) * hd + d];
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc += vxm_h2f(v[u]) * sc[j + u];
+        }
+        for (; j < j1; j++) acc += vxm_h2f(vb[(int64_t)j * hd + d]) * sc[j];
     }
     part[threadIdx.x] = acc;
     __syncthreads();
+    float tot = 0.0f;
     if (sl == 0) {
-        float tot = 0.0f;
         for (int s2 = 0; s2 < slices; s2++) tot += part[s2 * hd + d];
-        out[(int64_t)t * nh * hd + h * hd + d] = tot;
+        if (!xq) out[(int64_t)t * nh * hd + h * hd + d] = tot;
+    }
+    if (!xq) return;
+    if (sl == 0) sq[d] = tot;   // the query row is done with
+    __syncthreads();
+    if ((int)threadIdx.x < hd / 8) {   // 8 values per thread, 4 threads per block (hd % 32 == 0)
+        const float4 a = *(const float4 *)(sq + 8 * threadIdx.x), b = *(const float4 *)(sq + 8 * threadIdx.x + 4);
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const int64_t e = (int64_t)t * nh * hd + h * hd + 8 * threadIdx.x;
+        quant_block_4lanes(v, variant, xq + e, xd + e / 32, (threadIdx.x & 3) == 0);
     }
 }
 
@@ -886,10 +933,18 @@ int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const
     const size_t lds = (size_t)(hd + cap + 256) * sizeof(float);
     if (lds > 160 * 1024)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "attention: capacity %d exceeds the LDS score buffer", cap);
-    hipLaunchKernelGGL(k_attention, dim3(nh, (unsigned)M), dim3(256), lds, ctx->stream, q, kc, vc, out, nh, nkv,
-                       hd, cap, seg_stride, S, kv_base, causal);
+    // 16-byte key loads need whole 16-byte rows and bases (the caches and the workspace
+    // are 16-byte aligned, their heads and segments whole rows apart)
+    const bool vec = hd % 8 == 0 && !(((uintptr_t)kc | (uintptr_t)vc) & 15) && seg_stride % 8 == 0;
+    int8_t *fq = xq && hd % 32 == 0 ? xq : nullptr;   // a head's columns are whole Q8_0 blocks
+    if (vec)
+        hipLaunchKernelGGL(k_attention<true>, dim3(nh, (unsigned)M), dim3(256), lds, ctx->stream, q, kc, vc, out, nh,
+                           nkv, hd, cap, seg_stride, S, kv_base, causal, fq, xd, variant);
+    else
+        hipLaunchKernelGGL(k_attention<false>, dim3(nh, (unsigned)M), dim3(256), lds, ctx->stream, q, kc, vc, out, nh,
+                           nkv, hd, cap, seg_stride, S, kv_base, causal, fq, xd, variant);
     VXM_CHECK_LAUNCH(ctx);
-    return xq ? vxm_launch_quantize(ctx, out, M, (int64_t)nh * hd, variant, xq, xd) : VXM_OK;
+    return xq && !fq ? vxm_launch_quantize(ctx, out, M, (int64_t)nh * hd, variant, xq, xd) : VXM_OK;
 }
 
 // ---------------------------------------------------------------------------
