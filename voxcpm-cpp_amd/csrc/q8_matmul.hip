@@ -1212,7 +1212,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
 }
 
 // ---------------------------------------------------------------------------
-// Small-M MFMA GEMM (M <= 64: the CFM batch of both CFG branches, LocEnc
+// Small-M MFMA GEMM (M <= 128: the CFM batch of both CFG branches, LocEnc
 // patches, short prompts).  Each weight byte feeds at most 64 products here,
 // so the weight stream sets the time: every weight byte is loaded once, with
 // 16-byte loads, straight into MFMA operand registers; the activations (a few
@@ -1260,8 +1260,8 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
                                                                    int bps, int8_t *__restrict__ sq,
                                                                    uint16_t *__restrict__ sd, int variant,
                                                                    int32_t *__restrict__ dots) {
-    // KG groups of kSmallRG waves split the workgroup's K range in halves (KG = 2) and add
-    // their partial products through LDS at the end; NT = threads per group
+    // KG groups of kSmallRG waves split the workgroup's K range evenly and add their
+    // partial products through LDS at the end, in group order; NT = threads per group
     constexpr int SB = kSmallStage, ROWS = 16 * MT, NT = 64 * kSmallRG;
     __shared__ __align__(16) int8_t xs_all[KG][ROWS * kSmallPitch];
     __shared__ float xds_all[KG][ROWS][SB + 1];
@@ -1277,7 +1277,7 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     int8_t *const xs = xs_all[kg];
     float(*const xds)[SB + 1] = xds_all[kg];
     const int nw = g * 16 * kSmallRG + 16 * wave;
-    // this group's share of the split's K blocks (the plan makes both shares equal)
+    // this group's share of the split's K blocks (the plan makes the shares equal)
     const int zs0 = z * bps, zs1 = min(nb, zs0 + bps), share = (zs1 - zs0) / KG;
     const int zb0 = zs0 + kg * share, zb1 = zb0 + share;
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wq, (short)0, N * K, 0x00020000);
@@ -1401,20 +1401,25 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     }
     if (DOTS) return;
     if (KG > 1) {
-        // group 1 hands its partial products to group 0 (added as group 0 + group 1)
-        __shared__ float kred[kSmallRG][MT * 4][64];
-        if (kg == 1) {
+        // groups 1 .. KG - 1 hand their partial products to group 0, which adds them in
+        // group order; the stage buffers are free once every group is past its products
+        static_assert(sizeof(xs_all) >= sizeof(float) * (KG - 1) * kSmallRG * MT * 4 * 64, "partials over the stages");
+        float(*const kred)[kSmallRG][MT * 4][64] = (float(*)[kSmallRG][MT * 4][64])xs_all;
+        __syncthreads();
+        if (kg > 0) {
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) kred[wave][t * 4 + v][lane] = acc[t][v];
+                for (int v = 0; v < 4; v++) kred[kg - 1][wave][t * 4 + v][lane] = acc[t][v];
         }
         __syncthreads();
         if (kg == 0) {
 #pragma unroll
-            for (int t = 0; t < MT; t++)
+            for (int o = 0; o < KG - 1; o++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) acc[t][v] = acc[t][v] + kred[wave][t * 4 + v][lane];
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[t][v] = acc[t][v] + kred[o][wave][t * 4 + v][lane];
         }
     }
     if (sq) {
@@ -1786,28 +1791,58 @@ constexpr int kSmallPartsMinRows = 2;
 
 // Small-M plan: K splits in whole stages, doubling while the grid leaves CUs
 // idle (at most max_parts).  Shapes outside the kernel's layout (N % 64,
-// K % 256, M > 64, operands of 2 GiB) take the tiled GEMM.
+// K % 256, M > 128, operands of 2 GiB) take the tiled GEMM.
 struct SmallPlan {
     int mt, bps, splits, groups, mtiles, kg;
 };
+
+// Most wave groups whose registers hold a tile of mt 16-row tiles.
+constexpr int small_kg_max(int mt) { return mt <= 2 ? 3 : 2; }
 
 static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_parts, SmallPlan &p) {
     if (M < 1 || M > VXM_SMALL_MAX_ROWS || N % (16 * kSmallRG) || K % (32 * kSmallStage)) return false;
     // 32-bit buffer offsets: the weights, and the activation rows
     if (N * K >= ((int64_t)1 << 31) || VXM_SMALL_MAX_ROWS * K >= ((int64_t)1 << 31)) return false;
     const int nb = (int)(K / 32), stages = nb / kSmallStage;
-    p.mt = (int)((M + 15) / 16);
-    p.mtiles = 1;   // the kernel takes row tiles of 16 MT (blockIdx.z); M <= 64 is one tile
+    // row tiles of 16 mt <= 64 rows (blockIdx.z), about equal
+    p.mtiles = (int)((M + VXM_SMALL_TILE_ROWS - 1) / VXM_SMALL_TILE_ROWS);
+    p.mt = (int)((M + 16 * p.mtiles - 1) / (16 * p.mtiles));
     p.groups = (int)(N / (16 * kSmallRG));
     int s = 1;
     while (s * 2 <= max_parts && s * 2 <= stages && (int64_t)p.groups * p.mtiles * s < ctx->n_cu) s *= 2;
     const int per = (stages + s - 1) / s;   // stages per split
     p.bps = per * kSmallStage;
     p.splits = (nb + p.bps - 1) / p.bps;
-    // two wave groups per workgroup halve each split's serial stage chain when every
-    // split (the last one included) holds an even number of stages
-    p.kg = (per % 2 == 0 && stages % 2 == 0) ? 2 : 1;
+    // Wave groups per workgroup cut each split's serial stage chain (a stage costs one
+    // memory round trip): as many as divide every split's stages, the last split's
+    // included.  Three (a down projection's K = 6144 over 8 splits: one stage per group
+    // instead of three in a row, 7.3 -> 5.6 us at 5 rows, 8.3 -> 6.8 at 24) where the
+    // registers of 12 waves hold the tile; four gained nothing over two at K = 2048
+    // unsplit (11.5 against 11.9 us at 5 rows, 16.4 against 13.5 at 24).
+    p.kg = 1;
+    for (int kg = 2; kg <= small_kg_max(p.mt); kg++)
+        if (per % kg == 0 && stages % kg == 0) p.kg = kg;
     return true;
+}
+
+// The small-M kernel's plan for the product, where it is the one to run: any M it
+// takes up to one row tile; above that (each row tile reads the weights again)
+// where the tile GEMM would split K, whose tag launch, partial words and
+// last-workgroup fix-up cost more than the second read of the weights (M = 77, public
+// entry: 2048 x 2048 15.6 -> 11.5 us, 2048 x 6144 19.7 -> 16.9, 1024 x 4096 17.0 ->
+// 13.1 at M = 100; 12288 x 2048, which the tile GEMM takes unsplit, stays there: 19.0
+// against 28.2).  With a fix-up launch of its own (the public entries) only where its
+// grid is one round: 2560 x 2048, 320 workgroups, 16.6 against 15.7 us at M = 100.  With
+// three row tiles (M > 128) it loses: 2048 x 6144 30.1 against 23.4 us at M = 150.  K is
+// bounded there so that the slices and the quantized rows of any such product fit the
+// allocation-free entry's scratch together.
+static bool small_wins(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
+                       int max_parts, bool fixup, SmallPlan &p) {
+    if (!small_plan(ctx, M, w->n, w->k, max_parts, p)) return false;
+    if (M <= VXM_SMALL_TILE_ROWS) return true;
+    if (fixup && (int64_t)p.groups * p.mtiles * p.splits > ctx->n_cu) return false;
+    GemmPlan t;
+    return w->k <= 16384 && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
 }
 
 static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
@@ -1818,7 +1853,10 @@ static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, co
 #define VXM_SMALL_ARGS xq, xd, w->qs, w->d, y, (int)M, N, K, p.bps, sq, sd, variant, dots
 #define VXM_SMALL_KG(MT, D)                                                                                \
     do {                                                                                                   \
-        if (p.kg == 2)                                                                                     \
+        if (p.kg == 3)                                                                                     \
+            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, small_kg_max(MT), D>), grid, block, 0, ctx->stream,  \
+                               VXM_SMALL_ARGS);                                                            \
+        else if (p.kg == 2)                                                                                \
             hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 2, D>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
         else                                                                                               \
             hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 1, D>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
@@ -1877,7 +1915,7 @@ int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
     if (M <= 0) return VXM_OK;
     SmallPlan sp;
     const bool small = (ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows)) &&
-                       small_plan(ctx, M, w->n, w->k, max_parts < VXM_MAX_PARTS ? max_parts : VXM_MAX_PARTS, sp);
+                       small_wins(ctx, w, xq, xd, M, max_parts < VXM_MAX_PARTS ? max_parts : VXM_MAX_PARTS, false, sp);
     if (!small) return vxm_launch_mul_mat(ctx, w, xq, xd, M, y);
     launch_small(ctx, w, xq, xd, M, y, sp);
     VXM_CHECK_LAUNCH(ctx);
@@ -1898,7 +1936,7 @@ bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *
     const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
     if (!mfma || M <= 0 || N % 64) return false;
     SmallPlan sp;
-    if (small_plan(ctx, M, N, K, 1, sp)) {
+    if (M <= VXM_SMALL_TILE_ROWS && small_plan(ctx, M, N, K, 1, sp)) {
         // unsplit: each workgroup holds whole 32-pair blocks over all of K
         launch_small(ctx, w, xq, xd, M, nullptr, sp, sq, sd, variant);
     } else {
@@ -1922,7 +1960,7 @@ static bool use_mfma(const vxm_ctx *ctx, int64_t M);
 bool vxm_launch_qkv_rope(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                          const vxm_qkv_epi &qe, int cs_rows, int *rc) {
     *rc = VXM_OK;
-    if (M <= VXM_SMALL_MAX_ROWS || !use_mfma(ctx, M) || ctx->path == VXM_PATH_MFMA_TILED || !qe.q_out) return false;
+    if (M <= VXM_SMALL_TILE_ROWS || !use_mfma(ctx, M) || ctx->path == VXM_PATH_MFMA_TILED || !qe.q_out) return false;
     const int64_t N = w->n;
     if (qe.hd % 4 || N != (int64_t)(qe.nh + 2 * qe.nkv) * qe.hd || qe.S <= 0) return false;
     if (!gemm_fits(M, (int)N, (int)w->k)) return false;
@@ -1986,7 +2024,7 @@ static int launch_mul_mat(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, c
     if (M <= 0) return VXM_OK;
     if (use_mfma(ctx, M)) {
         SmallPlan sp;
-        if (ctx->path != VXM_PATH_MFMA_TILED && small_plan(ctx, M, w->n, w->k, VXM_MAX_PARTS, sp))
+        if (ctx->path != VXM_PATH_MFMA_TILED && small_wins(ctx, w, xq, xd, M, VXM_MAX_PARTS, true, sp))
             return launch_gemm_small(ctx, w, xq, xd, M, y, sp, wk);
         return launch_gemm(ctx, w, xq, xd, M, y, wk);
     }
@@ -2006,7 +2044,7 @@ static int launch_block_dots(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
                              int32_t *out) {
     if (use_mfma(ctx, M)) {
         SmallPlan sp;
-        if (ctx->path != VXM_PATH_MFMA_TILED && small_plan(ctx, M, w->n, w->k, VXM_MAX_PARTS, sp)) {
+        if (ctx->path != VXM_PATH_MFMA_TILED && small_wins(ctx, w, xq, xd, M, VXM_MAX_PARTS, true, sp)) {
             launch_small(ctx, w, xq, xd, M, nullptr, sp, nullptr, nullptr, 0, out);
         } else {
             const int N = (int)w->n, K = (int)w->k;

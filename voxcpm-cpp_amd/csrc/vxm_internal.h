@@ -190,7 +190,8 @@ struct vxm_parts {
 };
 __host__ __device__ inline vxm_parts vxm_one_part(const float *p) { return vxm_parts{p, 1, 0}; }
 
-constexpr int VXM_SMALL_MAX_ROWS = 64;   // rows of x the small-M GEMM takes
+constexpr int VXM_SMALL_MAX_ROWS = 128;  // rows of x the small-M GEMM takes
+constexpr int VXM_SMALL_TILE_ROWS = 64;  // of them in one row tile
 constexpr int VXM_MAX_PARTS = 8;         // its K splits
 
 // The product as up to max_parts slices of M x N at y, y + M*N, ...; *parts = the
