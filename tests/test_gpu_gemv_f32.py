@@ -1,0 +1,53 @@
+"""The GEMV that quantizes its fp32 rows itself equals quantization and GEMV in launches of their
+own bit for bit: every K that has a chunked kernel, the generic one, ragged row counts, the largest
+row count it takes, both quantizers, zero and non-finite blocks, and an output over the input."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _host(ctx, t):
+    ctx.sync()   # the library works on its own stream
+    return t.cpu().numpy()
+
+
+@pytest.mark.parametrize("N,K,M", [(64, 1024, 1), (1001, 1024, 5), (512, 2048, 1), (2051, 2048, 3), (2048, 4096, 2),
+                                   (1023, 6144, 1), (3, 6144, 5), (2048, 512, 5), (1024, 64, 4), (5, 32, 1),
+                                   (7, 3072, 5)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_fused_gemv_equals_two_launches(vxm_ctx, orc, N, K, M, variant):
+    import torch
+
+    rng = np.random.default_rng(N + K + M)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    x[0, :32] = 0.0
+    x[-1, -1] = 3e38
+    w = vxm_ctx.upload_q8_0(orc.quantize_rows(rng.normal(0, 0.02, (N, K)).astype(np.float32), orc.QUANT_REF), N, K)
+    xd = torch.from_numpy(x).to("cuda:0")
+    torch.cuda.synchronize()
+    vxm_ctx.set_quant_variant(variant)
+    try:
+        y = _host(vxm_ctx, vxm_ctx.mul_mat(w, xd))
+    finally:
+        vxm_ctx.set_quant_variant(1)
+    ref = _host(vxm_ctx, vxm_ctx.mul_mat_q8(w, *vxm_ctx.quantize_q8_0(xd, variant)))
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+    w.free()
+
+
+def test_output_over_the_input(vxm_ctx, orc):
+    """y over x: no workgroup may read a row that another has overwritten."""
+    import torch
+
+    rng = np.random.default_rng(3)
+    n = 2048
+    w = vxm_ctx.upload_q8_0(orc.quantize_rows(rng.normal(0, 0.02, (n, n)).astype(np.float32), orc.QUANT_REF), n, n)
+    x = torch.from_numpy(rng.normal(0, 1, (2, n)).astype(np.float32)).to("cuda:0")
+    torch.cuda.synchronize()
+    for rows in (1, 2):
+        ref = _host(vxm_ctx, vxm_ctx.mul_mat_q8(w, *vxm_ctx.quantize_q8_0(x[:rows], 1)))
+        y = x[:rows].clone()
+        torch.cuda.synchronize()
+        assert np.array_equal(_host(vxm_ctx, vxm_ctx.mul_mat(w, y, y)), ref)
+    w.free()

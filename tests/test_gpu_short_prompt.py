@@ -26,8 +26,10 @@ def test_small_gemm_row_tiles_and_wave_groups(vxm_ctx, orc, N, K, M):
     ref = orc.mul_mat_f64(wq, xq_ref, N, K, M)
     try:
         vxm_ctx.set_path(vxm.PATH_MFMA)
-        y = vxm_ctx.mul_mat_q8(w, xq, xd).cpu().numpy()
-        assert np.array_equal(vxm_ctx.block_dots(w, xq, xd).cpu().numpy(), orc.block_dots(wq, xq_ref, N, K, M))
+        y, dots = vxm_ctx.mul_mat_q8(w, xq, xd), vxm_ctx.block_dots(w, xq, xd)
+        vxm_ctx.sync()
+        y = y.cpu().numpy()
+        assert np.array_equal(dots.cpu().numpy(), orc.block_dots(wq, xq_ref, N, K, M))
     finally:
         vxm_ctx.set_path(vxm.PATH_AUTO)
     err = np.abs(y - ref)

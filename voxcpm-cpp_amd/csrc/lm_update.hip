@@ -18,6 +18,10 @@
 
 #include "vxm_model.h"
 
+// Patches whose in_proj k_locenc_assemble forms itself: its row of x in LDS, and few
+// rows, since every row's workgroup reads the whole weight.
+constexpr int kLocEncFuseFeat = 256, kLocEncFuseRows = 64;
+
 struct vxm_locenc {
     vxm_ctx *ctx = nullptr;
     vxm_locenc_config cfg{};
@@ -62,18 +66,44 @@ struct vxm_lm_update {
 // ---------------------------------------------------------------------------
 // LocEnc sequence (src/locenc.c:55-85): row 0 the special token when there is
 // one, then in_proj(x) + bias, all F32 (no BF16 here in the reference).
-__global__ void k_locenc_assemble(float *__restrict__ seq, const float *__restrict__ special,
-                                  const float *__restrict__ xh, const float *__restrict__ xb, int H) {
-    const int row = blockIdx.x, off = special ? 1 : 0;
+// xh != nullptr: the projection's rows, formed by launches of their own.  Else the
+// workgroup of a row quantizes its x (feat values) and forms the projection itself:
+// for a patch's few rows of 64 values three dependent launches (quantization,
+// product, this one) are mostly gaps (an encoder call of 5 rows 303 -> 300 us, of 13 rows 354 -> 349).
+__global__ __launch_bounds__(256) void k_locenc_assemble(float *__restrict__ seq, const float *__restrict__ special,
+                                                         const float *__restrict__ xh, const float *__restrict__ x,
+                                                         const int8_t *__restrict__ wq,
+                                                         const uint16_t *__restrict__ wd, int feat, int variant,
+                                                         const float *__restrict__ xb, int H) {
+    __shared__ __align__(16) int8_t q[kLocEncFuseFeat];
+    __shared__ uint16_t qd[kLocEncFuseFeat / 32];
+    const int row = blockIdx.x, off = special ? 1 : 0, nb = feat / 32;
     float *dst = seq + (int64_t)row * H;
-    for (int i = threadIdx.x; i < H; i += blockDim.x) {
-        float v;
-        if (row < off) {
-            v = special[i];
-        } else {
-            v = xh[(int64_t)(row - off) * H + i];
-            if (xb) v = v + xb[i];
+    if (row < off) {
+        for (int i = threadIdx.x; i < H; i += blockDim.x) dst[i] = special[i];
+        return;
+    }
+    if (!xh) {
+        if ((int)threadIdx.x < feat / 8) {   // 8 values per thread, 4 threads per block
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = x[(int64_t)(row - off) * feat + 8 * threadIdx.x + e];
+            quant_block_4lanes(v, variant, q + 8 * threadIdx.x, qd + threadIdx.x / 4, (threadIdx.x & 3) == 0);
         }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < H; i += blockDim.x) {
+        float v = 0.0f;
+        if (xh) {
+            v = xh[(int64_t)(row - off) * H + i];
+        } else {
+            for (int b = 0; b < nb; b++) {
+                const int4 *w = (const int4 *)(wq + ((int64_t)i * nb + b) * 32), *a = (const int4 *)(q + 32 * b);
+                const int s = vxm_dot16(w[1], a[1], vxm_dot16(w[0], a[0], 0));
+                v += (float)s * (vxm_h2f(wd[(int64_t)i * nb + b]) * vxm_h2f(qd[b]));
+            }
+        }
+        if (xb) v = v + xb[i];
         dst[i] = v;
     }
 }
@@ -128,6 +158,24 @@ __global__ void k_embed_rows_q8_0(const int8_t *__restrict__ qs, const uint16_t 
 }
 
 static unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+// One row's projection with e's bias, FSQ and copies: one launch, or (a forced matmul
+// path) quantization, product and e's work in launches of their own.
+static int project_row(vxm_ctx *ctx, const vxm_weight *w, const float *x, int8_t *aq, uint16_t *ad,
+                       const vxm_gemv_epi &e) {
+    int rc;
+    if (vxm_launch_gemv_f32(ctx, w, x, 1, ctx->quant_variant, e, &rc)) return rc;
+    if ((rc = vxm_launch_quantize(ctx, x, 1, w->k, ctx->quant_variant, aq, ad))) return rc;
+    if ((rc = vxm_launch_mul_mat(ctx, w, aq, ad, 1, e.y))) return rc;
+    if (e.fsq_scale > 0.0f)
+        hipLaunchKernelGGL(k_fsq, dim3(grid_of(w->n)), dim3(256), 0, ctx->stream, e.y, e.bias, e.y, w->n, e.fsq_scale,
+                           e.fsq_inv);
+    else if (e.bias || e.y2)
+        hipLaunchKernelGGL(k_bias_add, dim3(grid_of(w->n)), dim3(256), 0, ctx->stream, e.y, e.bias, e.y, e.y2, w->n);
+    VXM_CHECK_LAUNCH(ctx);
+    if (e.y3) VXM_HIP(ctx, hipMemcpyAsync(e.y3, e.y, w->n * 4, hipMemcpyDeviceToDevice, ctx->stream));
+    return VXM_OK;
+}
 
 int vxm_upload_vec(vxm_ctx *ctx, const float *src, int64_t n, float **out) {
     *out = nullptr;
@@ -243,9 +291,13 @@ extern "C" int vxm_locenc_forward(vxm_locenc *m, const float *x_dev, int32_t P, 
     if ((rc = vxm_ws_ensure(ctx, m->ws, S, H, qd, kvd, d.F, (int64_t)d.nkv * S * d.hd))) return rc;
     if ((rc = vxm_rope_ensure(ctx, m->dims, S))) return rc;
     if ((rc = locenc_bufs(m, S, P))) return rc;
-    if ((rc = vxm_launch_quantize(ctx, x_dev, P, m->cfg.feat_dim, var, m->aq, m->ad))) return rc;
-    if ((rc = vxm_launch_mul_mat(ctx, m->in_proj, m->aq, m->ad, P, m->xh))) return rc;
-    hipLaunchKernelGGL(k_locenc_assemble, dim3((unsigned)S), dim3(256), 0, ctx->stream, m->seq, m->special, m->xh,
+    const bool fuse_in = m->cfg.feat_dim <= kLocEncFuseFeat && P <= kLocEncFuseRows && ctx->path == VXM_PATH_AUTO;
+    if (!fuse_in) {
+        if ((rc = vxm_launch_quantize(ctx, x_dev, P, m->cfg.feat_dim, var, m->aq, m->ad))) return rc;
+        if ((rc = vxm_launch_mul_mat(ctx, m->in_proj, m->aq, m->ad, P, m->xh))) return rc;
+    }
+    hipLaunchKernelGGL(k_locenc_assemble, dim3((unsigned)S), dim3(256), 0, ctx->stream, m->seq, m->special,
+                       fuse_in ? nullptr : m->xh, x_dev, m->in_proj->qs, m->in_proj->d, (int)m->cfg.feat_dim, var,
                        m->in_bias, (int)H);
     VXM_CHECK_LAUNCH(ctx);
     // bidirectional blocks over the S fresh rows, positions 0..S-1, no cache
@@ -399,40 +451,31 @@ extern "C" int vxm_lm_update_step(vxm_lm_update *u, vxm_kv_cache *tslm_kv, vxm_k
     if (!prev_patch_dev || !base_hidden_dev || !ralm_hidden_dev || !tslm_kv || !ralm_kv || pos < 0)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "lm_update: bad patch / outputs / caches / pos");
     const int64_t L = u->cfg.lm_hidden, Fq = u->fsq_in ? u->cfg.fsq_dim : 0;
-    const int var = ctx->quant_variant;
     float *fsq_part = u->cat, *audio_part = u->cat + L;
     int rc;
     // audio embedding (src/gen_step.c:208-266)
     if ((rc = vxm_locenc_forward(u->enc, prev_patch_dev, P, u->fe))) return rc;
-    if ((rc = vxm_launch_quantize(ctx, u->fe, 1, u->cfg.enc_hidden, var, u->aq, u->ad))) return rc;
-    if ((rc = vxm_launch_mul_mat(ctx, u->enc_to_lm, u->aq, u->ad, 1, audio_part))) return rc;
-    hipLaunchKernelGGL(k_bias_add, dim3(grid_of(L)), dim3(256), 0, ctx->stream, audio_part, u->enc_to_lm_bias,
-                       audio_part, base_hidden_dev, L);
-    VXM_CHECK_LAUNCH(ctx);
-    if (audio_embed_dev)
-        VXM_HIP(ctx, hipMemcpyAsync(audio_embed_dev, audio_part, L * 4, hipMemcpyDeviceToDevice, ctx->stream));
+    if ((rc = project_row(ctx, u->enc_to_lm, u->fe, u->aq, u->ad,
+                          vxm_gemv_epi{audio_part, base_hidden_dev, audio_embed_dev, u->enc_to_lm_bias})))
+        return rc;
     // TSLM step at pos, in place on base_hidden (src/gen_step.c:741-771)
     if ((rc = vxm_minicpm4_forward(u->tslm, tslm_kv, base_hidden_dev, 1, pos))) return rc;
     // FSQ (src/gen_step.c:268-290), or the hidden unchanged without one
     if (Fq > 0) {
-        if ((rc = vxm_launch_quantize(ctx, base_hidden_dev, 1, L, var, u->aq, u->ad))) return rc;
-        if ((rc = vxm_launch_mul_mat(ctx, u->fsq_in, u->aq, u->ad, 1, u->fh))) return rc;
-        hipLaunchKernelGGL(k_fsq, dim3(grid_of(Fq)), dim3(256), 0, ctx->stream, u->fh, u->fsq_in_bias, u->fh, Fq,
-                           u->cfg.fsq_quant_scale, u->inv_scale);
-        VXM_CHECK_LAUNCH(ctx);
-        if ((rc = vxm_launch_quantize(ctx, u->fh, 1, Fq, var, u->aq, u->ad))) return rc;
-        if ((rc = vxm_launch_mul_mat(ctx, u->fsq_out, u->aq, u->ad, 1, fsq_part))) return rc;
-        hipLaunchKernelGGL(k_bias_add, dim3(grid_of(L)), dim3(256), 0, ctx->stream, fsq_part, u->fsq_out_bias,
-                           fsq_part, fsq_dev, L);
-        VXM_CHECK_LAUNCH(ctx);
+        if ((rc = project_row(ctx, u->fsq_in, base_hidden_dev, u->aq, u->ad,
+                              vxm_gemv_epi{u->fh, nullptr, nullptr, u->fsq_in_bias, u->cfg.fsq_quant_scale,
+                                           u->inv_scale})))
+            return rc;
+        if ((rc = project_row(ctx, u->fsq_out, u->fh, u->aq, u->ad,
+                              vxm_gemv_epi{fsq_part, fsq_dev, nullptr, u->fsq_out_bias})))
+            return rc;
     } else {
         VXM_HIP(ctx, hipMemcpyAsync(fsq_part, base_hidden_dev, L * 4, hipMemcpyDeviceToDevice, ctx->stream));
         if (fsq_dev)
             VXM_HIP(ctx, hipMemcpyAsync(fsq_dev, base_hidden_dev, L * 4, hipMemcpyDeviceToDevice, ctx->stream));
     }
     // RALM input = fusion_concat_proj([fsq ; audio_embed]) (src/gen_step.c:870-899), then the RALM step
-    if ((rc = vxm_launch_quantize(ctx, u->cat, 1, 2 * L, var, u->aq, u->ad))) return rc;
-    if ((rc = vxm_launch_mul_mat(ctx, u->fusion, u->aq, u->ad, 1, ralm_hidden_dev))) return rc;
+    if ((rc = project_row(ctx, u->fusion, u->cat, u->aq, u->ad, vxm_gemv_epi{ralm_hidden_dev}))) return rc;
     return vxm_minicpm4_forward(u->ralm, ralm_kv, ralm_hidden_dev, 1, pos);
 }
 

@@ -36,21 +36,14 @@ __device__ __forceinline__ float pair_sum(float v) {
 // VARIANT 0 (quantize_row_q8_0_ref): id = d ? 1/d : 0, q = roundf(x*id).
 // d = amax/127 is stored as fp16 (RNE).
 // ---------------------------------------------------------------------------
+// The calling lane's 4 values of a block (the 8 lanes of the block together, all of them
+// active): its packed quants, and the block's scale in every lane.
 template <int VARIANT>
-__global__ __launch_bounds__(256) void k_quantize_q8_0(const float *__restrict__ x, int64_t nblocks,
-                                                       int8_t *__restrict__ xq,
-                                                       uint16_t *__restrict__ xd) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t blk = t >> 3;
-    const int sub = threadIdx.x & 7;
-    const bool live = blk < nblocks;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) v = *(const float4 *)(x + blk * 32 + sub * 4);
+__device__ __forceinline__ uint32_t quant_block_8lanes(const float4 v, float &d) {
     float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
     amax = vxm_quad_max(amax);   // xor 1, xor 2 on DPP; then the other quad of the 8
     amax = fmaxf(amax, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), 0x141, 0xF, 0xF, false)));
-    if (!live) return;
-    const float d = __fdiv_rn(amax, 127.0f);
+    d = __fdiv_rn(amax, 127.0f);
     float id;
     if (VARIANT == VXM_QUANT_X86) id = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
     else id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
@@ -62,8 +55,23 @@ __global__ __launch_bounds__(256) void k_quantize_q8_0(const float *__restrict__
     } else {
         q0 = roundf(v.x * id); q1 = roundf(v.y * id); q2 = roundf(v.z * id); q3 = roundf(v.w * id);
     }
-    const uint32_t packed = ((uint32_t)(uint8_t)(int8_t)(int)q0) | ((uint32_t)(uint8_t)(int8_t)(int)q1 << 8) |
-                            ((uint32_t)(uint8_t)(int8_t)(int)q2 << 16) | ((uint32_t)(uint8_t)(int8_t)(int)q3 << 24);
+    return ((uint32_t)(uint8_t)(int8_t)(int)q0) | ((uint32_t)(uint8_t)(int8_t)(int)q1 << 8) |
+           ((uint32_t)(uint8_t)(int8_t)(int)q2 << 16) | ((uint32_t)(uint8_t)(int8_t)(int)q3 << 24);
+}
+
+template <int VARIANT>
+__global__ __launch_bounds__(256) void k_quantize_q8_0(const float *__restrict__ x, int64_t nblocks,
+                                                       int8_t *__restrict__ xq,
+                                                       uint16_t *__restrict__ xd) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t blk = t >> 3;
+    const int sub = threadIdx.x & 7;
+    const bool live = blk < nblocks;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (live) v = *(const float4 *)(x + blk * 32 + sub * 4);
+    float d;
+    const uint32_t packed = quant_block_8lanes<VARIANT>(v, d);
+    if (!live) return;
     *(uint32_t *)(xq + blk * 32 + sub * 4) = packed;
     if (sub == 0) xd[blk] = vxm_f2h(d);
 }
@@ -96,16 +104,18 @@ int vxm_launch_quantize(vxm_ctx *ctx, const float *x, int64_t M, int64_t K, int 
 // DOTS = true writes the exact int32 block sums this kernel forms (after the
 // lane-pair exchange) to dots[(m*N + n)*(K/32) + b] instead of y.
 // ---------------------------------------------------------------------------
-template <int C, int R, bool DOTS>
+// prep() runs once the weight loads are out (the fused kernel forms its
+// activation there, with a barrier: every wave of the workgroup gets to it);
+// store(i, row, v) writes output i = m * N + row.
+template <int C, int R, bool DOTS, typename Prep, typename Store>
 __device__ __forceinline__ void gemv_wave(const int8_t *__restrict__ qs, const uint16_t *__restrict__ dg,
                                           const int8_t *__restrict__ xq, const uint16_t *__restrict__ xd,
-                                          float *__restrict__ y, int N, int M, int32_t *__restrict__ dots,
-                                          int wave) {
+                                          int N, int M, int32_t *__restrict__ dots,
+                                          int wave, Prep prep, Store store) {
     constexpr int K = C * 1024;
     constexpr int NB = K / 32;
     const int lane = threadIdx.x & 63;
     const int row0 = wave * R;
-    if (row0 >= N) return;
     const int pair = lane >> 1;
 
     v4i wv[R][C];
@@ -124,6 +134,8 @@ __device__ __forceinline__ void gemv_wave(const int8_t *__restrict__ qs, const u
 #pragma unroll
         for (int c = 0; c < C; c++) dw[r][c] = vxm_h2f(__builtin_nontemporal_load(drow + c));
     }
+    prep();
+    if (row0 >= N) return;
     for (int m = 0; m < M; m++) {
         v4i xv[C];
         float xs[C];
@@ -162,7 +174,7 @@ __device__ __forceinline__ void gemv_wave(const int8_t *__restrict__ qs, const u
         if (lane == 0) {
 #pragma unroll
             for (int r = 0; r < R; r++)
-                if (row0 + r < N) y[(int64_t)m * N + row0 + r] = acc[r];
+                if (row0 + r < N) store((int64_t)m * N + row0 + r, row0 + r, acc[r]);
         }
     }
 }
@@ -173,7 +185,60 @@ __global__ __launch_bounds__(256) void k_gemv_q8_0(const int8_t *__restrict__ qs
                                                    const int8_t *__restrict__ xq,
                                                    const uint16_t *__restrict__ xd, float *__restrict__ y,
                                                    int N, int M, int32_t *__restrict__ dots) {
-    gemv_wave<C, R, DOTS>(qs, dg, xq, xd, y, N, M, dots, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    gemv_wave<C, R, DOTS>(qs, dg, xq, xd, N, M, dots, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), [] {},
+                          [&](int64_t i, int, float v) { y[i] = v; });
+}
+
+// ---------------------------------------------------------------------------
+// The GEMV of an fp32 activation of few rows: k_quantize_q8_0's arithmetic inside
+// the GEMV's launch, each workgroup quantizing the rows into its LDS while its
+// weight loads are in flight, and the per-wave code of the GEMV on them, so the
+// outputs are bit-identical to the two launches'.  A launch costs its caller
+// ~3.4 us of host time and the device a gap of ~1.5 us, against the ~0.3 us
+// (K = 2048) to 0.9 us (K = 6144) that a workgroup's own quantization takes per
+// row.  e: what else is done with an output (vxm_gemv_epi).
+// ---------------------------------------------------------------------------
+template <int VARIANT>
+__device__ __forceinline__ void quantize_lds(float4 v, int i, int8_t *xq, uint16_t *xd) {
+    float d;
+    const uint32_t packed = quant_block_8lanes<VARIANT>(v, d);
+    *(uint32_t *)(xq + 4 * i) = packed;
+    if ((i & 7) == 0) xd[i >> 3] = vxm_f2h(d);
+}
+
+__device__ __forceinline__ void gemv_store(const vxm_gemv_epi &e, int64_t i, int row, float v) {
+    if (e.bias) v = v + e.bias[row];
+    if (e.fsq_scale > 0.0f) v = roundf(tanhf(v) * e.fsq_scale) * e.fsq_inv;
+    e.y[i] = v;
+    if (e.y2) e.y2[i] = v;
+    if (e.y3) e.y3[i] = v;
+}
+
+template <int C, int R, int VARIANT>
+__global__ __launch_bounds__(256) void k_gemv_f32(const int8_t *__restrict__ qs, const uint16_t *__restrict__ dg,
+                                                  const float *__restrict__ x, int N, int M, const vxm_gemv_epi e) {
+    constexpr int K = C * 1024;
+    extern __shared__ __align__(16) int8_t gx[];   // quants [M][K], then scales [M][K / 32]
+    uint16_t *gd = (uint16_t *)(gx + M * K);
+    float4 v[C];   // the first row, loaded ahead of the weights
+#pragma unroll
+    for (int c = 0; c < C; c++) v[c] = *(const float4 *)(x + 4 * (c * 256 + threadIdx.x));
+    gemv_wave<C, R, false>(
+        qs, dg, gx, gd, N, M, nullptr, blockIdx.x * 4 + (threadIdx.x >> 6),
+        [&] {
+            for (int m = 0; m < M; m++) {
+#pragma unroll
+                for (int c = 0; c < C; c++)
+                    quantize_lds<VARIANT>(v[c], c * 256 + threadIdx.x, gx + m * K, gd + m * (K / 32));
+                if (m + 1 < M) {
+#pragma unroll
+                    for (int c = 0; c < C; c++)
+                        v[c] = *(const float4 *)(x + (int64_t)(m + 1) * K + 4 * (c * 256 + threadIdx.x));
+                }
+            }
+            vxm_lds_barrier();
+        },
+        [&](int64_t i, int row, float a) { gemv_store(e, i, row, a); });
 }
 
 // ---------------------------------------------------------------------------
@@ -210,7 +275,8 @@ __global__ __launch_bounds__(256) void k_gemv_q8_0_multi(const GemvBatch b, int 
         else hi = mid - 1;
     }
     const GemvItem &t = b.it[lo];
-    gemv_wave<C, R, false>(t.qs, t.dg, t.xq, t.xd, t.y, t.n, M, nullptr, (bid - t.wg0) * 4 + (threadIdx.x >> 6));
+    gemv_wave<C, R, false>(t.qs, t.dg, t.xq, t.xd, t.n, M, nullptr, (bid - t.wg0) * 4 + (threadIdx.x >> 6), [] {},
+                           [&](int64_t i, int, float v) { t.y[i] = v; });
 }
 
 // ---------------------------------------------------------------------------
@@ -265,16 +331,11 @@ __global__ __launch_bounds__(256) void k_stream_read(const ReadBatch b, uint32_t
 // row's 16-byte half blocks (the two halves of a block sit in lanes 2p, 2p+1).
 // DOTS = true writes the int32 block sums instead (as k_gemv_q8_0).
 // ---------------------------------------------------------------------------
-template <bool DOTS>
-__global__ __launch_bounds__(256) void k_gemv_q8_0_generic(const int8_t *__restrict__ qs,
-                                                           const uint16_t *__restrict__ d,
-                                                           const int8_t *__restrict__ xq,
-                                                           const uint16_t *__restrict__ xd,
-                                                           float *__restrict__ y, int N, int K, int M,
-                                                           int32_t *__restrict__ dots) {
+template <bool DOTS, typename Store>
+__device__ __forceinline__ void gemv_row(const int8_t *__restrict__ qs, const uint16_t *__restrict__ d,
+                                         const int8_t *__restrict__ xq, const uint16_t *__restrict__ xd, int N, int K,
+                                         int M, int row, int32_t *__restrict__ dots, Store store) {
     const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (row >= N) return;
     const int nh = K / 16, nb = K / 32;
     const int8_t *wrow = qs + (int64_t)row * K;
     const uint16_t *drow = d + (int64_t)row * nb;
@@ -301,8 +362,36 @@ __global__ __launch_bounds__(256) void k_gemv_q8_0_generic(const int8_t *__restr
         }
         if (DOTS) continue;
         acc = pair_sum(acc);
-        if (lane == 0) y[(int64_t)m * N + row] = acc;
+        if (lane == 0) store((int64_t)m * N + row, row, acc);
     }
+}
+
+template <bool DOTS>
+__global__ __launch_bounds__(256) void k_gemv_q8_0_generic(const int8_t *__restrict__ qs,
+                                                           const uint16_t *__restrict__ d,
+                                                           const int8_t *__restrict__ xq,
+                                                           const uint16_t *__restrict__ xd,
+                                                           float *__restrict__ y, int N, int K, int M,
+                                                           int32_t *__restrict__ dots) {
+    const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= N) return;
+    gemv_row<DOTS>(qs, d, xq, xd, N, K, M, row, dots, [&](int64_t i, int, float v) { y[i] = v; });
+}
+
+// ... of an fp32 activation (as k_gemv_f32).
+template <int VARIANT>
+__global__ __launch_bounds__(256) void k_gemv_f32_generic(const int8_t *__restrict__ qs,
+                                                          const uint16_t *__restrict__ d,
+                                                          const float *__restrict__ x, int N, int K, int M,
+                                                          const vxm_gemv_epi e) {
+    extern __shared__ __align__(16) int8_t gx[];
+    uint16_t *gd = (uint16_t *)(gx + M * K);
+    // M K / 4 is a multiple of 8: the lanes of a block run the same iterations
+    for (int i = threadIdx.x; i < M * K / 4; i += 256) quantize_lds<VARIANT>(*(const float4 *)(x + 4 * i), i, gx, gd);
+    vxm_lds_barrier();
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= N) return;
+    gemv_row<false>(qs, d, gx, gd, N, K, M, row, nullptr, [&](int64_t i, int r, float v) { gemv_store(e, i, r, v); });
 }
 
 
@@ -750,21 +839,6 @@ static size_t tile_lds_bytes(int tm, int tn, int bps) {
 
 static int tile_max_bps(int tm) { return tm == 128 ? TileCfg<128, 128>::MaxBps : TileCfg<64, 64>::MaxBps; }
 
-// 16 bytes per lane from src into LDS at lds_base + 16 lane.
-__device__ __forceinline__ void lds_dma16(uint32_t lds_base, const void *src) {
-    const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_base);
-    uint32_t saved_m0;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %2, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved_m0)
-        : "s"(m0v), "v"(src)
-        : "memory");
-}
-
 // 16 bytes per lane of lanes 0..7 only (exec = 0xff), into LDS at lds_base + 16 lane.
 __device__ __forceinline__ void lds_dma16_8(uint32_t lds_base, const void *src) {
     const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_base);
@@ -811,12 +885,6 @@ __device__ __forceinline__ void vm_wait_stages(int stages) {
     else vm_wait<0>();
 }
 
-__device__ __forceinline__ void ring_barrier() {   // orders LDS only: loads in flight stay in flight
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <int TM, int TN, bool DOTS>
 __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
     const int8_t *__restrict__ xq, const uint16_t *__restrict__ xd, const int8_t *__restrict__ wq,
@@ -852,7 +920,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
     for (int i = wave; i < (TM / 64) * (P + 1); i += 8) {
         const int f = 64 * i + lane, row = f / (P + 1), pc = f % (P + 1);
         const int r = min(m0 + row, M - 1), q = pc < P ? pc : 0;
-        lds_dma16(ring_lds + kTileSlots * C::Slot + 1024 * i, xd + (int64_t)r * nb + b0 + 8 * q);
+        vxm_lds_dma16(ring_lds + kTileSlots * C::Slot + 1024 * i, xd + (int64_t)r * nb + b0 + 8 * q);
     }
     // this wave's loads of stage st: operand instruction i < LoadsAB is instruction
     // wave * LoadsAB + i of the stage's A | B rows; i == LoadsAB is the wave's
@@ -866,7 +934,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
             const int pg = (lane % C::R16) ^ C::swz(rr);
             const int8_t *src = rr < TM ? xq + (int64_t)min(m0 + rr, M - 1) * K
                                         : wq + (int64_t)min(n0 + rr - TM, N - 1) * K;
-            lds_dma16(base + q * 1024, src + kb0 * 32 + pg * 16);
+            vxm_lds_dma16(base + q * 1024, src + kb0 * 32 + pg * 16);
         } else {
             // 16-byte piece p = 8 wave + lane of the stage's 1 KiB: 64-row group
             // p >> 5 (TN = 128) or 4-block step p >> 5 (TN = 64), rows 2 (p & 31) ..
@@ -927,7 +995,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
     for (int st = 0; st < kTileSlots - 1; st++)
         if (st < ns) issue(st);
     vm_wait_stages<L>(min(2, ns - 1));
-    ring_barrier();   // the panel and stage 0 are in LDS
+    vxm_lds_barrier();   // the panel and stage 0 are in LDS
 
     // Block pipeline: X = the first block of a pair, Y = its second (a wave takes
     // PAIRS pairs of every stage).  Each MFMA is followed by a third of the
@@ -1015,7 +1083,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
             // stage st + 1 has landed once at most the stages after it remain in flight
             vm_wait_stages<L>(min(2, ns - 2 - st));
             VXM_TILE_TS(st, 2);
-            ring_barrier();   // every wave's part of stage st + 1 is visible; slot st is free
+            vxm_lds_barrier();   // every wave's part of stage st + 1 is visible; slot st is free
             VXM_TILE_TS(st, 3);
         }
     }
@@ -2019,6 +2087,56 @@ static bool use_mfma(const vxm_ctx *ctx, int64_t M) {
            (ctx->path == VXM_PATH_AUTO && M >= kMfmaMinRows);
 }
 
+// The fused GEMV's range: one row, or up to five while the values that all workgroups
+// quantize together (each of them the M rows) cost less than the launch saved.
+// Measured (us a call, fused against two launches): one row 4.0 / 7.3 (6144 x 2048), 4.5 /
+// 7.0 (2048 x 6144), 5.5 / 7.0 (12288 x 2048); 3 rows of 6144 x 2048 (4.7 M values) 6.2 /
+// 7.4, 4 rows (6.3 M) 7.6 / 7.2; 2 rows of 12288 x 2048 (6.3 M) 7.8 / 7.2; 5 rows of 1024 x
+// 1024 7.2 / 7.3, 7 rows 9.2 / 8.2.
+constexpr int kGemvF32MaxRows = 5, kGemvF32MaxLds = 48 * 1024;
+constexpr int64_t kGemvF32MaxValues = 5 << 20;
+
+template <int C, int R>
+static void launch_gemv_f32_c(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant, unsigned lds,
+                              const vxm_gemv_epi &e) {
+    const dim3 grid((unsigned)((w->n + 4 * R - 1) / (4 * R)));
+    if (variant == VXM_QUANT_X86)
+        hipLaunchKernelGGL((k_gemv_f32<C, R, VXM_QUANT_X86>), grid, dim3(256), lds, ctx->stream, w->qs, w->dg, x,
+                           (int)w->n, (int)M, e);
+    else
+        hipLaunchKernelGGL((k_gemv_f32<C, R, VXM_QUANT_REF>), grid, dim3(256), lds, ctx->stream, w->qs, w->dg, x,
+                           (int)w->n, (int)M, e);
+}
+
+bool vxm_launch_gemv_f32(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant,
+                         const vxm_gemv_epi &e, int *rc) {
+    *rc = VXM_OK;
+    const int64_t K = w->k, lds = M * K + M * (K / VXM_QK) * 2;
+    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || lds > kGemvF32MaxLds) return false;
+    // an output over the input: workgroups would still read rows that others have written
+    const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)M * K * sizeof(float);
+    for (const float *o : {e.y, e.y2, e.y3})
+        if (o && (uintptr_t)o < x1 && (uintptr_t)o + (size_t)M * w->n * sizeof(float) > x0) return false;
+    const int c = w->dg ? (int)(K / 1024) : 0;
+    const int64_t wg_rows = c == 1 ? 16 : c == 2 ? 8 : 4;   // rows of a workgroup: 4 waves of R
+    if (M > 1 && M * K * ((w->n + wg_rows - 1) / wg_rows) > kGemvF32MaxValues) return false;
+    if (c == 1) launch_gemv_f32_c<1, 4>(ctx, w, x, M, variant, (unsigned)lds, e);
+    else if (c == 2) launch_gemv_f32_c<2, 2>(ctx, w, x, M, variant, (unsigned)lds, e);
+    else if (c == 4) launch_gemv_f32_c<4, 1>(ctx, w, x, M, variant, (unsigned)lds, e);
+    else if (c == 6) launch_gemv_f32_c<6, 1>(ctx, w, x, M, variant, (unsigned)lds, e);
+    else {
+        const dim3 grid((unsigned)((w->n + 3) / 4));
+        if (variant == VXM_QUANT_X86)
+            hipLaunchKernelGGL(k_gemv_f32_generic<VXM_QUANT_X86>, grid, dim3(256), (unsigned)lds, ctx->stream, w->qs,
+                               w->d, x, (int)w->n, (int)K, (int)M, e);
+        else
+            hipLaunchKernelGGL(k_gemv_f32_generic<VXM_QUANT_REF>, grid, dim3(256), (unsigned)lds, ctx->stream, w->qs,
+                               w->d, x, (int)w->n, (int)K, (int)M, e);
+    }
+    if (hipGetLastError() != hipSuccess) *rc = vxm_fail(ctx, VXM_ERR_BACKEND, "GEMV launch failed");
+    return true;
+}
+
 static int launch_mul_mat(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                           float *y, const MmWork *wk) {
     if (M <= 0) return VXM_OK;
@@ -2103,6 +2221,7 @@ extern "C" int vxm_mul_mat_q8_0(vxm_ctx *ctx, const vxm_weight *w, const float *
                                 float *y_dev) {
     int rc = check_mm(ctx, w, x_dev, x_dev, M, y_dev);
     if (rc) return rc;
+    if (vxm_launch_gemv_f32(ctx, w, x_dev, M, ctx->quant_variant, vxm_gemv_epi{y_dev}, &rc)) return rc;
     const int64_t K = w->k;
     const size_t qbytes = ((size_t)M * K + 255) & ~(size_t)255;
     rc = vxm_ensure_act(ctx, qbytes + (size_t)M * (K / VXM_QK) * 2);

@@ -176,11 +176,47 @@ __device__ __forceinline__ float vxm_wave_max(float v) {
     return v;
 }
 
+// 16 bytes per lane from src into LDS at lds_base + 16 lane.
+__device__ __forceinline__ void vxm_lds_dma16(uint32_t lds_base, const void *src) {
+    const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds_base);
+    uint32_t saved_m0;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %2, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved_m0)
+        : "s"(m0v), "v"(src)
+        : "memory");
+}
+
+// Waits for every load of this wave, DMA included.
+__device__ __forceinline__ void vxm_vm_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+__device__ __forceinline__ void vxm_lds_barrier() {   // orders LDS only: loads in flight stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---- host-side launch helpers implemented per translation unit ------------
 int vxm_launch_quantize(vxm_ctx *ctx, const float *x, int64_t M, int64_t K, int variant,
                         int8_t *xq, uint16_t *xd);
 int vxm_launch_mul_mat(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd,
                        int64_t M, float *y);
+// What the fused GEMV does with output row `row`: v + bias[row], then with
+// fsq_scale > 0 the FSQ core of it (k_fsq's arithmetic: round(tanh(v) * scale) *
+// fsq_inv), into y and, where given, y2 and y3.
+struct vxm_gemv_epi {
+    float *y, *y2 = nullptr, *y3 = nullptr;
+    const float *bias = nullptr;
+    float fsq_scale = 0.0f, fsq_inv = 0.0f;
+};
+// The GEMV of fp32 rows x with their quantization in the same launch.  Returns false
+// without launching where vxm_launch_quantize + vxm_launch_mul_mat have to run.
+bool vxm_launch_gemv_f32(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant,
+                         const vxm_gemv_epi &e, int *rc);
 // A matmul output held as n fp32 slices `stride` elements apart whose sum, added in
 // slice order, is the product (the small-M GEMM's K splits, left for the consumer).
 struct vxm_parts {
