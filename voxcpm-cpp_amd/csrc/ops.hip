@@ -377,530 +377,301 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
 // The same attention for many queries of one segment (prefill), on f16 MFMA
 // (v_mfma_f32_32x32x16_f16: lane l supplies A[l%32][8(l/32)..+8] and
 // B[8(l/32)..+8][l%32]; result register v of lane l is row 8(v/4) + 4(l/32)
-// + v%4, column l%32).  One workgroup of 8 waves (2 per SIMD) per (query
-// head, tile of AQ = 32 consecutive tokens).  Every phase is a chain of
-// dependent loads and products, so the work is cut into as many independent
-// chains as the waves:
-//   scores  S = Q K^T * scale, the tile's 32-key blocks of [0, kv_end) split
-//           into 8 contiguous runs, one per wave.  The queries are BF16 values
-//           and the cache holds f16, both exact in f16, so every product is
-//           exact and only the fp32 summation order differs from the
-//           reference's.  A lane's B operands (16 bytes of a key row) come
-//           straight from the cache; every load of a wave (Q, K and its V
-//           rows) is issued at once;
-//   softmax per query row over its own kv_len, on the scores in registers
-//           (computed as S^T = K Q^T, so a lane holds 16 keys of one query per
-//           block): max over the lane's keys, its partner lane's and the 8
-//           waves', e = expf(s - max), sums in double the same way, p = e *
-//           (float)(1 / sum), 0 past kv_len;
-//   output  wave (kq, dh) = (w % 4, w / 4) forms the partial P V of key quarter
-//           kq for dims [64 dh, 64 dh + 64): P enters the MFMA as f16 hi + lo
-//           halves (two products, ~22 bits of p), V through the wave's own LDS
-//           buffer, transposed as key-pair words; the four key quarters are
-//           added in order at the end.
-// The score buffer holds AKV keys: longer spans take k_attention_mfma_long.
+// + v%4, column l%32).  One workgroup takes a tile of AQ = 32 consecutive tokens
+// and NH query heads of one kv head; wave (hh, sp) = (w % NH, w / NH) takes head hh
+// and every fourth 32-key block (block 4 r + sp in round r), so a wave runs its
+// scores, softmax and P V without another wave's data:
+//   scores  S^T = K Q^T * scale: the key rows are the A operands (LDS), the
+//           queries the B operands (registers), so a lane holds 16 keys of one
+//           query.  The queries are BF16 values and the cache holds f16, both
+//           exact in f16, so every product is exact and only the fp32 summation
+//           order differs from the reference's;
+//   softmax with a running max m per query and wave: e = expf(s - m), the sums of e
+//           in double, both in registers (one exchange with lane l ^ 32, the other
+//           half of the query's keys); when m rises, O and the sum are rescaled by
+//           expf(m_old - m) (skipped while no query's m rises);
+//   output  O^T = V^T P^T: the lane's 16 e values are its B operands as they are.
+//           A contraction may take its keys in any order that both operands share,
+//           so V^T is stored with the 16 keys of a step in the order in which the
+//           lane halves hold them (0-3, 8-11 | 4-7, 12-15).  P enters as f16 hi +
+//           lo halves (two products, ~22 bits of e).
+// Each round's 128 key rows go to LDS by DMA and its V rows through registers,
+// transposed as key-pair words, both one round ahead into the other half of the
+// LDS, for one barrier per round.  At the end the four waves of a head merge in
+// block order: m = max, weights expf(m_i - m), o = sum(w_i O_i) * (float)(1 / sum(w_i
+// l_i)), the sums l in double, and the output goes out as Q8_0 or fp32.
+// Every row below is at least one cache line and consecutive lanes take consecutive
+// pieces of it.  The LDS is swizzled: 16-byte piece p of key row r at p ^ swz(r), 4-word
+// piece p of V^T row d at p ^ ((d ^ d >> 3) & 15), so an operand read of 16 lanes and a
+// transposing write of 64 fall on (nearly) distinct banks.
+//
+// Bound by the VALU work per score (max, exp, the double sum, the hi / lo split: ~16
+// instructions) and the matrix products next to it, two waves per SIMD, and by what a
+// wave waits while its loads queue at the address unit.  The tiles with the most keys
+// are launched first.  Measured on 16 / 2 heads x 128, causal: 2048 tokens 57 us, 1000
+// tokens 28, 512 tokens 16, 256 tokens 11.  (A workgroup per head whose eight waves split
+// each 512-key chunk, with the scores' exponentials through LDS, two barriers and a
+// drained load queue per chunk, took 134 and 46 us at 2048 and 1000 tokens; one pass over
+// at most 512 keys that way 17 us.)  Variants: the V loads issued after the scores 63 us at
+// 2048 tokens, two chains of score products 58.5, the max followed exactly (a rescale in
+// almost every block) with a general expf and separate masks 74.
 // ---------------------------------------------------------------------------
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr int AQ = 32, AKV = 512, ATH = 512;
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+constexpr int AQ = 32;
+// A query's running max follows its scores only when one exceeds it by more than this:
+// e then stays below e^8, far inside f16's range and no less precise relative to the
+// sum, and the rescale of O is rare instead of due in almost every block (any of a
+// wave's 32 queries may have a new max).
+constexpr float kMaxSlack = 8.0f;
 
-#ifdef VXM_ATTN_TRACE
-// per-workgroup timestamps (s_memtime) of wave 0: [workgroup][entry, scores, softmax, P V, end]
-__device__ uint64_t vxm_attn_trace[4096 * 8];
-#define VXM_ATTN_TS(k)                                                                                        \
-    do {                                                                                                      \
-        if (tid == 0 && blockIdx.x * gridDim.y + blockIdx.y < 4096)                                           \
-            vxm_attn_trace[(blockIdx.x * gridDim.y + blockIdx.y) * 8 + (k)] = __builtin_amdgcn_s_memtime(); \
-    } while (0)
-extern "C" int vxm_attn_trace_read(void *host, size_t bytes) {   // profiling builds only
-    return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(vxm_attn_trace), bytes, 0, hipMemcpyDeviceToHost);
+// exp(x) as 2^(x log2 e): v_exp_f32 (1 ulp) of the product's leading part, its rounding
+// error and log2 e's added as a first-order factor (they are below 2^-17).  No range
+// reduction: results below 2^-126 are 0, which no sum of e with a largest term near 1
+// notices.  exp_near(-inf) = 0, NaN stays NaN.
+__device__ __forceinline__ float exp_near(float x) {
+    const float L = 1.44269502f, Lo = 1.92596299e-8f;   // log2 e in two parts
+    const float ph = x * L;
+    const float pl = fmaxf(__builtin_fmaf(x, Lo, __builtin_fmaf(x, L, -ph)), -1.0f);   // -inf - -inf is no error
+    const float e = __builtin_amdgcn_exp2f(ph);
+    return __builtin_fmaf(e, pl * 0.693147182f, e);
 }
-#else
-#define VXM_ATTN_TS(k) \
-    do {               \
-    } while (0)
-#endif
 
-template <int HD>
-__global__ __launch_bounds__(ATH) void k_attention_mfma(const float *__restrict__ q, const uint16_t *__restrict__ kc,
-                                                        const uint16_t *__restrict__ vc, float *__restrict__ out,
-                                                        int M, int nh, int nkv, int cap, int kv_base, int causal,
-                                                        int8_t *__restrict__ xq, uint16_t *__restrict__ xd,
-                                                        int variant) {
-    constexpr int NW = ATH / 64;       // waves
-    constexpr int SP = AKV + 4;        // fp32 P row pitch
-    constexpr int KSTEPS = HD / 16;    // MFMA steps over the head dimension
-    constexpr int HDH = HD / 2;        // dims of one output half
-    constexpr int DT = HDH / 32;       // 32-dim output tiles per wave
-    constexpr int VP = 32 + 8;         // f16 pitch of a wave's transposed V block (32 keys + pad)
-    constexpr int VITEMS = 16 * (HDH / 8) / 64;   // (key pair, 8-dim chunk) items per lane and block
-    constexpr int SB = AKV / 32 / NW;  // most score blocks of one wave
-    constexpr int VB = AKV / 32 / 4;   // most P V blocks of one key quarter
-    __shared__ __align__(16) float Sc[AQ * SP];
-    __shared__ __align__(16) _Float16 Vt[NW][HDH * VP];
-    __shared__ float smax[AQ][NW];
-    __shared__ double ssum[AQ][NW];
-    constexpr int QP = HD + 8;         // f16 pitch of the query tile (16-byte pad)
-    __shared__ __align__(16) _Float16 Qh[AQ * QP];
-    static_assert(NW == 8 && VITEMS >= 1 && 4 * AQ * HD <= AQ * SP, "8 waves; the key-quarter sums reuse P's buffer");
-    const int h = blockIdx.x, t0 = blockIdx.y * AQ, tid = threadIdx.x, lane = tid & 63;
+template <int HD, int NH>
+__global__ __launch_bounds__(256 * NH, 1) void k_attention_mfma(
+    const float *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,
+    float *__restrict__ out, int M, int nh, int nkv, int cap, int kv_base, int causal, int8_t *__restrict__ xq,
+    uint16_t *__restrict__ xd, int variant) {
+    constexpr int NS = 4, KB = 32 * NS;        // key splits, keys of a round
+    constexpr int NT = 256 * NH, NW = NT / 64;
+    constexpr int KSTEPS = HD / 16;            // MFMA steps over the head dimension
+    constexpr int DT = HD / 32;                // 32-dim output tiles
+    constexpr int R16 = HD / 8;                // 16-byte pieces of a key or value row
+    constexpr int KBytes = KB * HD * 2, Slot = 2 * KBytes;
+    constexpr int KI = KBytes / 1024 / NW;     // DMA instructions per wave and round
+    constexpr int VI = (KB / 2) * R16 / NT;    // (key pair, 8-dim piece) items per thread and round
+    __shared__ __align__(1024) int8_t lds[2 * Slot];
+    __shared__ float sm[NH][NS][32];
+    __shared__ double sl[NH][NS][32];
+    static_assert(NW * DT * 16 * 64 * 4 <= 2 * Slot, "the merge reuses the key and value rows");
+    static_assert(KI >= 1 && VI >= 1 && (R16 == 8 || R16 == 16), "whole instructions");
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kvh = h / (nh / nkv);
+    const int hh = wave % NH, sp = wave / NH, h = blockIdx.x * NH + hh;
+    const int t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * AQ;
+    const int kvh = (blockIdx.x * NH) / (nh / nkv);
     const uint16_t *kb = kc + (int64_t)kvh * cap * HD;
     const uint16_t *vb = vc + (int64_t)kvh * cap * HD;
     const int nq = min(AQ, M - t0);
     const int kv_end = causal ? kv_base + t0 + nq : M;
+    const int kv_all = causal ? kv_base + t0 + 1 : M;                    // keys that every live query sees
+    const int kvl = lr < nq ? (causal ? kv_base + t0 + lr + 1 : M) : 0;  // keys of query t0 + lr
     const float scale = __fdiv_rn(1.0f, __fsqrt_rn((float)HD));
-    const int lr = lane & 31, lh = lane >> 5;
-    const int nblk = (kv_end + 31) / 32;
-    const int bw0 = nblk * wave / NW, nbw = nblk * (wave + 1) / NW - bw0;   // this wave's score blocks
-    const int kq = wave & 3, dh = wave >> 2;
-    const int bq0 = nblk * kq / 4, nbq = nblk * (kq + 1) / 4 - bq0;        // its P V blocks
-    VXM_ATTN_TS(0);
+    const int nblk = (kv_end + 31) / 32, nr = (nblk + NS - 1) / NS;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+    auto kswz = [](int r) { return R16 == 8 ? (r & 7) ^ ((r >> 3) & 1) : r & 15; };
 
-    // loads in the order they are needed: the query tile (once per workgroup, 4 values
-    // per thread and round, into LDS as f16) and the rows of the wave's score blocks'
-    // keys (A operands: 16 bytes of key 32 b + lr's row per step); after the scores, the
-    // V rows of its P V blocks (item (key pair p, dims 8c .. 8c+7 of its half), p = item
-    // % 16 fastest).
-    // Every load is unconditional (rows past the span, and blocks past a wave's share,
-    // read the clamped last row, whose values are masked or multiplied by p = 0), so the
-    // loads stay in one straight-line block and each product waits only for its own.
-    constexpr int QL = AQ * HD / 4 / ATH;   // float4 query loads per thread
-    float4 qf[QL];
+    uint4 vr[VI][2];
+    // round r's key rows into its slot, its value rows into registers; rows past the span
+    // read the clamped last row (their scores are masked, their e zero)
+    auto load = [&](int r) {
+        const int k0 = KB * r;
 #pragma unroll
-    for (int u = 0; u < QL; u++) {
-        const int i = (u * ATH + tid) * 4, r = i / HD, d = i % HD;
-        qf[u] = *(const float4 *)(q + (int64_t)(t0 + min(r, nq - 1)) * nh * HD + h * HD + d);
-    }
-    uint4 kr[SB][KSTEPS];
-#pragma unroll
-    for (int i = 0; i < SB; i++) {
-        const int key = min(32 * (bw0 + i) + lr, kv_end - 1);
-#pragma unroll
-        for (int kk = 0; kk < KSTEPS; kk++) kr[i][kk] = *(const uint4 *)(kb + (int64_t)key * HD + 16 * kk + 8 * lh);
-    }
-#pragma unroll
-    for (int u = 0; u < QL; u++) {
-        const int i = (u * ATH + tid) * 4, r = i / HD, d = i % HD;
-        const bool qlive = r < nq;
-        _Float16 *dst = Qh + r * QP + d;
-        dst[0] = (_Float16)(qlive ? qf[u].x : 0.0f);
-        dst[1] = (_Float16)(qlive ? qf[u].y : 0.0f);
-        dst[2] = (_Float16)(qlive ? qf[u].z : 0.0f);
-        dst[3] = (_Float16)(qlive ? qf[u].w : 0.0f);
-    }
-    __syncthreads();
-
-    // pass 1: scores of this wave's blocks in registers, as S^T = K Q^T (the key rows are
-    // the A operands, the queries the B operands): value v of block i in lane (lr, lh) is
-    // query t0 + lr, key 32 (bw0 + i) + kr(v) with kr(v) = 8 (v / 4) + 4 lh + v % 4
-    v8h qa[KSTEPS];   // B operands: query t0 + lr, dims 16 kk + 8 lh .. + 8
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; kk++) qa[kk] = *(const v8h *)(Qh + lr * QP + 16 * kk + 8 * lh);
-    v16f sc[SB];
-#pragma unroll
-    for (int i = 0; i < SB; i++) {
-        v16f c = v16f{};
-#pragma unroll
-        for (int kk = 0; kk < KSTEPS; kk++) {
-            v8h av;
-            __builtin_memcpy(&av, &kr[i][kk], 16);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, qa[kk], c, 0, 0, 0);
+        for (int i = 0; i < KI; i++) {
+            const int in = wave * KI + i, row = in * (64 / R16) + lane / R16;
+            const int pc = (lane % R16) ^ kswz(row);
+            vxm_lds_dma16(lds0 + (r & 1) * Slot + in * 1024, kb + (int64_t)min(k0 + row, kv_end - 1) * HD + 8 * pc);
         }
 #pragma unroll
-        for (int v = 0; v < 16; v++) sc[i][v] = c[v] * scale;
-    }
-    // the V rows of the wave's P V blocks, in flight during the softmax
-    const uint16_t *vbh = vb + HDH * dh;
-    uint4 vr[VB][VITEMS][2];
-#pragma unroll
-    for (int i = 0; i < VB; i++)
-#pragma unroll
-        for (int u = 0; u < VITEMS; u++) {
-            const int item = u * 64 + lane, r = 32 * (bq0 + i) + 2 * (item % 16), d = 8 * (item / 16);
+        for (int u = 0; u < VI; u++) {
+            const int item = u * NT + tid, c = item % R16, p = item / R16;
 #pragma unroll
             for (int e = 0; e < 2; e++)
-                vr[i][u][e] = *(const uint4 *)(vbh + (int64_t)min(r + e, kv_end - 1) * HD + d);
-        }
-    VXM_ATTN_TS(1);
-    // pass 2: softmax of query t0 + lr over its kv_len: max over the lane's keys, its
-    // partner lane's (lr + 32: the other half of every block) and the 8 waves' (through
-    // LDS); e = exp(s - max), the double sums the same way; p = e * (float)(1 / sum),
-    // 0 past kv_len
-    const int kvl = lr < nq ? (causal ? kv_base + t0 + lr + 1 : M) : 0;
-    auto live = [&](int i, int v) { return i < nbw && 32 * (bw0 + i) + 8 * (v >> 2) + 4 * lh + (v & 3) < kvl; };
-    float m = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < SB; i++)
-#pragma unroll
-        for (int v = 0; v < 16; v++)
-            if (live(i, v)) m = fmaxf(m, sc[i][v]);
-    m = fmaxf(m, __shfl_xor(m, 32));
-    if (lh == 0) smax[lr][wave] = m;
-    __syncthreads();
-    m = smax[lr][0];
-#pragma unroll
-    for (int w = 1; w < NW; w++) m = fmaxf(m, smax[lr][w]);
-    double sum = 0.0;
-#pragma unroll
-    for (int i = 0; i < SB; i++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const float e = live(i, v) ? expf(sc[i][v] - m) : 0.0f;
-            sc[i][v] = e;
-            sum += (double)e;
-        }
-    sum += __shfl_xor(sum, 32);
-    if (lh == 0) ssum[lr][wave] = sum;
-    __syncthreads();
-    sum = ssum[lr][0];
-#pragma unroll
-    for (int w = 1; w < NW; w++) sum += ssum[lr][w];
-    const float inv = kvl > 0 ? (float)(1.0 / sum) : 0.0f;
-    // P rows in LDS: the lane's 4 runs of 4 consecutive keys per block
-#pragma unroll
-    for (int i = 0; i < SB; i++) {
-        if (i >= nbw) break;
-#pragma unroll
-        for (int r4 = 0; r4 < 4; r4++)
-            *(float4 *)(Sc + lr * SP + 32 * (bw0 + i) + 8 * r4 + 4 * lh) =
-                make_float4(sc[i][4 * r4] * inv, sc[i][4 * r4 + 1] * inv, sc[i][4 * r4 + 2] * inv,
-                            sc[i][4 * r4 + 3] * inv);
-    }
-    __syncthreads();
-    VXM_ATTN_TS(2);
-    // pass 3: partial O = P V of key quarter kq, dims [64 dh, 64 dh + 64); each block's V
-    // goes to this wave's LDS buffer as key-pair words, dims as rows
-    v16f o[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++) o[dt] = v16f{};
-    _Float16 *vt = Vt[wave];
-#pragma unroll
-    for (int i = 0; i < VB; i++) {
-        if (i >= nbq) break;
-        const int b = bq0 + i;
-#pragma unroll
-        for (int u = 0; u < VITEMS; u++) {
-            const int item = u * 64 + lane, r = 2 * (item % 16), d = 8 * (item / 16);
-            const uint32_t a[4] = {vr[i][u][0].x, vr[i][u][0].y, vr[i][u][0].z, vr[i][u][0].w};
-            const uint32_t bb[4] = {vr[i][u][1].x, vr[i][u][1].y, vr[i][u][1].z, vr[i][u][1].w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                *(uint32_t *)(vt + (d + 2 * e) * VP + r) = (a[e] & 0xffffu) | (bb[e] << 16);
-                *(uint32_t *)(vt + (d + 2 * e + 1) * VP + r) = (a[e] >> 16) | (bb[e] & 0xffff0000u);
-            }
-        }
-        // the wave's own LDS writes are seen by its later reads (one wave, in order)
-#pragma unroll
-        for (int ks = 0; ks < 32; ks += 16) {
-            const float *pr = Sc + lr * SP + 32 * b + ks + 8 * lh;
-            const float4 p0 = *(const float4 *)pr, p1 = *(const float4 *)(pr + 4);
-            const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-            v8h ahi, alo;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const _Float16 hi = (_Float16)pv[e];
-                ahi[e] = hi;
-                alo[e] = (_Float16)(pv[e] - (float)hi);
-            }
-#pragma unroll
-            for (int dt = 0; dt < DT; dt++) {
-                const v8h bv = *(const v8h *)(vt + (32 * dt + lr) * VP + ks + 8 * lh);
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahi, bv, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(alo, bv, o[dt], 0, 0, 0);
-            }
-        }
-    }
-    // the key quarters in order through LDS (P's buffer is free)
-    __syncthreads();
-    VXM_ATTN_TS(3);
-    float *red = Sc;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-        for (int v = 0; v < 16; v++)
-            red[(kq * AQ + 8 * (v >> 2) + 4 * lh + (v & 3)) * HD + HDH * dh + 32 * dt + lr] = o[dt][v];
-    __syncthreads();
-    if (xq) {
-        // Q8_0 of the output rows (the O projection's input; the arithmetic of
-        // k_quantize_q8_0): 8 values per lane, 4 lanes per 32-value block, the
-        // blocks of a row never crossing a head
-        for (int i = 8 * tid; i < AQ * HD; i += 8 * ATH) {
-            const int qi = i / HD, d = i % HD;
-            float v[8];
-#pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                float4 s = *(const float4 *)(red + i + 4 * hf);
-#pragma unroll
-                for (int w = 1; w < 4; w++) {
-                    const float4 t = *(const float4 *)(red + w * AQ * HD + i + 4 * hf);
-                    s.x = s.x + t.x; s.y = s.y + t.y; s.z = s.z + t.z; s.w = s.w + t.w;
-                }
-                v[4 * hf] = s.x; v[4 * hf + 1] = s.y; v[4 * hf + 2] = s.z; v[4 * hf + 3] = s.w;
-            }
-            const int64_t o = (int64_t)(t0 + min(qi, nq - 1)) * nh * HD + h * HD + d;
-            quant_block_4lanes(v, variant, xq + o, xd + o / 32, (tid & 3) == 0, qi < nq);
-        }
-    } else {
-        for (int i = 4 * tid; i < AQ * HD; i += 4 * ATH) {
-            const int qi = i / HD, d = i % HD;
-            if (qi >= nq) continue;
-            float4 s = *(const float4 *)(red + i);
-#pragma unroll
-            for (int w = 1; w < 4; w++) {
-                const float4 t = *(const float4 *)(red + w * AQ * HD + i);
-                s.x = s.x + t.x; s.y = s.y + t.y; s.z = s.z + t.z; s.w = s.w + t.w;
-            }
-            *(float4 *)(out + (int64_t)(t0 + qi) * nh * HD + h * HD + d) = s;
-        }
-    }
-    VXM_ATTN_TS(4);
-}
-
-// Spans above AKV keys: the same tiles, lane layouts and score arithmetic in one
-// pass over chunks of AKV keys with a running row max (every K and V row read
-// once, every score formed once).  Per chunk: the chunk's row max m_c over all 8
-// waves, m = max(m, m_c), the rescale a = exp(m_old - m) of the row's running
-// P V sums and double exp sum, e = exp(s - m) into LDS and the P V products.  At
-// the end the output is divided by the sum: o = (sum e v) * (float)(1 / sum e).
-// Against the one-pass kernel only the rounding differs (each chunk's rescale,
-// e instead of e / sum entering P V, and the summation orders).
-template <int HD>
-__global__ __launch_bounds__(ATH) void k_attention_mfma_long(const float *__restrict__ q,
-                                                             const uint16_t *__restrict__ kc,
-                                                             const uint16_t *__restrict__ vc, float *__restrict__ out,
-                                                             int M, int nh, int nkv, int cap, int kv_base, int causal,
-                                                             int8_t *__restrict__ xq, uint16_t *__restrict__ xd,
-                                                             int variant) {
-    constexpr int NW = ATH / 64;       // waves
-    constexpr int SP = AKV + 4;        // fp32 P row pitch
-    constexpr int KSTEPS = HD / 16;    // MFMA steps over the head dimension
-    constexpr int HDH = HD / 2;        // dims of one output half
-    constexpr int DT = HDH / 32;       // 32-dim output tiles per wave
-    constexpr int VP = 32 + 8;         // f16 pitch of a wave's transposed V block
-    constexpr int VITEMS = 16 * (HDH / 8) / 64;
-    constexpr int CB = AKV / 32;       // key blocks per chunk
-    constexpr int SB = CB / NW;        // most score blocks of one wave per chunk
-    constexpr int VB = CB / 4;         // most P V blocks of one key quarter per chunk
-    __shared__ __align__(16) float Sc[AQ * SP];
-    __shared__ __align__(16) _Float16 Vt[NW][HDH * VP];
-    __shared__ float smax[AQ][NW];
-    __shared__ double ssum[AQ][NW];
-    __shared__ float salpha[AQ], sinv[AQ];
-    constexpr int QP = HD + 8;
-    __shared__ __align__(16) _Float16 Qh[AQ * QP];
-    static_assert(NW == 8 && VITEMS >= 1 && 4 * AQ * HD <= AQ * SP, "8 waves; the key-quarter sums reuse P's buffer");
-    const int h = blockIdx.x, t0 = blockIdx.y * AQ, tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kvh = h / (nh / nkv);
-    const uint16_t *kb = kc + (int64_t)kvh * cap * HD;
-    const uint16_t *vb = vc + (int64_t)kvh * cap * HD;
-    const int nq = min(AQ, M - t0);
-    const int kv_end = causal ? kv_base + t0 + nq : M;
-    const float scale = __fdiv_rn(1.0f, __fsqrt_rn((float)HD));
-    const int lr = lane & 31, lh = lane >> 5;
-    const int nblk = (kv_end + 31) / 32, nch = (nblk + CB - 1) / CB;
-    const int kq = wave & 3, dh = wave >> 2;
-    constexpr int QL = AQ * HD / 4 / ATH;
-#pragma unroll
-    for (int u = 0; u < QL; u++) {
-        const int i = (u * ATH + tid) * 4, r = i / HD, d = i % HD;
-        const float4 qf = *(const float4 *)(q + (int64_t)(t0 + min(r, nq - 1)) * nh * HD + h * HD + d);
-        const bool qlive = r < nq;
-        _Float16 *dst = Qh + r * QP + d;
-        dst[0] = (_Float16)(qlive ? qf.x : 0.0f);
-        dst[1] = (_Float16)(qlive ? qf.y : 0.0f);
-        dst[2] = (_Float16)(qlive ? qf.z : 0.0f);
-        dst[3] = (_Float16)(qlive ? qf.w : 0.0f);
-    }
-    __syncthreads();
-    v8h qa[KSTEPS];
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; kk++) qa[kk] = *(const v8h *)(Qh + lr * QP + 16 * kk + 8 * lh);
-    const int kvl = lr < nq ? (causal ? kv_base + t0 + lr + 1 : M) : 0;
-    // the scores (S^T = K Q^T, scaled) of this wave's blocks of chunk c: block cb0 + i,
-    // i < ncb; value v of lane (lr, lh) is query t0 + lr, key 32 b + 8 (v / 4) + 4 lh + v % 4
-    auto scores = [&](int c, v16f (&sc)[SB], int &cb0, int &ncb) {
-        const int nbc = min(CB, nblk - c * CB);
-        cb0 = c * CB + nbc * wave / NW;
-        ncb = c * CB + nbc * (wave + 1) / NW - cb0;
-        uint4 kr[SB][KSTEPS];
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-            const int key = min(32 * (cb0 + i) + lr, kv_end - 1);   // unconditional: clamped rows
-#pragma unroll
-            for (int kk = 0; kk < KSTEPS; kk++) kr[i][kk] = *(const uint4 *)(kb + (int64_t)key * HD + 16 * kk + 8 * lh);
-        }
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-            v16f acc = v16f{};
-#pragma unroll
-            for (int kk = 0; kk < KSTEPS; kk++) {
-                v8h av;
-                __builtin_memcpy(&av, &kr[i][kk], 16);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, qa[kk], acc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int v = 0; v < 16; v++) sc[i][v] = acc[v] * scale;
+                vr[u][e] = *(const uint4 *)(vb + (int64_t)min(k0 + 2 * p + e, kv_end - 1) * HD + 8 * c);
         }
     };
-    auto live = [&](int i, int ncb, int b, int v) { return i < ncb && 32 * b + 8 * (v >> 2) + 4 * lh + (v & 3) < kvl; };
-    v16f sc[SB];
-    int cb0, ncb;
-    float mrow = -INFINITY;   // running max of row lr (the same in every lane and wave)
-    double lsum = 0.0;        // this lane's running double sum of e over its keys
+    auto put_v = [&](int r) {
+        uint32_t *vt = (uint32_t *)(lds + (r & 1) * Slot + KBytes);
+#pragma unroll
+        for (int u = 0; u < VI; u++) {
+            const int item = u * NT + tid, c = item % R16, p = item / R16, pp = p & 7;
+            const int w = (p & ~7) | (pp & 1) | ((pp >> 1) & 2) | ((pp << 1) & 4);
+            const uint32_t a[4] = {vr[u][0].x, vr[u][0].y, vr[u][0].z, vr[u][0].w};
+            const uint32_t b[4] = {vr[u][1].x, vr[u][1].y, vr[u][1].z, vr[u][1].w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int d = 8 * c + e;
+                vt[d * (KB / 2) + (w ^ (((d ^ (d >> 3)) & 15) << 2))] =
+                    e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u) : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
+            }
+        }
+    };
+
+    load(0);
+    v8h qa[KSTEPS];   // B operands: query t0 + lr, dims 16 kk + 8 lh .. + 8
+    {
+        const float *qr = q + (int64_t)(t0 + min(lr, nq - 1)) * nh * HD + h * HD + 8 * lh;
+#pragma unroll
+        for (int kk = 0; kk < KSTEPS; kk++) {
+            const float4 x = *(const float4 *)(qr + 16 * kk), y = *(const float4 *)(qr + 16 * kk + 4);
+            const float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) qa[kk][e] = (_Float16)(lr < nq ? f[e] : 0.0f);
+        }
+    }
+    float m = -INFINITY;
+    double lsum = 0.0;   // this lane's keys (half of the wave's)
     v16f o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = v16f{};
-    _Float16 *vt = Vt[wave];
-    const uint16_t *vbh = vb + HDH * dh;
-    for (int c = 0; c < nch; c++) {
-        const int nbc = min(CB, nblk - c * CB), cbase = c * CB;
-        const int bq0 = cbase + nbc * kq / 4, nbq = cbase + nbc * (kq + 1) / 4 - bq0;
-        // the V rows of the wave's P V blocks, in flight during the scores
-        uint4 vr[VB][VITEMS][2];
+    put_v(0);
+    vxm_vm_wait_all();
+    vxm_lds_barrier();
+    for (int r = 0; r < nr; r++) {
+        if (r + 1 < nr) load(r + 1);
+        const int b = NS * r + sp;
+        if (b < nblk) {
+            const int8_t *ks = lds + (r & 1) * Slot, *vs = ks + KBytes;
+            v16f s = v16f{};
+            const int row = 32 * sp + lr;
 #pragma unroll
-        for (int i = 0; i < VB; i++)
-#pragma unroll
-            for (int u = 0; u < VITEMS; u++) {
-                const int item = u * 64 + lane, r = 32 * (bq0 + i) + 2 * (item % 16), d = 8 * (item / 16);
-#pragma unroll
-                for (int e = 0; e < 2; e++)
-                    vr[i][u][e] = *(const uint4 *)(vbh + (int64_t)min(r + e, kv_end - 1) * HD + d);
+            for (int kk = 0; kk < KSTEPS; kk++) {
+                const v8h ka = *(const v8h *)(ks + row * (HD * 2) + (((2 * kk + lh) ^ kswz(row)) << 4));
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qa[kk], s, 0, 0, 0);
             }
-        scores(c, sc, cb0, ncb);
-        // the chunk's row max (the lane's, its partner's, the waves')
-        float mc = -INFINITY;
+            if (32 * b + 32 > kv_all) {   // some query does not see the whole block
 #pragma unroll
-        for (int i = 0; i < SB; i++)
+                for (int v = 0; v < 16; v++)
+                    if (32 * b + 8 * (v >> 2) + 4 * lh + (v & 3) >= kvl) s[v] = -INFINITY;
+            }
+            float mx = s[0];
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                if (live(i, ncb, cb0 + i, v)) mc = fmaxf(mc, sc[i][v]);
-        mc = fmaxf(mc, __shfl_xor(mc, 32));
-        if (lh == 0) smax[lr][wave] = mc;
-        __syncthreads();   // every wave's chunk max
-        float mn = mrow;
+            for (int v = 1; v < 16; v++) mx = fmaxf(mx, s[v]);
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * scale;   // scale > 0
+            if (__any(mx > m + kMaxSlack)) {
+                const float mn = fmaxf(m, mx), alpha = mn == -INFINITY ? 1.0f : expf(m - mn);
+                m = mn;
+                lsum *= (double)alpha;
 #pragma unroll
-        for (int w = 0; w < NW; w++) mn = fmaxf(mn, smax[lr][w]);
-        // rescale of the row's sums so far (0 for the first live chunk, 1 while m holds;
-        // a row with no live key yet keeps -inf and scale 1 over its zero sums)
-        const float alpha = mn == -INFINITY ? 1.0f : expf(mrow - mn);
-        mrow = mn;
-        if (wave == 0 && lh == 0) salpha[lr] = alpha;
-        lsum *= (double)alpha;
+                for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-        for (int i = 0; i < SB; i++) {
-            if (i >= ncb) break;
-            float pv[16];
+                    for (int v = 0; v < 16; v++) o[dt][v] = o[dt][v] * alpha;
+            }
+            // a query without a live key so far has m = -inf and only masked scores: e = 0
+            const float mneg = m == -INFINITY ? 0.0f : -m;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                pv[v] = live(i, ncb, cb0 + i, v) ? expf(sc[i][v] - mn) : 0.0f;
-                lsum += (double)pv[v];
+                s[v] = exp_near(__builtin_fmaf(s[v], scale, mneg));
+                lsum += (double)s[v];
             }
 #pragma unroll
-            for (int r4 = 0; r4 < 4; r4++)
-                *(float4 *)(Sc + lr * SP + 32 * (cb0 + i - cbase) + 8 * r4 + 4 * lh) =
-                    make_float4(pv[4 * r4], pv[4 * r4 + 1], pv[4 * r4 + 2], pv[4 * r4 + 3]);
-        }
-        __syncthreads();   // every wave's e rows of the chunk and the rows' rescales in LDS
-        // the partial P V of earlier chunks, rescaled to the new max (row of value v of
-        // the accumulators: 8 (v / 4) + 4 lh + v % 4)
-        float al[16];
+            for (int st = 0; st < 2; st++) {
+                v8h hi, lo;
 #pragma unroll
-        for (int v = 0; v < 16; v++) al[v] = salpha[8 * (v >> 2) + 4 * lh + (v & 3)];
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) o[dt][v] = o[dt][v] * al[v];
-#pragma unroll
-        for (int i = 0; i < VB; i++) {
-            if (i >= nbq) break;
-            const int b = bq0 + i;
-#pragma unroll
-            for (int u = 0; u < VITEMS; u++) {
-                const int item = u * 64 + lane, r = 2 * (item % 16), d = 8 * (item / 16);
-                const uint32_t a[4] = {vr[i][u][0].x, vr[i][u][0].y, vr[i][u][0].z, vr[i][u][0].w};
-                const uint32_t bb[4] = {vr[i][u][1].x, vr[i][u][1].y, vr[i][u][1].z, vr[i][u][1].w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    *(uint32_t *)(vt + (d + 2 * e) * VP + r) = (a[e] & 0xffffu) | (bb[e] << 16);
-                    *(uint32_t *)(vt + (d + 2 * e + 1) * VP + r) = (a[e] >> 16) | (bb[e] & 0xffff0000u);
-                }
-            }
-#pragma unroll
-            for (int ks = 0; ks < 32; ks += 16) {
-                const float *pr = Sc + lr * SP + 32 * (b - cbase) + ks + 8 * lh;
-                const float4 p0 = *(const float4 *)pr, p1 = *(const float4 *)(pr + 4);
-                const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-                v8h ahi, alo;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const _Float16 hi = (_Float16)pv[e];
-                    ahi[e] = hi;
-                    alo[e] = (_Float16)(pv[e] - (float)hi);
+                for (int e = 0; e < 8; e += 2) {
+                    const v2f p = {s[8 * st + e], s[8 * st + e + 1]};
+                    const v2h h2 = __builtin_convertvector(p, v2h);
+                    const v2f l = {__builtin_fmaf((float)h2[0], -1.0f, p[0]), __builtin_fmaf((float)h2[1], -1.0f, p[1])};
+                    const v2h l2 = __builtin_convertvector(l, v2h);
+                    hi[e] = h2[0]; hi[e + 1] = h2[1];
+                    lo[e] = l2[0]; lo[e + 1] = l2[1];
                 }
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++) {
-                    const v8h bv = *(const v8h *)(vt + (32 * dt + lr) * VP + ks + 8 * lh);
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ahi, bv, o[dt], 0, 0, 0);
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(alo, bv, o[dt], 0, 0, 0);
+                    const int d = 32 * dt + lr;
+                    const v8h va = *(const v8h *)(vs + d * (KB * 2) +
+                                                  (((4 * sp + 2 * st + lh) ^ ((d ^ (d >> 3)) & 15)) << 4));
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, hi, o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, lo, o[dt], 0, 0, 0);
                 }
             }
         }
-        __syncthreads();   // the chunk's e rows, maxima and rescales are read before the next chunk's
+        if (r + 1 < nr) put_v(r + 1);
+        vxm_vm_wait_all();   // this wave's key rows of the next round
+        vxm_lds_barrier();   // every wave's; and this round's slot is free
     }
-    // the row's double sum (lanes, partner, waves) and its inverse for the output rows
+
+    // merge the head's four waves in block order
     lsum += __shfl_xor(lsum, 32);
-    if (lh == 0) ssum[lr][wave] = lsum;
-    __syncthreads();
-    if (wave == 0 && lh == 0) {
-        double sum = ssum[lr][0];
-#pragma unroll
-        for (int w = 1; w < NW; w++) sum += ssum[lr][w];
-        sinv[lr] = kvl > 0 ? (float)(1.0 / sum) : 0.0f;
+    if (lh == 0) {
+        sm[hh][sp][lr] = m;
+        sl[hh][sp][lr] = lsum;
     }
-    // the key quarters in order through LDS (P's buffer is free)
-    float *red = Sc;
+    float *red = (float *)lds;   // [head][split][dim tile][16 values][64 lanes]
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-        for (int v = 0; v < 16; v++)
-            red[(kq * AQ + 8 * (v >> 2) + 4 * lh + (v & 3)) * HD + HDH * dh + 32 * dt + lr] = o[dt][v];
+        for (int v = 0; v < 16; v++) red[(((hh * NS + sp) * DT + dt) * 16 + v) * 64 + lane] = o[dt][v];
     __syncthreads();
-    if (xq) {
-        for (int i = 8 * tid; i < AQ * HD; i += 8 * ATH) {
-            const int qi = i / HD, d = i % HD;
-            float v[8];
-            const float inv = sinv[qi];
+    if (sp >= DT) return;
+    const int dt = sp;   // this wave's output tile
+    static_assert(DT <= NS, "one output tile per wave");
+    float mm = sm[hh][0][lr];
 #pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                float4 s = *(const float4 *)(red + i + 4 * hf);
+    for (int i = 1; i < NS; i++) mm = fmaxf(mm, sm[hh][i][lr]);
+    float w[NS];
+    double sum = 0.0;
 #pragma unroll
-                for (int w = 1; w < 4; w++) {
-                    const float4 t = *(const float4 *)(red + w * AQ * HD + i + 4 * hf);
-                    s.x = s.x + t.x; s.y = s.y + t.y; s.z = s.z + t.z; s.w = s.w + t.w;
-                }
-                v[4 * hf] = s.x * inv; v[4 * hf + 1] = s.y * inv; v[4 * hf + 2] = s.z * inv; v[4 * hf + 3] = s.w * inv;
-            }
-            const int64_t o2 = (int64_t)(t0 + min(qi, nq - 1)) * nh * HD + h * HD + d;
-            quant_block_4lanes(v, variant, xq + o2, xd + o2 / 32, (tid & 3) == 0, qi < nq);
-        }
-    } else {
-        for (int i = 4 * tid; i < AQ * HD; i += 4 * ATH) {
-            const int qi = i / HD, d = i % HD;
-            if (qi >= nq) continue;
-            float4 s = *(const float4 *)(red + i);
-#pragma unroll
-            for (int w = 1; w < 4; w++) {
-                const float4 t = *(const float4 *)(red + w * AQ * HD + i);
-                s.x = s.x + t.x; s.y = s.y + t.y; s.z = s.z + t.z; s.w = s.w + t.w;
-            }
-            const float inv = sinv[qi];
-            s.x = s.x * inv; s.y = s.y * inv; s.z = s.z * inv; s.w = s.w * inv;
-            *(float4 *)(out + (int64_t)(t0 + qi) * nh * HD + h * HD + d) = s;
-        }
+    for (int i = 0; i < NS; i++) {
+        const float mi = sm[hh][i][lr];
+        w[i] = mi == -INFINITY ? 0.0f : expf(mi - mm);
+        sum += sl[hh][i][lr] * (double)w[i];
     }
+    const float inv = kvl > 0 ? (float)(1.0 / sum) : 0.0f;
+    float ov[16], amax = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        float a = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NS; i++) a += red[(((hh * NS + i) * DT + dt) * 16 + v) * 64 + lane] * w[i];
+        ov[v] = a * inv;
+        amax = fmaxf(amax, fabsf(ov[v]));
+    }
+    // value v of lane (lr, lh): query t0 + lr, dim 32 dt + 8 (v / 4) + 4 lh + v % 4
+    const int64_t e0 = (int64_t)(t0 + min(lr, nq - 1)) * nh * HD + h * HD + 32 * dt;
+    if (xq) {
+        // Q8_0 of the 32 dims (the arithmetic of quant_block_4lanes; two lanes per block)
+        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        const float d = __fdiv_rn(amax, 127.0f);
+        float id;
+        if (variant == VXM_QUANT_X86) id = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
+        else id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
+        if (lr >= nq) return;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t b = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x = ov[4 * j + e] * id;
+                const float qv = fminf(fmaxf(variant == VXM_QUANT_X86 ? rintf(x) : roundf(x), -128.0f), 127.0f);
+                b |= (uint32_t)(uint8_t)(int8_t)(int)qv << (8 * e);
+            }
+            *(uint32_t *)(xq + e0 + 8 * j + 4 * lh) = b;
+        }
+        if (lh == 0) xd[e0 / 32] = vxm_f2h(d);
+    } else if (lr < nq) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            *(float4 *)(out + e0 + 8 * j + 4 * lh) = make_float4(ov[4 * j], ov[4 * j + 1], ov[4 * j + 2], ov[4 * j + 3]);
+    }
+}
+
+template <int HD>
+static void launch_attention_mfma(vxm_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
+                                  int64_t M, int nh, int nkv, int cap, int kv_base, int causal, int8_t *xq,
+                                  uint16_t *xd, int variant) {
+    const unsigned tiles = (unsigned)((M + AQ - 1) / AQ);
+    // two heads per workgroup share its key and value rows where that still fills the device
+    // (16 / 2 x 128: 1000 tokens 28.2 against 33.6 us, 512 tokens 18.0 against 16.3)
+    if (nh / nkv % 2 == 0 && (int64_t)nh / 2 * tiles >= ctx->n_cu)
+        hipLaunchKernelGGL((k_attention_mfma<HD, 2>), dim3(nh / 2, tiles), dim3(512), 0, ctx->stream, q, kc, vc, out,
+                           (int)M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
+    else
+        hipLaunchKernelGGL((k_attention_mfma<HD, 1>), dim3(nh, tiles), dim3(256), 0, ctx->stream, q, kc, vc, out,
+                           (int)M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
 }
 
 int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
@@ -909,24 +680,15 @@ int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const
     if (M <= 0) return VXM_OK;
     if (hd > 256 || hd <= 0 || nkv <= 0 || nh % nkv)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "attention: head_dim %d / heads %d,%d unsupported", hd, nh, nkv);
-    // many queries of a single segment whose key span fits the score buffer: the MFMA kernel
+    // the MFMA kernel: the queries of a single segment, a tile of them or at least two whose
+    // keys k_attention would walk for longer than a tile's padding costs (16 heads of 128:
+    // 24 queries over 24 keys 8.9 against 8.6 us, over 474 keys 14.7 against 23.5)
     const int64_t span = causal ? kv_base + M : M;
-    if (S == M && M >= AQ && span <= cap && (hd == 128 || hd == 64)) {
-        const dim3 grid(nh, (unsigned)((M + AQ - 1) / AQ));
-        if (span <= AKV) {
-            if (hd == 128)
-                hipLaunchKernelGGL(k_attention_mfma<128>, grid, dim3(ATH), 0, ctx->stream, q, kc, vc, out, (int)M, nh,
-                                   nkv, cap, kv_base, causal, xq, xd, variant);
-            else
-                hipLaunchKernelGGL(k_attention_mfma<64>, grid, dim3(ATH), 0, ctx->stream, q, kc, vc, out, (int)M, nh,
-                                   nkv, cap, kv_base, causal, xq, xd, variant);
-        } else if (hd == 128) {
-            hipLaunchKernelGGL(k_attention_mfma_long<128>, grid, dim3(ATH), 0, ctx->stream, q, kc, vc, out, (int)M,
-                               nh, nkv, cap, kv_base, causal, xq, xd, variant);
-        } else {
-            hipLaunchKernelGGL(k_attention_mfma_long<64>, grid, dim3(ATH), 0, ctx->stream, q, kc, vc, out, (int)M,
-                               nh, nkv, cap, kv_base, causal, xq, xd, variant);
-        }
+    if (S == M && (M >= AQ || (M >= 2 && span > 128)) && span <= cap && (hd == 128 || hd == 64)) {
+        if (hd == 128)
+            launch_attention_mfma<128>(ctx, q, kc, vc, out, M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
+        else
+            launch_attention_mfma<64>(ctx, q, kc, vc, out, M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
         VXM_CHECK_LAUNCH(ctx);
         return VXM_OK;
     }
