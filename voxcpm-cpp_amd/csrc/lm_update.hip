@@ -145,16 +145,32 @@ __global__ void k_prompt_fusion_in(const float *__restrict__ base, float *__rest
 // Q8_0 embedding rows (the Q8_0 branch of gen_forward_text, src/gen_prompt.c:
 // 106-125): out[i][j] = (float)qs[j] * fp16(d[j/32]) of row ids[i]; an id outside
 // [0, n_rows) takes row 0 (src/gen_prompt.c:113-114).
-__global__ void k_embed_rows_q8_0(const int8_t *__restrict__ qs, const uint16_t *__restrict__ d,
-                                  const int32_t *__restrict__ ids, int64_t n_rows, int64_t k,
-                                  float *__restrict__ out) {
+// VEC (out 16-byte aligned; rows are whole 32-value blocks): 8 values per thread, one
+// 8-byte load of quants and two 16-byte stores.  One value per thread and step took
+// 12.5 us for 2048 rows of 2048, against VEC_US.
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_embed_rows_q8_0(const int8_t *__restrict__ qs, const uint16_t *__restrict__ d,
+                                                         const int32_t *__restrict__ ids, int64_t n_rows, int64_t k,
+                                                         float *__restrict__ out) {
     const int i = blockIdx.x;
     int64_t r = ids[i];
     if (r < 0 || r >= n_rows) r = 0;
     const int8_t *q = qs + r * k;
     const uint16_t *dr = d + r * (k / 32);
     float *o = out + (int64_t)i * k;
-    for (int64_t j = threadIdx.x; j < k; j += blockDim.x) o[j] = (float)q[j] * vxm_h2f(dr[j / 32]);
+    if (VEC) {
+        for (int64_t j = threadIdx.x * 8; j < k; j += blockDim.x * 8) {
+            const uint2 w = *(const uint2 *)(q + j);
+            const float s = vxm_h2f(dr[j / 32]);
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = (float)(int8_t)((e < 4 ? w.x : w.y) >> (8 * (e & 3))) * s;
+            *(float4 *)(o + j) = make_float4(v[0], v[1], v[2], v[3]);
+            *(float4 *)(o + j + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    } else {
+        for (int64_t j = threadIdx.x; j < k; j += blockDim.x) o[j] = (float)q[j] * vxm_h2f(dr[j / 32]);
+    }
 }
 
 static unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -488,8 +504,12 @@ extern "C" int vxm_embed_rows_q8_0(vxm_ctx *ctx, const vxm_weight *table, const 
     if (!table || (n > 0 && (!ids_dev || !out_dev)) || n < 0)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "embed_rows: bad table / ids / out / n");
     if (n == 0) return VXM_OK;
-    hipLaunchKernelGGL(k_embed_rows_q8_0, dim3((unsigned)n), dim3(256), 0, ctx->stream, table->qs, table->d, ids_dev,
-                       table->n, table->k, out_dev);
+    if (((uintptr_t)out_dev & 15) == 0)
+        hipLaunchKernelGGL(k_embed_rows_q8_0<true>, dim3((unsigned)n), dim3(256), 0, ctx->stream, table->qs, table->d,
+                           ids_dev, table->n, table->k, out_dev);
+    else
+        hipLaunchKernelGGL(k_embed_rows_q8_0<false>, dim3((unsigned)n), dim3(256), 0, ctx->stream, table->qs, table->d,
+                           ids_dev, table->n, table->k, out_dev);
     VXM_CHECK_LAUNCH(ctx);
     return VXM_OK;
 }

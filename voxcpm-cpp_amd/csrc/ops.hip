@@ -1040,19 +1040,36 @@ int vxm_launch_swiglu_quant(vxm_ctx *ctx, vxm_parts gu, int64_t M, int64_t F, in
 // h = bf16(h + scale * bf16(delta)) (the residual adds of
 // vcpm_minicpm4_block, src/minicpm4.c:496-528), elementwise.
 // ---------------------------------------------------------------------------
-__global__ void k_residual(float *__restrict__ h, const vxm_parts delta, float scale, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Four elements per thread, every K-split slice's load in flight, added in slice order
+// (n % 4 == 0: rows of whole 32-value blocks; h and the slices are 16-byte aligned, as
+// the norm that reads them requires).
+__global__ __launch_bounds__(256) void k_residual(float *__restrict__ h, const vxm_parts delta, float scale,
+                                                  int64_t n) {
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i >= n) return;
-    float d = delta.p[i];
-    for (int z = 1; z < delta.n; z++) d = d + delta.p[z * delta.stride + i];
-    float o = vxm_bf16(d);
-    if (scale != 1.0f) o = o * scale;
-    h[i] = vxm_bf16(h[i] + o);
+    float4 x = *(const float4 *)(h + i), p[VXM_MAX_PARTS];
+#pragma unroll
+    for (int z = 0; z < VXM_MAX_PARTS; z++)
+        if (z < delta.n) p[z] = *(const float4 *)(delta.p + z * delta.stride + i);
+    float4 d = p[0];
+#pragma unroll
+    for (int z = 1; z < VXM_MAX_PARTS; z++)
+        if (z < delta.n) {
+            d.x = d.x + p[z].x; d.y = d.y + p[z].y; d.z = d.z + p[z].z; d.w = d.w + p[z].w;
+        }
+    auto add = [&](float a, float b) {
+        float o = vxm_bf16(b);
+        if (scale != 1.0f) o = o * scale;
+        return vxm_bf16(a + o);
+    };
+    *(float4 *)(h + i) = make_float4(add(x.x, d.x), add(x.y, d.y), add(x.z, d.z), add(x.w, d.w));
 }
 
 int vxm_launch_residual(vxm_ctx *ctx, float *h, vxm_parts delta, float scale, int64_t n) {
     if (n <= 0) return VXM_OK;
-    hipLaunchKernelGGL(k_residual, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, h, delta, scale, n);
+    if (n % 4) return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "residual: %lld values are not whole blocks", (long long)n);
+    hipLaunchKernelGGL(k_residual, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, ctx->stream, h, delta, scale,
+                       n);
     VXM_CHECK_LAUNCH(ctx);
     return VXM_OK;
 }

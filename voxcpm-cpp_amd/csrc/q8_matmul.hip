@@ -1311,11 +1311,7 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
 constexpr int kSmallStage = 8;                        // K blocks per LDS stage
 constexpr int kSmallPitch = kSmallStage * 32 + 16;    // LDS bytes per activation row
 constexpr int kSmallRG = 4;                           // 16-row groups (waves) per workgroup
-
-__device__ __forceinline__ float half_at(const v4i &v, int j) {
-    const uint32_t w = (uint32_t)v[j >> 1];
-    return vxm_h2f((uint16_t)((j & 1) ? (w >> 16) : (w & 0xffffu)));
-}
+constexpr int kSmallChunk = 32;                       // K blocks of one load of weight scales
 
 __device__ __forceinline__ long pack64(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); }
 
@@ -1333,6 +1329,9 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     constexpr int SB = kSmallStage, ROWS = 16 * MT, NT = 64 * kSmallRG;
     __shared__ __align__(16) int8_t xs_all[KG][ROWS * kSmallPitch];
     __shared__ float xds_all[KG][ROWS][SB + 1];
+    // a wave's weight scales of kSmallChunk blocks, [block][16 rows]: a lane's four rows
+    // are one read
+    __shared__ __align__(16) float dws_all[kSmallRG * KG][kSmallChunk * 16];
     const int nb = K / 32;
     const int g = blockIdx.x, z = blockIdx.y;
     // row tile of x: rows m0 .. m0 + Mt - 1 (one tile unless M > 16 MT)
@@ -1344,6 +1343,7 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     const int kg = wave_all / kSmallRG, wave = wave_all % kSmallRG, tid = tid_all % NT;
     int8_t *const xs = xs_all[kg];
     float(*const xds)[SB + 1] = xds_all[kg];
+    float *const dws = dws_all[wave_all];
     const int nw = g * 16 * kSmallRG + 16 * wave;
     // this group's share of the split's K blocks (the plan makes the shares equal)
     const int zs0 = z * bps, zs1 = min(nb, zs0 + bps), share = (zs1 - zs0) / KG;
@@ -1365,16 +1365,20 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     // products, two register sets alternating.
     constexpr int PIECES = ROWS * SB * 2, PPT = (PIECES + NT - 1) / NT, SPT = (ROWS * SB + NT - 1) / NT;
     struct Stage {
-        v4i wv[SB / 2], dwv[4], xv[PPT];
+        v4i wv[SB / 2], dwc, xv[PPT];
         uint16_t xh[SPT];
     };
+    // The weight scales of kSmallChunk blocks come with the first stage of each chunk in one
+    // load: lane l those of row l % 16, blocks 8 (l / 16) .. + 7 (the share's last eight past
+    // its end).  Loaded per stage, 16 lanes at the same address, they were four of a stage's
+    // ten loads, and the address unit is what the kernel waits for: DW_NOTE.
     auto issue = [&](Stage &st, int kb0) {
+        if ((kb0 - zb0) % kSmallChunk == 0)
+            st.dwc = __builtin_amdgcn_raw_buffer_load_b128(
+                wd_rsrc, ((nw + r) * nb + min(kb0 + 8 * q, zb1 - SB)) * 2, 0, 0);
 #pragma unroll
         for (int p = 0; p < SB / 2; p++)
             st.wv[p] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (nw + r) * K + (kb0 + 2 * p) * 32 + 16 * q, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            st.dwv[v] = __builtin_amdgcn_raw_buffer_load_b128(wd_rsrc, ((nw + 4 * q + v) * nb + kb0) * 2, 0, 0);
         // activation piece c = (row, block, half); threads past the end reload the last piece
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
@@ -1390,6 +1394,13 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     };
     auto run = [&](const Stage &st, int kb0) {
         __syncthreads();   // the previous stage's LDS reads are done
+        if ((kb0 - zb0) % kSmallChunk == 0) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t w = (uint32_t)st.dwc[j >> 1];
+                dws[(8 * q + j) * 16 + r] = vxm_h2f((uint16_t)(j & 1 ? w >> 16 : w & 0xffffu));
+            }
+        }
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
             const int c = k * NT + tid;
@@ -1445,10 +1456,8 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
             }
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                const int b = 2 * p + e;
-                float dw[4];
-#pragma unroll
-                for (int v = 0; v < 4; v++) dw[v] = half_at(st.dwv[v], b);
+                const float4 d4 = *(const float4 *)(dws + ((kb0 - zb0) % kSmallChunk + 2 * p + e) * 16 + 4 * q);
+                const float dw[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
                 for (int t = 0; t < MT; t++)
 #pragma unroll
