@@ -223,6 +223,15 @@ __device__ __forceinline__ int attn_wg_chunk(int h, int c) {
     return ((k / 8) * S::QPK + h % S::QPK) * 8 + k % 8;
 }
 
+// Its inverse: the query head that workgroup wg attends for with n chunks per head, and
+// the chunk; -1 for a workgroup without one.
+template <class S>
+__device__ __forceinline__ int attn_head_of(int wg, int n, int &chunk) {
+    const int sb = wg / 8 / S::QPK, k = sb * 8 + wg % 8;
+    chunk = k / S::NKV;
+    return chunk < n ? (k % S::NKV) * S::QPK + wg / 8 % S::QPK : -1;
+}
+
 __device__ __forceinline__ uint32_t make_tag(uint32_t epoch, int layer, int phase) {
     return (epoch << 12) | ((uint32_t)layer << 3) | (uint32_t)phase;
 }
@@ -1315,7 +1324,7 @@ __device__ __forceinline__ void attention_phase(const vxm_pparams &p, int l, int
 // waves 1..7 also stream weights and publish the outputs.  All waves walk
 // the same phase schedule and barrier sequence.
 template <class S>
-__device__ __forceinline__ void decode_run(const vxm_pparams &p, float *lds, int *bail, uint32_t ep) {
+__device__ __forceinline__ void decode_run(const vxm_pparams &p, float *lds, int *bail, uint32_t *ep_sh) {
     constexpr int H = S::H, QD = S::QD, KVD = S::KVD, HD = S::HD, F = S::F, NH = S::NH;
     constexpr int SX = rep_stride(H / 2), SQ = rep_stride(S::NQKV / 2), SAT = rep_stride(QD), SP = rep_stride(F / 2);
     const int wg = blockIdx.x;
@@ -1330,22 +1339,8 @@ __device__ __forceinline__ void decode_run(const vxm_pparams &p, float *lds, int
     const int t = tid_now() - 64 * kNR;                         // compute thread index
     const int pos = p.pos;
     // the query head this workgroup attends for, or -1
-    int head = -1, chunk = 0;
-    for (int h = 0; h < NH; h++)
-        for (int c = 0; c < p.att_split; c++)
-            if (attn_wg_chunk<S>(h, c) == wg) {
-                head = h;
-                chunk = c;
-            }
-
-    // rope cos/sin of this token's position (ggml_rope_ext NEOX angles, host table)
-    if (!p.no_rope) {
-        for (int i = tid_now(); i < HD / 2; i += kThreads) {
-            const float2 r = p.rope_cs[(int64_t)pos * (HD / 2) + i];
-            cs[2 * i] = r.x;
-            cs[2 * i + 1] = r.y;
-        }
-    }
+    int chunk;
+    const int head = attn_head_of<S>(wg, p.att_split, chunk);
 
     // this wave's ring slots in LDS (compute waves only)
     const int8_t *ring = (const int8_t *)lds + S::RING_OFF + (reader ? 0 : ci) * S::RING * kSlot;
@@ -1353,33 +1348,62 @@ __device__ __forceinline__ void decode_run(const vxm_pparams &p, float *lds, int
     UnitBases cur = unit_bases(p, 0);
     if (!reader) ring_prime<S>(p, cur, ring_lds, wg, ci, lane, std::make_integer_sequence<int, S::P>{});
 
+    // The launch's own inputs -- its tag epoch, x, the first gain and the rope cos/sin of this
+    // token's position (ggml_rope_ext NEOX angles, host table) -- all loaded at once by wave 0,
+    // which has no ring, while the other waves fill theirs.  Every wave waiting for the epoch
+    // before its ring, the head found by a search over all heads and chunks, and cos/sin, gain
+    // and x one round trip after another (behind the rings' loads at the memory side) had x
+    // ready 8.1 us after the launch's start, now 3.9 (one layer at 512 keys 31.3 -> 27.7 us).
+    static_assert(kNR >= 1 && H % 256 == 0 && HD / 2 <= 64, "wave 0 loads the launch's inputs");
+    if (wave == 0) {
+        constexpr int XV = H / 256;
+        float4 x0[XV], g0[XV];
+        const uint32_t e = __hip_atomic_load(p.state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < XV; i++) x0[i] = *(const float4 *)(p.x + lane * 4 + 256 * i);
+        const float *g = layer_at(p, 0)->g_in;
+#pragma unroll
+        for (int i = 0; i < XV; i++) g0[i] = *(const float4 *)(g + lane * 4 + 256 * i);
+        if (!p.no_rope && lane < HD / 2) {
+            const float2 r = p.rope_cs[(int64_t)pos * (HD / 2) + lane];
+            cs[2 * lane] = r.x;
+            cs[2 * lane + 1] = r.y;
+        }
+        double ss = 0.0;
+#pragma unroll
+        for (int i = 0; i < XV; i++) {
+            const float4 v = x0[i];
+            *(float4 *)(xs + lane * 4 + 256 * i) = v;
+            *(float4 *)(gn + lane * 4 + 256 * i) = g0[i];
+            ss += (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
+        }
+        ss = wave_sum_63_d(ss);
+        if (lane == 63) ssq[0] = ss;
+        if (lane == 0) *ep_sh = e;
+    } else if (wave < kXReaders && lane == 63) {
+        ssq[wave] = 0.0;
+    }
+    lds_barrier();
+    const uint32_t ep = __builtin_amdgcn_readfirstlane(*ep_sh);
+
     for (int l = 0; l < p.n_layers; l++) {
         vxm_ptab Ly = layer_at(p, l);
         const UnitBases nxt = unit_bases(p, l + 1);
         // ---------------- A: norm + QKV + rope ----------------
         static_assert((H / 2) % (128 * kXReaders) == 0 && H / 2 / kXReaders <= 64 * 64, "x readers");
-        if (wave == 0) stage_f32(Ly->g_in, H, gn);
-        if (wave < kXReaders) {
-            // waves 0 .. kXReaders-1 each read a share of x (and its sum of squares)
-            constexpr int XW = H / 2 / kXReaders;   // words per reading wave
-            double ss = 0.0;
-            if (l == 0) {
-                if (wave == 0) {
-                    for (int i = lane * 4; i < H; i += 256) {
-                        const float4 v = *(const float4 *)(p.x + i);
-                        *(float4 *)(xs + i) = v;
-                        ss += (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
-                    }
-                }
-            } else {
-                ss = read_words<cdiv(XW / 2, 64), true>(p, p.xb + ((l & 1) * kRep + rp) * SX + wave * XW, XW / 2,
-                                                        make_tag(ep, l, PH_X), xs + 2 * wave * XW, bail);
+        if (l > 0) {
+            if (wave == 0) stage_f32(Ly->g_in, H, gn);
+            if (wave < kXReaders) {
+                // waves 0 .. kXReaders-1 each read a share of x (and its sum of squares)
+                constexpr int XW = H / 2 / kXReaders;   // words per reading wave
+                double ss = read_words<cdiv(XW / 2, 64), true>(p, p.xb + ((l & 1) * kRep + rp) * SX + wave * XW, XW / 2,
+                                                               make_tag(ep, l, PH_X), xs + 2 * wave * XW, bail);
+                ss = wave_sum_63_d(ss);
+                if (lane == 63) ssq[wave] = ss;
             }
-            ss = wave_sum_63_d(ss);
-            if (lane == 63) ssq[wave] = ss;
+            lds_barrier();
+            if (*bail) return;
         }
-        lds_barrier();
-        if (*bail) return;
         VXM_TS(tid_now() == 0, 0);
         if (p.dump && wg == 0)
             for (int i = tid_now() * 4; i < H; i += kThreads * 4)
@@ -1603,10 +1627,10 @@ __global__ __launch_bounds__(kThreads, 1) void k_decode_persistent(vxm_pparams p
 #ifdef VXM_PERSISTENT_TRACE
     if (threadIdx.x == 0 && p.trace) p.trace[(size_t)blockIdx.x * p.trace_stride] = __builtin_amdgcn_s_memrealtime();
 #endif
-    // a scalar load: the previous launch's last workgroup wrote it before that launch ended
-    const uint32_t ep = __builtin_amdgcn_readfirstlane(*(const volatile uint32_t *)p.state);
-    // bail is read only after the first barrier of decode_run
-    decode_run<S>(p, lds, bail, ep);
+    // the launch's epoch, written by decode_run before its first barrier (the previous launch's
+    // last workgroup advanced it before that launch ended); bail is read only after that barrier
+    uint32_t *ep_sh = (uint32_t *)(bail + 2);
+    decode_run<S>(p, lds, bail, ep_sh);
     // every ring load of the wave (the refills past the last layer, or those in
     // flight when a wait gave up) lands before the workgroup ends
     ring_wait<0>();
@@ -1619,7 +1643,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_decode_persistent(vxm_pparams p
     if (!*last) return;
     // the last workgroup: every other workgroup has read the epoch and finished
     // with the channels
-    uint32_t next = (ep + 1u) & kEpochMask;
+    uint32_t next = (*ep_sh + 1u) & kEpochMask;
     if (next == 0) {
         next = 1;
         for (uint64_t i = threadIdx.x; i < p.n_chan; i += kThreads)
@@ -1668,7 +1692,7 @@ static constexpr int kMaxLds = 160 * 1024;
 // interleave their workgroups.
 template <class S>
 static int launch_decode(vxm_ctx *ctx, const vxm_pparams &prm) {
-    const int lds = S::BYTES + 16;   // the layout + the bail and last-workgroup flags
+    const int lds = S::BYTES + 16;   // the layout + the bail and last-workgroup flags and the epoch
     auto kern = k_decode_persistent<S>;
     if (lds > kMaxLds)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "persistent decode: kv capacity %d needs %d B of LDS", prm.cap, lds);
