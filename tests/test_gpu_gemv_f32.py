@@ -51,3 +51,37 @@ def test_output_over_the_input(vxm_ctx, orc):
         torch.cuda.synchronize()
         assert np.array_equal(_host(vxm_ctx, vxm_ctx.mul_mat(w, y, y)), ref)
     w.free()
+
+
+@pytest.mark.parametrize("N,K,M", [(64, 256, 8), (2048, 6144, 16), (2048, 2048, 17), (1024, 4096, 31), (512, 2048, 32),
+                                   (6144, 2048, 9), (64, 512, 10)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_fused_small_gemm_equals_three_launches(vxm_ctx, orc, N, K, M, variant):
+    """The small-M GEMM's own quantization (one and two row tiles, one to three wave groups, split
+    and unsplit K) gives the bits of the separate launches."""
+    import torch
+
+    rng = np.random.default_rng(2 * N + K + M)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    x[0, :32] = 0.0
+    x[-1, -1] = 3e38
+    w = vxm_ctx.upload_q8_0(orc.quantize_rows(rng.normal(0, 0.02, (N, K)).astype(np.float32), orc.QUANT_REF), N, K)
+    xd = torch.from_numpy(x).to("cuda:0")
+    torch.cuda.synchronize()
+    vxm_ctx.set_quant_variant(variant)
+    try:
+        y = _host(vxm_ctx, vxm_ctx.mul_mat(w, xd))
+    finally:
+        vxm_ctx.set_quant_variant(1)
+    ref = _host(vxm_ctx, vxm_ctx.mul_mat_q8(w, *vxm_ctx.quantize_q8_0(xd, variant)))
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+    if N <= K:   # over the input: the same bits
+        buf = xd.clone()
+        torch.cuda.synchronize()
+        vxm_ctx.set_quant_variant(variant)
+        try:
+            over = _host(vxm_ctx, vxm_ctx.mul_mat(w, buf, buf.view(-1)[:M * N].view(M, N)))
+        finally:
+            vxm_ctx.set_quant_variant(1)
+        assert np.array_equal(over.view(np.uint32), ref.view(np.uint32))
+    w.free()

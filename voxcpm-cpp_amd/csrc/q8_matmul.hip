@@ -1307,6 +1307,10 @@ __global__ __launch_bounds__(kTileThreads, 1) void k_gemm_q8_0_tile(
 // Rows past M read as zeros (outside the buffer range) and are not written.
 // DOTS = true writes the int32 block sums of the MFMAs to dots[(m*N + n)*nb + b]
 // instead (every split its own blocks; no scaling, no epilogue).
+// XF = true takes fp32 activations xf and quantizes each stage's pieces on the way to
+// LDS (k_quantize_q8_0's arithmetic, the two threads of a block exchanging their
+// maxima): the public entry's quantization launch goes, at the price of every
+// workgroup quantizing the rows of its K range (one or two row tiles only).
 // ---------------------------------------------------------------------------
 constexpr int kSmallStage = 8;                        // K blocks per LDS stage
 constexpr int kSmallPitch = kSmallStage * 32 + 16;    // LDS bytes per activation row
@@ -1315,9 +1319,10 @@ constexpr int kSmallChunk = 32;                       // K blocks of one load of
 
 __device__ __forceinline__ long pack64(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); }
 
-template <int MT, int KG, bool DOTS>
+template <int MT, int KG, bool DOTS, bool XF>
 __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const int8_t *__restrict__ xq,
                                                                    const uint16_t *__restrict__ xd,
+                                                                   const float *__restrict__ xf,
                                                                    const int8_t *__restrict__ wq,
                                                                    const uint16_t *__restrict__ wd,
                                                                    float *__restrict__ y, int M, int N, int K,
@@ -1338,6 +1343,7 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     const int m0 = blockIdx.z * ROWS, Mt = min(ROWS, M - m0);
     xq += (int64_t)m0 * K;
     xd += (int64_t)m0 * nb;
+    xf += (int64_t)m0 * K;
     const int tid_all = threadIdx.x, lane = tid_all & 63, q = lane >> 4, r = lane & 15;
     const int wave_all = __builtin_amdgcn_readfirstlane(tid_all >> 6);
     const int kg = wave_all / kSmallRG, wave = wave_all % kSmallRG, tid = tid_all % NT;
@@ -1349,7 +1355,8 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     const int zs0 = z * bps, zs1 = min(nb, zs0 + bps), share = (zs1 - zs0) / KG;
     const int zb0 = zs0 + kg * share, zb1 = zb0 + share;
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wq, (short)0, N * K, 0x00020000);
-    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)xq, (short)0, Mt * K, 0x00020000);
+    const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        XF ? (void *)xf : (void *)xq, (short)0, XF ? Mt * K * 4 : Mt * K, 0x00020000);
     const __amdgpu_buffer_rsrc_t wd_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void *)wd, (short)0, N * nb * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t xd_rsrc =
@@ -1365,7 +1372,7 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
     // products, two register sets alternating.
     constexpr int PIECES = ROWS * SB * 2, PPT = (PIECES + NT - 1) / NT, SPT = (ROWS * SB + NT - 1) / NT;
     struct Stage {
-        v4i wv[SB / 2], dwc, xv[PPT];
+        v4i wv[SB / 2], dwc, xv[XF ? 4 * PPT : PPT];
         uint16_t xh[SPT];
     };
     // The weight scales of kSmallChunk blocks come with the first stage of each chunk in one
@@ -1385,10 +1392,17 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
         for (int k = 0; k < PPT; k++) {
             const int c = min(k * NT + tid, PIECES - 1);
             const int row = c / (2 * SB), b = (c / 2) % SB, h = c & 1;
-            st.xv[k] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, row * K + (kb0 + b) * 32 + 16 * h, 0, 0);
+            const int at = row * K + (kb0 + b) * 32 + 16 * h;
+            if (XF) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    st.xv[4 * k + j] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, 4 * (at + 4 * j), 0, 0);
+            } else {
+                st.xv[k] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, at, 0, 0);
+            }
         }
 #pragma unroll
-        for (int k = 0; k < SPT; k++) {
+        for (int k = 0; k < (XF ? 0 : SPT); k++) {
             const int c = min(k * NT + tid, ROWS * SB - 1);
             st.xh[k] = __builtin_amdgcn_raw_buffer_load_b16(xd_rsrc, ((c / SB) * nb + kb0 + c % SB) * 2, 0, 0);
         }
@@ -1405,15 +1419,45 @@ __global__ __launch_bounds__(64 * kSmallRG * KG) void k_gemm_q8_0_small(const in
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
             const int c = k * NT + tid;
+            v4i piece;
+            float dsc = 0.0f;
+            if (XF) {   // every lane: the two of a block exchange their maxima
+                float f[16], amax = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    f[j] = __int_as_float(st.xv[4 * k + j / 4][j & 3]);
+                    amax = fmaxf(amax, fabsf(f[j]));
+                }
+                amax = fmaxf(amax, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(amax), 0xB1, 0xF, 0xF, false)));
+                const float d = __fdiv_rn(amax, 127.0f);
+                float id;
+                if (variant == VXM_QUANT_X86) id = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
+                else id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
+                dsc = vxm_h2f(vxm_f2h(d));
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    uint32_t b4 = 0;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float t = f[4 * w + j] * id;
+                        const float qv = variant == VXM_QUANT_X86 ? fminf(fmaxf(rintf(t), -128.0f), 127.0f) : roundf(t);
+                        b4 |= (uint32_t)(uint8_t)(int8_t)(int)qv << (8 * j);
+                    }
+                    piece[w] = (int)b4;
+                }
+            } else {
+                piece = st.xv[k];
+            }
             if (PIECES % NT == 0 || c < PIECES) {
                 const int row = c / (2 * SB), b = (c / 2) % SB, h = c & 1;
                 int8_t *dst = xs + row * kSmallPitch + b * 32;
-                *(long *)(dst + 8 * h) = pack64((uint32_t)st.xv[k].x, (uint32_t)st.xv[k].y);
-                *(long *)(dst + 8 * h + 16) = pack64((uint32_t)st.xv[k].z, (uint32_t)st.xv[k].w);
+                *(long *)(dst + 8 * h) = pack64((uint32_t)piece.x, (uint32_t)piece.y);
+                *(long *)(dst + 8 * h + 16) = pack64((uint32_t)piece.z, (uint32_t)piece.w);
+                if (XF && h == 0) xds[row][b] = dsc;
             }
         }
 #pragma unroll
-        for (int k = 0; k < SPT; k++) {
+        for (int k = 0; k < (XF ? 0 : SPT); k++) {
             const int c = k * NT + tid;
             if ((ROWS * SB) % NT == 0 || c < ROWS * SB) xds[c / SB][c % SB] = kb0 + c % SB < zb1 ? vxm_h2f(st.xh[k]) : 0.0f;
         }
@@ -1860,6 +1904,13 @@ static int launch_gemm(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, cons
     return VXM_OK;
 }
 
+// The small-M GEMM quantizes fp32 activations itself in one or two row tiles, while what all
+// workgroups quantize together (padding rows included) costs less than the launch saved.
+// Measured (us a call, 8 rows unless said, against three launches): 2048 x 2048 7.3 / 10.2,
+// 2048 x 6144 (3.1 M values) 9.2 / 11.4, 6144 x 2048 (3.1 M) 8.8 / 12.0, 1024 x 4096 at 32 rows (2.1 M)
+// 10.4 / 11.0; 12288 x 2048 (6.3 M) 12.6 / 12.1, 6144 x 2048 at 24 rows (6.3 M) 14.8 / 12.9.
+constexpr int kSmallF32MaxRows = 32;
+constexpr int64_t kSmallF32MaxValues = 4 << 20;
 // Rows of activations from which the MFMA GEMM replaces the weight-streaming
 // GEMV (which re-reads each activation row per weight row group).
 constexpr int kMfmaMinRows = 8;
@@ -1903,46 +1954,53 @@ static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_pa
     return true;
 }
 
+// Rows up to which the small-M kernel takes every product of its layout: one 16-row tile,
+// where it is level with the tile GEMM at worst (12288 x 2048, 16 rows: 13.1 / 12.9 us).
+constexpr int kSmallAlwaysRows = 16;
+
 // The small-M kernel's plan for the product, where it is the one to run: any M it
-// takes up to one row tile; above that (each row tile reads the weights again)
-// where the tile GEMM would split K, whose tag launch, partial words and
-// last-workgroup fix-up cost more than the second read of the weights (M = 77, public
-// entry: 2048 x 2048 15.6 -> 11.5 us, 2048 x 6144 19.7 -> 16.9, 1024 x 4096 17.0 ->
-// 13.1 at M = 100; 12288 x 2048, which the tile GEMM takes unsplit, stays there: 19.0
-// against 28.2).  With a fix-up launch of its own (the public entries) only where its
-// grid is one round: 2560 x 2048, 320 workgroups, 16.6 against 15.7 us at M = 100.  With
-// three row tiles (M > 128) it loses: 2048 x 6144 30.1 against 23.4 us at M = 150.  K is
-// bounded there so that the slices and the quantized rows of any such product fit the
-// allocation-free entry's scratch together.
+// takes up to kSmallAlwaysRows; above that (each row tile of its waves repeats the
+// scaling work, and past 64 rows the read of the weights) where the tile GEMM would
+// split K, whose tag launch, partial words and last-workgroup fix-up cost more (M = 77,
+// public entry: 2048 x 2048 15.6 -> 11.5 us, 2048 x 6144 19.7 -> 16.9, 1024 x 4096 17.0 ->
+// 13.1 at M = 100).  12288 x 2048, which the tile GEMM takes unsplit, goes there: 24.3 ->
+// 13.0 us at M = 64, 17.4 -> 12.9 at 24, 28.2 / 19.0 at 77.  Past 64 rows and with a fix-up
+// launch of its own (the public entries) only where its grid is one round: 2560 x 2048,
+// 320 workgroups, 16.6 against 15.7 us at M = 100.  With three row tiles (M > 128) it
+// loses: 2048 x 6144 30.1 against 23.4 us at M = 150.  K is bounded there so that the
+// slices and the quantized rows of any such product fit the allocation-free entry's
+// scratch together.
 static bool small_wins(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                        int max_parts, bool fixup, SmallPlan &p) {
     if (!small_plan(ctx, M, w->n, w->k, max_parts, p)) return false;
-    if (M <= VXM_SMALL_TILE_ROWS) return true;
-    if (fixup && (int64_t)p.groups * p.mtiles * p.splits > ctx->n_cu) return false;
+    if (M <= kSmallAlwaysRows) return true;
+    if (M > VXM_SMALL_TILE_ROWS && fixup && (int64_t)p.groups * p.mtiles * p.splits > ctx->n_cu) return false;
     GemmPlan t;
-    return w->k <= 16384 && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
+    return (M <= VXM_SMALL_TILE_ROWS || w->k <= 16384) && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
 }
 
+// xf != nullptr: fp32 activations, quantized by the kernel with `variant` (p.mt <= 2, no dots).
 static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                          float *y, const SmallPlan &p, int8_t *sq = nullptr, uint16_t *sd = nullptr,
-                         int variant = 0, int32_t *dots = nullptr) {
+                         int variant = 0, int32_t *dots = nullptr, const float *xf = nullptr) {
     const dim3 grid(p.groups, p.splits, p.mtiles), block(64 * kSmallRG * p.kg);
     const int N = (int)w->n, K = (int)w->k;
-#define VXM_SMALL_ARGS xq, xd, w->qs, w->d, y, (int)M, N, K, p.bps, sq, sd, variant, dots
-#define VXM_SMALL_KG(MT, D)                                                                                \
-    do {                                                                                                   \
-        if (p.kg == 3)                                                                                     \
-            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, small_kg_max(MT), D>), grid, block, 0, ctx->stream,  \
-                               VXM_SMALL_ARGS);                                                            \
-        else if (p.kg == 2)                                                                                \
-            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 2, D>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
-        else                                                                                               \
-            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 1, D>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
+#define VXM_SMALL_ARGS xq, xd, xf, w->qs, w->d, y, (int)M, N, K, p.bps, sq, sd, variant, dots
+#define VXM_SMALL_KG(MT, D, X)                                                                                \
+    do {                                                                                                      \
+        if (p.kg == 3)                                                                                        \
+            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, small_kg_max(MT), D, X>), grid, block, 0, ctx->stream,  \
+                               VXM_SMALL_ARGS);                                                               \
+        else if (p.kg == 2)                                                                                   \
+            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 2, D, X>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
+        else                                                                                                  \
+            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 1, D, X>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
     } while (0)
-#define VXM_SMALL_MT(MT)                    \
-    do {                                    \
-        if (dots) VXM_SMALL_KG(MT, true);   \
-        else VXM_SMALL_KG(MT, false);       \
+#define VXM_SMALL_MT(MT)                                 \
+    do {                                                 \
+        if (xf) VXM_SMALL_KG(MT, false, (MT <= 2));      \
+        else if (dots) VXM_SMALL_KG(MT, true, false);    \
+        else VXM_SMALL_KG(MT, false, false);             \
     } while (0)
     switch (p.mt) {
         case 1: VXM_SMALL_MT(1); break;
@@ -1958,9 +2016,10 @@ static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, co
 // Public entry: a split product goes through the context's scratch and one
 // fix-up launch that adds the slices in order.
 static int launch_gemm_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
-                             float *y, const SmallPlan &p, const MmWork *wk = nullptr) {
+                             float *y, const SmallPlan &p, const MmWork *wk = nullptr, const float *xf = nullptr) {
+    const int variant = ctx->quant_variant;
     if (p.splits == 1) {
-        launch_small(ctx, w, xq, xd, M, y, p);
+        launch_small(ctx, w, xq, xd, M, y, p, nullptr, nullptr, variant, nullptr, xf);
         VXM_CHECK_LAUNCH(ctx);
         return VXM_OK;
     }
@@ -1978,7 +2037,7 @@ static int launch_gemm_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
         if (rc) return rc;
         scratch = (float *)ctx->parts_buf;
     }
-    launch_small(ctx, w, xq, xd, M, scratch, p);
+    launch_small(ctx, w, xq, xd, M, scratch, p, nullptr, nullptr, variant, nullptr, xf);
     VXM_CHECK_LAUNCH(ctx);
     const int64_t threads = count / 4;   // N % 64 == 0
     hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, scratch,
@@ -2004,9 +2063,13 @@ int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 // The gate/up projection with SwiGLU and the Q8_0 of its output fused into the
 // GEMM's epilogue (rows of w interleave gate n = row 2n and up n = row 2n+1): sq
 // [M][N/2] and sd [M][N/64] are the down projection's input.  The small-M kernel
-// takes M <= 64, the tile GEMM larger M when its plan needs no K split.  Returns
+// takes M <= 32, the tile GEMM larger M when its plan needs no K split.  Returns
 // false without launching otherwise (and under PATH_MFMA_TILED, which keeps the
 // unfused GEMM + k_swiglu_quant as the reference of the fused epilogue).
+// (up to two of the small-M kernel's row tiles it is level with the tile GEMM; one layer at
+// 64 rows 64.7 -> 58.7 us on the tile GEMM, at 33 rows 54.5)
+constexpr int kSmallGateUpRows = 32;
+
 bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                                int8_t *sq, uint16_t *sd, int variant, int *rc) {
     *rc = VXM_OK;
@@ -2014,7 +2077,7 @@ bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *
     const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
     if (!mfma || M <= 0 || N % 64) return false;
     SmallPlan sp;
-    if (M <= VXM_SMALL_TILE_ROWS && small_plan(ctx, M, N, K, 1, sp)) {
+    if (M <= kSmallGateUpRows && small_plan(ctx, M, N, K, 1, sp)) {
         // unsplit: each workgroup holds whole 32-pair blocks over all of K
         launch_small(ctx, w, xq, xd, M, nullptr, sp, sq, sd, variant);
     } else {
@@ -2233,6 +2296,15 @@ extern "C" int vxm_mul_mat_q8_0(vxm_ctx *ctx, const vxm_weight *w, const float *
     if (rc) return rc;
     if (vxm_launch_gemv_f32(ctx, w, x_dev, M, ctx->quant_variant, vxm_gemv_epi{y_dev}, &rc)) return rc;
     const int64_t K = w->k;
+    // one or two row tiles on the small-M GEMM: quantized inside it (not over the input where
+    // it writes y itself: workgroups still read rows that others have finished)
+    SmallPlan sp;
+    const bool over = (uintptr_t)y_dev < (uintptr_t)x_dev + (size_t)M * K * 4 &&
+                      (uintptr_t)y_dev + (size_t)M * w->n * 4 > (uintptr_t)x_dev;
+    if (M <= kSmallF32MaxRows && use_mfma(ctx, M) && ctx->path != VXM_PATH_MFMA_TILED &&
+        small_wins(ctx, w, nullptr, nullptr, M, VXM_MAX_PARTS, true, sp) &&
+        (int64_t)16 * sp.mt * K * sp.groups <= kSmallF32MaxValues && !(over && sp.splits == 1))
+        return launch_gemm_small(ctx, w, nullptr, nullptr, M, y_dev, sp, nullptr, x_dev);
     const size_t qbytes = ((size_t)M * K + 255) & ~(size_t)255;
     rc = vxm_ensure_act(ctx, qbytes + (size_t)M * (K / VXM_QK) * 2);
     if (rc) return rc;
