@@ -321,9 +321,18 @@ extern "C" int vxm_locenc_forward(vxm_locenc *m, const float *x_dev, int32_t P, 
     const bool persistent = m->cfg.n_layers > 0 && vxm_locdit_persistent_pick(ctx, d, S, (int)S, m->block_mode);
     if (m->block_mode == VXM_DECODE_PERSISTENT && !persistent)
         return vxm_fail(ctx, VXM_ERR_NOT_IMPLEMENTED, "locenc: no persistent block kernel for this shape / device");
+    // the rows that are returned, normalised: the special token's row (src/locenc.c:118-128),
+    // or every row
+    const int64_t rows = off ? 1 : S;
     if (persistent) {
-        // all blocks in one launch; seq then holds the last block's output, residual included
-        if ((rc = vxm_locdit_persistent_run(ctx, d, m->blocks, &m->lp, m->seq, S, (int)S, m->block_dump))) return rc;
+        // all blocks in one launch, the returned rows' final norm included (a launch of its own
+        // for it took an encoder call of 5 rows from 289.7 to 295.5 us); seq then holds the last
+        // block's output.  One row tile only, the form built for it; the norm writes pairs, so an
+        // output that is not 8-byte aligned keeps its launch too.
+        vxm_lfinal fin{};
+        if (S <= 16 && ((uintptr_t)out_dev & 7) == 0) fin = vxm_lfinal{m->norm, 0, nullptr, nullptr, out_dev, (int)rows};
+        if ((rc = vxm_locdit_persistent_run(ctx, d, m->blocks, &m->lp, m->seq, S, (int)S, m->block_dump, fin))) return rc;
+        if (fin.g) return VXM_OK;
     } else {
         const vxm_attn_site site{m->ws.lk, m->ws.lv, (int)S, (int64_t)d.nkv * S * d.hd, (int)S, 0, 0, 0};
         for (int l = 0; l < m->cfg.n_layers; l++) {
@@ -345,9 +354,7 @@ extern "C" int vxm_locenc_forward(vxm_locenc *m, const float *x_dev, int32_t P, 
                                         (size_t)S * H * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
         }
     }
-    // last residual + final RMSNorm of the rows that are returned: the
-    // special token's row (src/locenc.c:118-128), or every row
-    const int64_t rows = off ? 1 : S;
+    // last residual + final RMSNorm of the rows that are returned
     return vxm_launch_rmsnorm(ctx, m->seq, m->cfg.n_layers && !persistent && !residual_added ? m->ws.dn_out : vxm_parts{},
                               1.0f, m->norm,
                               rows, H, d.eps, out_dev, nullptr, nullptr, var);

@@ -118,7 +118,8 @@ struct vxm_lparams {
     uint32_t *state;         // [0] epoch, [1] workgroups finished in this launch
     float *dump;             // debug: [L + 1][M][1024] rows entering each block, then the output; or null
     // the final RMSNorm of rows fin_r0 .. S - 1 of each segment (gain fin_g, or none: null)
-    // as Q8_0 rows fin_q / fin_d, segment-major
+    // as Q8_0 rows fin_q / fin_d, segment-major; in the fp32 form of the launch (FY) that
+    // of the first fin_r0 rows, as fp32 rows at fin_q
     const float *fin_g;
     int fin_r0;
     int8_t *fin_q;
@@ -641,11 +642,25 @@ __device__ __forceinline__ void row_final_norm(uint8_t *lds, int xr, int gn, int
     if ((t & 15) == 0) dsc[t / 16] = vxm_f2h(d);
 }
 
+// The same norm as fp32 (k_rmsnorm's output), y [1024] of the output row.
+__device__ __forceinline__ void row_final_norm_f32(uint8_t *lds, int xr, int gn, int misc, float eps, float *y) {
+    const int c = 2 * (int)threadIdx.x;
+    const float *x = (const float *)(lds + xr);
+    const float2 g = *(const float2 *)(lds + gn + 4 * c);
+    const float x0 = x[c], x1 = x[c + 1];
+    const double tot = wg_sum_d((double)(x0 * x0) + (double)(x1 * x1), lds, misc);
+    const float mean = (float)(tot / (double)kH);
+    const float sc = __fdiv_rn(1.0f, __fsqrt_rn(mean + eps));
+    *(float2 *)(y + c) = make_float2(bf16r(bf16r(x0 * sc) * g.x), bf16r(bf16r(x1 * sc) * g.y));
+}
+
 // One wave's program for all blocks.  DMA = wave 7: it streams the weight tiles and
 // computes with the others, but reads no exchanged words and loads nothing else, so
 // its only outstanding vector loads are its prefetches and the compiler, which sees
 // none of them, never makes it wait for one.  Waves 0-6 read the exchanged words.
-template <class LS, int MT, bool DMA>
+// FY: the final norm goes out as fp32 rows (the LocEnc's); an instantiation of its own, since
+// a branch for it in the others moved their code (CFM solves at 2 x 11 rows 3.20 -> 3.24 ms).
+template <class LS, int MT, bool DMA, bool FY>
 __device__ __forceinline__ void run_blocks(const vxm_lparams &p, uint8_t *lds, int *bail, uint32_t ep) {
     const int wg = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = p.M, S = p.S, L = p.L;
@@ -1339,7 +1354,7 @@ __device__ __forceinline__ void run_blocks(const vxm_lparams &p, uint8_t *lds, i
         // the last block: row owners add its down projection and write x out (and with
         // fin_g, the x rows their final norm)
         if (!solve && last && row >= 0) {
-            const bool fin = p.fin_g && row % S >= p.fin_r0;
+            const bool fin = FY ? row < p.fin_r0 : p.fin_g && row % S >= p.fin_r0;
             if (!DMA) {
                 if (fin) stage_gain(p.fin_g);
                 poll_partials<(kDSplits * kH / 2 + kPollThreads - 1) / kPollThreads>(
@@ -1356,7 +1371,10 @@ __device__ __forceinline__ void run_blocks(const vxm_lparams &p, uint8_t *lds, i
             if (!DMA && p.dump)
                 for (int c = tid * 4; c < kH; c += kPollThreads * 4)
                     *(float4 *)(p.dump + ((size_t)L * M + row) * kH + c) = *(const float4 *)(lds + LS::XR + c * 4);
-            if (fin) {
+            if (FY) {
+                if (fin)
+                    row_final_norm_f32(lds, LS::XR, LS::GN, LS::MISC, p.eps, (float *)p.fin_q + (size_t)row * kH);
+            } else if (fin) {
                 const int orow = (row / S) * (S - p.fin_r0) + row % S - p.fin_r0;
                 row_final_norm(lds, LS::XR, LS::GN, LS::MISC, p.eps, p.variant, p.fin_q + (size_t)orow * kH,
                                p.fin_d + (size_t)orow * (kH / 32));
@@ -1499,7 +1517,7 @@ __device__ __forceinline__ void run_blocks(const vxm_lparams &p, uint8_t *lds, i
     }
 }
 
-template <class LS, int MT>
+template <class LS, int MT, bool FY = false>
 __global__ __launch_bounds__(kThreads, 1) void k_locdit_persistent(vxm_lparams p) {
     // All of the workgroup's LDS is this one dynamic array, so it starts at address 0
     // (the weight DMAs address it absolutely) and every layout offset is aligned.
@@ -1521,8 +1539,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_locdit_persistent(vxm_lparams p
     __builtin_amdgcn_s_waitcnt(kVmcnt0);
     lds_barrier();
     const uint32_t ep = *ep_sh;
-    if ((tid >> 6) == kWaves - 1) run_blocks<LS, MT, true>(p, lds, bail, ep);
-    else run_blocks<LS, MT, false>(p, lds, bail, ep);
+    if ((tid >> 6) == kWaves - 1) run_blocks<LS, MT, true, FY>(p, lds, bail, ep);
+    else run_blocks<LS, MT, false, FY>(p, lds, bail, ep);
     // every weight load of wave 7 has landed before the workgroup ends
     vm_wait<0>();
     lds_barrier();
@@ -1682,16 +1700,18 @@ int vxm_locdit_persistent_run(vxm_ctx *ctx, const vxm_block_dims &d, const std::
             return vxm_fail(ctx, VXM_ERR_BACKEND, "persistent blocks: buffer set-up failed");
         }
         // the kernels' LDS limit, set here rather than at a launch that may be under graph capture
-        const void *kern[6] = {(const void *)k_locdit_persistent<ShapeDitMha, 1>,
+        const void *kern[8] = {(const void *)k_locdit_persistent<ShapeDitMha, 1>,
                                (const void *)k_locdit_persistent<ShapeDitMha, 2>,
                                (const void *)k_locdit_persistent<ShapeDitMha, 3>,
+                               (const void *)k_locdit_persistent<ShapeDitMha, 1, true>,
+                               (const void *)k_locdit_persistent<ShapeDitGqa, 1, true>,
                                (const void *)k_locdit_persistent<ShapeDitGqa, 1>,
                                (const void *)k_locdit_persistent<ShapeDitGqa, 2>,
                                (const void *)k_locdit_persistent<ShapeDitGqa, 3>};
         bool attr_ok = true;
-        for (int i = 0; i < 6; i++)
+        for (int i = 0; i < 8; i++)
             attr_ok &= hipFuncSetAttribute(kern[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           i < 3 ? ShapeDitMha::BYTES : ShapeDitGqa::BYTES) == hipSuccess;
+                                           i < 4 ? ShapeDitMha::BYTES : ShapeDitGqa::BYTES) == hipSuccess;
         if (!attr_ok) {
             (void)hipGetLastError();
             vxm_locdit_persistent_free(st);
@@ -1721,12 +1741,17 @@ int vxm_locdit_persistent_run(vxm_ctx *ctx, const vxm_block_dims &d, const std::
     prm.state = st->state;
     prm.dump = dump;
     if (fin.g) {
-        if (fin.r0 < 0 || fin.r0 >= S || (!sv && (!fin.q || !fin.d)))
+        if (fin.r0 < 0 || fin.r0 >= S || (!sv && !fin.y && (!fin.q || !fin.d)) ||
+            (fin.y && (sv || M != S || S > 16 || fin.r0)))
             return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "persistent blocks: final norm rows %d of %d", fin.r0, S);
         prm.fin_g = fin.g;
         prm.fin_r0 = fin.r0;
         prm.fin_q = fin.q;
         prm.fin_d = fin.d;
+        if (fin.y) {
+            prm.fin_r0 = fin.n;
+            prm.fin_q = (int8_t *)fin.y;
+        }
     }
     if (sv) {
         prm.n_eval = sv->n_eval;
@@ -1789,9 +1814,13 @@ int vxm_locdit_persistent_run(vxm_ctx *ctx, const vxm_block_dims &d, const std::
     vxm_launch_slot *slot = nullptr;
     bool capturing = false;
     if (int rc = vxm_ordered_launch_begin(ctx, &slot, &capturing)) return rc;
-#define VXM_LP_LAUNCH(LS, MT)                                                                                \
-    hipLaunchKernelGGL((k_locdit_persistent<LS, MT>), dim3(kG), dim3(kThreads), (unsigned)LS::BYTES, ctx->stream, prm)
-    if (d.nkv == 16) {
+#define VXM_LP_LAUNCH(LS, ...)                                                                               \
+    hipLaunchKernelGGL((k_locdit_persistent<LS, __VA_ARGS__>), dim3(kG), dim3(kThreads), (unsigned)LS::BYTES, \
+                       ctx->stream, prm)
+    if (fin.y) {
+        if (d.nkv == 16) VXM_LP_LAUNCH(ShapeDitMha, 1, true);
+        else VXM_LP_LAUNCH(ShapeDitGqa, 1, true);
+    } else if (d.nkv == 16) {
         if (mt == 1) VXM_LP_LAUNCH(ShapeDitMha, 1);
         else if (mt == 2) VXM_LP_LAUNCH(ShapeDitMha, 2);
         else VXM_LP_LAUNCH(ShapeDitMha, 3);

@@ -114,6 +114,9 @@ struct vxm_lfinal {
     int r0 = 0;
     int8_t *q = nullptr;
     uint16_t *d = nullptr;
+    // instead of q and d: fp32 rows y of the first n rows (one segment)
+    float *y = nullptr;
+    int n = 0;
 };
 // A whole CFM solve in the launch (vxm_cfm_solve's Euler loop): n_eval steps of sizes dts
 // (host), time rows tc [n_eval][H], segment 0 with mu (n_mu = 1) or none, cond rows
