@@ -1,6 +1,7 @@
 """The MFMA attention at the edges of its query tiles (32), key blocks (32), rounds (128 keys) and
-head pairs, through a block: causal behind an existing context, fewer queries than a tile, and
-scores whose row max keeps rising over the keys."""
+head pairs, through a block: causal behind an existing context, and scores whose row max keeps
+rising over the keys.  Fewer queries than a tile take the scalar kernel, here with long contexts
+and with a value row that overflows the f16 cache."""
 import numpy as np
 import pytest
 
@@ -64,4 +65,38 @@ def test_block_noncausal_tile_edges(vxm_ctx, orc):
         ref = orc.minicpm4_block(orc_cfg(orc, c), to_orc(orc, lw), x, None, None, 0, 0, 1)
         y = xd.cpu().numpy().astype(np.float64)
         assert np.linalg.norm(y - ref) <= 5e-3 * np.linalg.norm(ref), M
+    model.free()
+
+
+@pytest.mark.parametrize("M,pos,hd", [(2, 127, 128), (5, 300, 64), (31, 98, 128), (31, 1000, 64)])
+def test_overflowing_value_row_reaches_no_earlier_token(vxm_ctx, orc, M, pos, hd):
+    """The last token's value row holds infinities (past f16); the tokens before it do not see it."""
+    import vxm
+
+    rng = np.random.default_rng(M + pos)
+    H, nh, nkv, F, cap = 256, 4, 2, 256, (M + pos + 63) // 64 * 64
+    lw = rand_layer(orc, rng, H, nh, nkv, hd, F)
+    wv = rng.normal(0, 0.02, (nkv * hd, H)).astype(np.float32)
+    wv[:, 0] = 0
+    wv[::hd] = 0
+    wv[::hd, 0] = 1e6            # dim 0 of every value head: 1e6 x channel 0 of the normalised row
+    lw["v_proj"] = orc.quantize_rows(wv, orc.QUANT_REF)
+    k = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    v = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    x = rng.normal(0, 1, (M, H)).astype(np.float32)
+    x[:, 0] = 0                  # no other token has channel 0
+    model = vxm.MiniCPM4(vxm_ctx, cfg_dict(H, 1, nh, nkv, hd, F), [lw])
+    kv = vxm.KVCache(vxm_ctx, 1, nkv, hd, cap)
+    ys = []
+    for big in (0.0, 5.0):
+        kv.upload(0, k, v)
+        x[-1, 0] = big
+        xd = _dev(x)
+        model.block(kv, 0, xd, pos)
+        vxm_ctx.sync()
+        ys.append(xd.cpu().numpy())
+    assert np.isfinite(ys[0]).all()
+    assert np.isinf(kv.download(0)[1].view(np.float16)[:, pos + M - 1, 0]).all()
+    assert np.array_equal(ys[0][:-1], ys[1][:-1])
+    kv.free()
     model.free()

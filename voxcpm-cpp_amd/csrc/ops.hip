@@ -680,11 +680,13 @@ int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const
     if (M <= 0) return VXM_OK;
     if (hd > 256 || hd <= 0 || nkv <= 0 || nh % nkv)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "attention: head_dim %d / heads %d,%d unsupported", hd, nh, nkv);
-    // the MFMA kernel: the queries of a single segment, a tile of them or at least two whose
-    // keys k_attention would walk for longer than a tile's padding costs (16 heads of 128:
-    // 24 queries over 24 keys 8.9 against 8.6 us, over 474 keys 14.7 against 23.5)
+    // the MFMA kernel: the queries of a single segment, from a tile of them.  Fewer keep
+    // k_attention although it is slower over a long context (16 heads of 128, 24 queries over
+    // 474 keys: 23.5 against 14.7 us): it reads only the keys that a query sees, so a cache row
+    // of infinities or NaN reaches no query before it, and its queries and probabilities stay
+    // fp32 (a BF16 query past f16's range stays finite).
     const int64_t span = causal ? kv_base + M : M;
-    if (S == M && (M >= AQ || (M >= 2 && span > 128)) && span <= cap && (hd == 128 || hd == 64)) {
+    if (S == M && M >= AQ && span <= cap && (hd == 128 || hd == 64)) {
         if (hd == 128)
             launch_attention_mfma<128>(ctx, q, kc, vc, out, M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
         else
