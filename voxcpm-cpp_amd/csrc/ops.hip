@@ -405,16 +405,18 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
 // piece p of V^T row d at p ^ ((d ^ d >> 3) & 15), so an operand read of 16 lanes and a
 // transposing write of 64 fall on (nearly) distinct banks.
 //
-// Bound by the VALU work per score (max, exp, the double sum, the hi / lo split: ~16
-// instructions) and the matrix products next to it, two waves per SIMD, and by what a
+// Bound by the VALU work per score (max, exp, the double sum, the hi / lo split: ~22
+// instructions) and the matrix products next to it, at two waves per SIMD (two heads per
+// workgroup; one wave with one head, as the LDS holds one workgroup), and by what a
 // wave waits while its loads queue at the address unit.  The tiles with the most keys
-// are launched first.  Measured on 16 / 2 heads x 128, causal: 2048 tokens 57 us, 1000
-// tokens 28, 512 tokens 16, 256 tokens 11.  (A workgroup per head whose eight waves split
-// each 512-key chunk, with the scores' exponentials through LDS, two barriers and a
-// drained load queue per chunk, took 134 and 46 us at 2048 and 1000 tokens; one pass over
-// at most 512 keys that way 17 us.)  Variants: the V loads issued after the scores 63 us at
-// 2048 tokens, two chains of score products 58.5, the max followed exactly (a rescale in
-// almost every block) with a general expf and separate masks 74.
+// are launched first.  Measured on 16 / 2 heads x 128, causal, back to back: 2048 tokens
+// 56.2 us, 1500 tokens 38.3, 512 tokens 15.4, 333 tokens 12.8, 77 tokens 8.3.  (A workgroup
+// per head whose eight waves split each 512-key chunk, with the scores' exponentials through
+// LDS, two barriers and a drained load queue per chunk, one pass over at most 512 keys:
+// 121.9, 75.9, 15.6, 14.1 and 10.4 us.)  Variants: the V loads issued after the scores +6 us at
+// 2048 tokens, two chains of score products +1.5, the max followed exactly (a rescale in
+// almost every block) with separate masks +15; expf without its range checks -0.3, as 2^(x
+// log2 e) at once with the product's rounding error as a factor -2.7, but 1.26 ulp against 0.86.
 // ---------------------------------------------------------------------------
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -426,18 +428,6 @@ constexpr int AQ = 32;
 // sum, and the rescale of O is rare instead of due in almost every block (any of a
 // wave's 32 queries may have a new max).
 constexpr float kMaxSlack = 8.0f;
-
-// exp(x) as 2^(x log2 e): v_exp_f32 (1 ulp) of the product's leading part, its rounding
-// error and log2 e's added as a first-order factor (they are below 2^-17).  No range
-// reduction: results below 2^-126 are 0, which no sum of e with a largest term near 1
-// notices.  exp_near(-inf) = 0, NaN stays NaN.
-__device__ __forceinline__ float exp_near(float x) {
-    const float L = 1.44269502f, Lo = 1.92596299e-8f;   // log2 e in two parts
-    const float ph = x * L;
-    const float pl = fmaxf(__builtin_fmaf(x, Lo, __builtin_fmaf(x, L, -ph)), -1.0f);   // -inf - -inf is no error
-    const float e = __builtin_amdgcn_exp2f(ph);
-    return __builtin_fmaf(e, pl * 0.693147182f, e);
-}
 
 template <int HD, int NH>
 __global__ __launch_bounds__(256 * NH, 1) void k_attention_mfma(
@@ -564,7 +554,7 @@ __global__ __launch_bounds__(256 * NH, 1) void k_attention_mfma(
             const float mneg = m == -INFINITY ? 0.0f : -m;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                s[v] = exp_near(__builtin_fmaf(s[v], scale, mneg));
+                s[v] = expf(__builtin_fmaf(s[v], scale, mneg));
                 lsum += (double)s[v];
             }
 #pragma unroll
