@@ -82,7 +82,11 @@ int         vxm_set_path(vxm_ctx *ctx, int path);
  * position, a time step) are recorded with the values they had.  Run the
  * sequence once eagerly first: a call that would have to grow a scratch
  * buffer or set up a single-launch kernel's buffers (and so allocate and
- * synchronise) fails under capture with VXM_ERR_INVALID_ARG.
+ * synchronise) fails under capture with VXM_ERR_INVALID_ARG.  A recording
+ * holds the buffers of the moment it was made: a later eager call that outgrows
+ * them (a forward of more rows, or at positions past the rope table, than any
+ * before it on the model; a larger matmul on the context) replaces them, and
+ * the recording has to be made again.  A model's call of fewer rows never does.
  * vxm_locdit_forward stages host-computed time embeddings and cannot be
  * captured; vxm_cfm_solve records and replays its own Euler loop.  Every tag
  * a kernel compares lives in device memory, so every replay is exact. */

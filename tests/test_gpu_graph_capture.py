@@ -176,3 +176,91 @@ def test_capture_refuses_first_single_launch_blocks(orc):
                 g.free()
         finally:
             enc.free()
+
+
+def _model(vxm, orc, ctx, seed, H=512, nh=4, nkv=2, hd=128, F=1024):
+    from test_gpu_minicpm4 import cfg_dict, rand_layer
+
+    rng = np.random.default_rng(seed)
+    m = vxm.MiniCPM4(ctx, cfg_dict(H, 1, nh, nkv, hd, F), [rand_layer(orc, rng, H, nh, nkv, hd, F)],
+                     (1 + rng.normal(0, 0.02, H)).astype(np.float32))
+    return m, vxm.KVCache(ctx, 1, nkv, hd, 2048)
+
+
+def test_captured_forward_outlives_shorter_calls(orc):
+    """A forward recorded at 512 rows replays exactly after eager forwards of fewer rows, whose
+    K-split slices fit the workspace that it holds; and such a forward captures without a
+    run of its own, since nothing has to grow for it."""
+    import torch
+    import vxm
+
+    with vxm.Context(0) as ctx:
+        m, kv = _model(vxm, orc, ctx, 31)
+        rng = np.random.default_rng(32)
+        xs = {M: torch.from_numpy(rng.normal(0, 1, (M, 512)).astype(np.float32)).to("cuda:0")
+              for M in (512, 130, 128, 100, 65, 64, 31, 2)}
+        bufs = {M: x.clone() for M, x in xs.items()}
+        torch.cuda.synchronize()
+        m.forward(kv, bufs[512], 0)
+        ctx.sync()
+        ref = {512: bufs[512].cpu().numpy()}
+        graphs = {}
+        try:
+            for M in xs:   # only the longest has run
+                ctx.capture_begin()
+                try:
+                    m.forward(kv, bufs[M], 0)
+                finally:
+                    graphs[M] = ctx.capture_end()
+            for M in list(xs)[1:] + [512]:
+                y = xs[M].clone()
+                torch.cuda.synchronize()
+                m.forward(kv, y, 0)
+                ctx.sync()
+                ref.setdefault(M, y.cpu().numpy())
+                for G in (512, M, 512):
+                    bufs[G].copy_(xs[G])
+                    torch.cuda.synchronize()
+                    graphs[G].launch()
+                    ctx.sync()
+                    assert np.array_equal(bufs[G].cpu().numpy(), ref[G]), (M, G)
+        finally:
+            for g in graphs.values():
+                g.free()
+        kv.free()
+        m.free()
+
+
+def test_capture_refuses_model_growth(orc):
+    """More rows than the model's workspace holds, or a position past its rope table, fail
+    under capture with a clear error; after one eager run both capture."""
+    import torch
+    import vxm
+
+    with vxm.Context(0) as ctx:
+        m, kv = _model(vxm, orc, ctx, 33)
+        x = torch.zeros((40, 512), dtype=torch.float32, device="cuda:0")
+        torch.cuda.synchronize()
+        m.forward(kv, x[:8], 0)
+        ctx.sync()
+        for rows, pos, what in ((40, 0, "workspace"), (8, 1500, "rope table")):
+            for attempt in range(2):
+                ctx.capture_begin()
+                err = None
+                try:
+                    m.forward(kv, x[:rows], pos)
+                except vxm.VxmError as e:
+                    err = e
+                finally:
+                    try:
+                        ctx.capture_end().free()
+                    except vxm.VxmError:
+                        pass   # the capture recorded nothing
+                if attempt == 0:
+                    assert err is not None and err.code == 1 and what in str(err) and "capture" in str(err), err
+                    m.forward(kv, x[:rows], pos)
+                    ctx.sync()
+                else:
+                    assert err is None, err
+        kv.free()
+        m.free()

@@ -218,6 +218,7 @@ static int locenc_bufs(vxm_locenc *m, int64_t S, int64_t P) {
     size_t total = 0;
     for (size_t p : parts) total += (p + 255) & ~(size_t)255;
     if (total > m->buf_bytes) {
+        if (int rc = vxm_may_grow(ctx, "locenc: buffers", total)) return rc;
         VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (m->buf) VXM_HIP(ctx, hipFree(m->buf));
         m->buf = nullptr;
@@ -537,6 +538,7 @@ extern "C" int vxm_prompt_prefill(vxm_lm_update *u, vxm_kv_cache *tslm_kv, vxm_k
     const size_t cat_b = ((size_t)n * 2 * L * 4 + 255) & ~(size_t)255, q_b = ((size_t)n * 2 * L + 255) & ~(size_t)255,
                  d_b = (size_t)n * (2 * L / 32) * 2;
     if (u->pbytes < cat_b + q_b + d_b) {
+        if ((rc = vxm_may_grow(ctx, "prompt_prefill: fusion buffers", cat_b + q_b + d_b))) return rc;
         VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (u->pbuf) VXM_HIP(ctx, hipFree(u->pbuf));
         u->pbuf = nullptr;

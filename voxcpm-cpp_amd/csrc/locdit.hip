@@ -303,6 +303,7 @@ static int ensure_bufs(vxm_locdit *m, int64_t S, int64_t P, int64_t Pc, int64_t 
     size_t total = 0;
     for (auto &p : parts) total += (p.bytes + 255) & ~(size_t)255;
     if (total > m->buf_bytes) {
+        if (int rc = vxm_may_grow(ctx, "locdit: buffers", total)) return rc;
         VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (m->buf) VXM_HIP(ctx, hipFree(m->buf));
         m->buf = nullptr;

@@ -44,19 +44,19 @@ static const float kVoxcpm2RopeShortFactors[64] = {
 int vxm_ws_ensure(vxm_ctx *ctx, vxm_workspace &ws, int64_t M, int64_t H, int64_t qd, int64_t kvd, int64_t F,
                   int64_t local_kv) {
     const int64_t kmax = std::max(std::max(H, qd), F);
-    // small batches: the projections may arrive as K-split slices of the small-M GEMM
-    const int pf = M <= VXM_SMALL_MAX_ROWS ? VXM_MAX_PARTS : 1;
-    ws.max_parts = pf;
+    // the projections of small batches may arrive as K-split slices of the small-M GEMM;
+    // every size below grows with M, so a call of fewer rows finds its room
+    auto slices = [&](int64_t N) { return (size_t)(vxm_part_rows(ctx, M, N) * N * 4); };
     struct Part { size_t bytes; void **dst; };
     std::vector<Part> parts = {
         {(size_t)(M * kmax), (void **)&ws.xq},
         {(size_t)(M * (kmax / 32) * 2), (void **)&ws.xd},
-        {(size_t)(pf * M * (qd + 2 * kvd) * 4), (void **)&ws.qkv},
+        {slices(qd + 2 * kvd), (void **)&ws.qkv},
         {(size_t)(M * qd * 4), (void **)&ws.q},
         {(size_t)(M * qd * 4), (void **)&ws.att},
-        {(size_t)(pf * M * H * 4), (void **)&ws.o},
-        {(size_t)(pf * M * 2 * F * 4), (void **)&ws.gu},
-        {(size_t)(pf * M * H * 4), (void **)&ws.dn},
+        {slices(H), (void **)&ws.o},
+        {slices(2 * F), (void **)&ws.gu},
+        {slices(H), (void **)&ws.dn},
         {(size_t)(local_kv * 2), (void **)&ws.lk},
         {(size_t)(local_kv * 2), (void **)&ws.lv},
     };
@@ -67,6 +67,7 @@ int vxm_ws_ensure(vxm_ctx *ctx, vxm_workspace &ws, int64_t M, int64_t H, int64_t
         for (auto &p : parts) { *p.dst = b; b += (p.bytes + 255) & ~(size_t)255; }
         return VXM_OK;
     }
+    if (int rc = vxm_may_grow(ctx, "workspace", total)) return rc;
     VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (ws.base) VXM_HIP(ctx, hipFree(ws.base));
     ws.base = nullptr;
@@ -174,6 +175,7 @@ int vxm_rope_ensure(vxm_ctx *ctx, vxm_block_dims &d, int64_t n_pos) {
     if (n_pos > (1 << 24)) return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "rope: position %lld", (long long)n_pos);
     const int64_t rows = std::max<int64_t>(std::max<int64_t>(n_pos, 2 * (int64_t)d.rope_rows), 1024);
     const int64_t half = d.hd / 2;
+    if (int rc = vxm_may_grow(ctx, "rope table", (size_t)(rows * half * 8))) return rc;
     std::vector<float> host((size_t)(rows * half * 2));
     int rc = vxm_host_rope_cache(d.rope_base, d.hd, d.ff_host.empty() ? nullptr : d.ff_host.data(), 0,
                                  (int32_t)rows, host.data());
@@ -217,7 +219,7 @@ int vxm_block_run(vxm_ctx *ctx, const vxm_block_dims &d, const vxm_block &b, vxm
         fused_rope = vxm_launch_qkv_rope(ctx, b.wqkv, ws.xq, ws.xd, M, qe, d.rope_rows, &rc);
         if (rc) return rc;
     }
-    if (!fused_rope && (rc = vxm_launch_mul_mat_parts(ctx, b.wqkv, ws.xq, ws.xd, M, ws.qkv, ws.max_parts, &np)))
+    if (!fused_rope && (rc = vxm_launch_mul_mat_parts(ctx, b.wqkv, ws.xq, ws.xd, M, ws.qkv, VXM_MAX_PARTS, &np)))
         return rc;
     if (local) {
         // fresh K/V within each segment: RoPE, attention and the output's Q8_0 in one launch
@@ -236,7 +238,7 @@ int vxm_block_run(vxm_ctx *ctx, const vxm_block_dims &d, const vxm_block &b, vxm
                                        site.seg_stride, site.S, site.cache_pos0, site.causal, ws.xq, ws.xd, var)))
             return rc;
     }
-    if ((rc = vxm_launch_mul_mat_parts(ctx, b.wo, ws.xq, ws.xd, M, ws.o, ws.max_parts, &np))) return rc;
+    if ((rc = vxm_launch_mul_mat_parts(ctx, b.wo, ws.xq, ws.xd, M, ws.o, VXM_MAX_PARTS, &np))) return rc;
     // x = bf16(x + scale*bf16(o)); post-attention norm -> Q8_0
     if ((rc = vxm_launch_rmsnorm(ctx, x, vxm_parts{ws.o, np, M * d.H}, d.res_scale, b.g_post, M, d.H, d.eps, nullptr,
                                  ws.xq, ws.xd, var)))
@@ -253,12 +255,12 @@ int vxm_block_run(vxm_ctx *ctx, const vxm_block_dims &d, const vxm_block &b, vxm
         pq = fq;
         pd = fd;
     } else {
-        if ((rc = vxm_launch_mul_mat_parts(ctx, b.wgu, ws.xq, ws.xd, M, ws.gu, ws.max_parts, &np))) return rc;
+        if ((rc = vxm_launch_mul_mat_parts(ctx, b.wgu, ws.xq, ws.xd, M, ws.gu, VXM_MAX_PARTS, &np))) return rc;
         if ((rc = vxm_launch_swiglu_quant(ctx, vxm_parts{ws.gu, np, M * 2 * d.F}, M, d.F, 2 * d.F, ws.xq, ws.xd,
                                           nullptr, var)))
             return rc;
     }
-    if ((rc = vxm_launch_mul_mat_parts(ctx, b.wd, pq, pd, M, ws.dn, ws.max_parts, &np))) return rc;
+    if ((rc = vxm_launch_mul_mat_parts(ctx, b.wd, pq, pd, M, ws.dn, VXM_MAX_PARTS, &np))) return rc;
     ws.dn_out = vxm_parts{ws.dn, np, M * d.H};
     return VXM_OK;
 }

@@ -1937,8 +1937,8 @@ static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_pa
     p.mtiles = (int)((M + VXM_SMALL_TILE_ROWS - 1) / VXM_SMALL_TILE_ROWS);
     p.mt = (int)((M + 16 * p.mtiles - 1) / (16 * p.mtiles));
     p.groups = (int)(N / (16 * kSmallRG));
-    int s = 1;
-    while (s * 2 <= max_parts && s * 2 <= stages && (int64_t)p.groups * p.mtiles * s < ctx->n_cu) s *= 2;
+    int s = vxm_parts_limit(ctx, M, N);   // a power of two
+    while (s > max_parts || s > stages) s /= 2;
     const int per = (stages + s - 1) / s;   // stages per split
     p.bps = per * kSmallStage;
     p.splits = (nb + p.bps - 1) / p.bps;
@@ -2033,7 +2033,7 @@ static int launch_gemm_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
                             (long long)M, (long long)w->n, (long long)w->k, pbytes, wk->parts_bytes);
         scratch = wk->parts;
     } else {
-        int rc = vxm_ensure_parts(ctx, pbytes);
+        int rc = vxm_ensure_parts(ctx, (size_t)(vxm_part_rows(ctx, M, w->n) * w->n) * sizeof(float));
         if (rc) return rc;
         scratch = (float *)ctx->parts_buf;
     }

@@ -139,16 +139,14 @@ static bool capturing(vxm_ctx *ctx) {
     return st != hipStreamCaptureStatusNone;
 }
 
-// A scratch buffer that must grow cannot be replaced under graph capture (the
-// free and the allocation would synchronise the stream being recorded).
-#define VXM_NO_GROWTH_UNDER_CAPTURE(ctx, what, bytes)                                                    \
-    do {                                                                                                 \
-        if (capturing(ctx))                                                                              \
-            return vxm_fail((ctx), VXM_ERR_INVALID_ARG,                                                  \
-                            "%s of %zu bytes would have to grow under graph capture: run the sequence " \
-                            "once before capturing it",                                                  \
-                            (what), (size_t)(bytes));                                                    \
-    } while (0)
+// A buffer that must grow cannot be replaced under graph capture (the free and the
+// allocation would synchronise the stream being recorded).
+int vxm_may_grow(vxm_ctx *ctx, const char *what, size_t bytes) {
+    if (!capturing(ctx)) return VXM_OK;
+    return vxm_fail(ctx, VXM_ERR_INVALID_ARG,
+                    "%s of %zu bytes would have to grow under graph capture: run the sequence once before capturing it",
+                    what, bytes);
+}
 
 // ---- one launch order per device for the single-launch kernels --------------
 
@@ -340,7 +338,7 @@ extern "C" int vxm_memcpy_d2h(vxm_ctx *ctx, void *dst_host, const void *src_dev,
 
 int vxm_ensure_act(vxm_ctx *ctx, size_t bytes) {
     if (ctx->act_bytes >= bytes) return VXM_OK;
-    VXM_NO_GROWTH_UNDER_CAPTURE(ctx, "activation scratch", bytes);
+    if (int rc = vxm_may_grow(ctx, "activation scratch", bytes)) return rc;
     VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (ctx->act_buf) VXM_HIP(ctx, hipFree(ctx->act_buf));
     ctx->act_buf = nullptr;
@@ -356,7 +354,7 @@ int vxm_ensure_act(vxm_ctx *ctx, size_t bytes) {
 
 int vxm_ensure_parts(vxm_ctx *ctx, size_t bytes) {
     if (ctx->parts_bytes >= bytes) return VXM_OK;
-    VXM_NO_GROWTH_UNDER_CAPTURE(ctx, "GEMM slice scratch", bytes);
+    if (int rc = vxm_may_grow(ctx, "GEMM slice scratch", bytes)) return rc;
     VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (ctx->parts_buf) VXM_HIP(ctx, hipFree(ctx->parts_buf));
     ctx->parts_buf = nullptr;
@@ -371,7 +369,7 @@ int vxm_ensure_parts(vxm_ctx *ctx, size_t bytes) {
 
 int vxm_ensure_split(vxm_ctx *ctx, size_t bytes, size_t n_counters) {
     if (ctx->split_bytes < bytes || ctx->split_ncnt < n_counters)
-        VXM_NO_GROWTH_UNDER_CAPTURE(ctx, "GEMM split scratch", bytes);
+        if (int rc = vxm_may_grow(ctx, "GEMM split scratch", bytes)) return rc;
     if (ctx->split_bytes < bytes) {
         VXM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->split_buf) VXM_HIP(ctx, hipFree(ctx->split_buf));

@@ -230,6 +230,27 @@ constexpr int VXM_SMALL_MAX_ROWS = 128;  // rows of x the small-M GEMM takes
 constexpr int VXM_SMALL_TILE_ROWS = 64;  // of them in one row tile
 constexpr int VXM_MAX_PARTS = 8;         // its K splits
 
+// The K splits into which the small-M GEMM cuts a product of M rows and N columns at
+// most (it doubles them while its grid leaves CUs idle): what its plans use.
+inline int vxm_parts_limit(const vxm_ctx *ctx, int64_t M, int64_t N) {
+    if (M > VXM_SMALL_MAX_ROWS) return 1;
+    const int64_t wgs = N / 64 * ((M + VXM_SMALL_TILE_ROWS - 1) / VXM_SMALL_TILE_ROWS);
+    int s = 1;
+    while (2 * s <= VXM_MAX_PARTS && wgs * s < ctx->n_cu) s *= 2;
+    return s;
+}
+// Rows of N values that hold the slices of M rows and those of any fewer (64 rows may have
+// more splits than 65): a buffer of so many never grows for a shorter call, which would
+// free it under a recorded graph.
+inline int64_t vxm_part_rows(const vxm_ctx *ctx, int64_t M, int64_t N) {
+    int64_t rows = M;
+    for (int64_t tile : {VXM_SMALL_TILE_ROWS, VXM_SMALL_MAX_ROWS}) {
+        const int64_t m = M < tile ? M : tile, r = m * vxm_parts_limit(ctx, m, N);
+        if (r > rows) rows = r;
+    }
+    return rows;
+}
+
 // The product as up to max_parts slices of M x N at y, y + M*N, ...; *parts = the
 // number written (1 unless the small-M GEMM splits K).
 int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd,
@@ -248,6 +269,8 @@ struct vxm_qkv_epi {
 };
 bool vxm_launch_qkv_rope(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                          const vxm_qkv_epi &qe, int cs_rows, int *rc);
+// VXM_OK where a buffer that must grow may be replaced, an error under graph capture.
+int vxm_may_grow(vxm_ctx *ctx, const char *what, size_t bytes);
 int vxm_ensure_act(vxm_ctx *ctx, size_t bytes);
 // Finds the allocation-free matmul's scratch array on ctx's (current) device.
 int vxm_scratch_setup(vxm_ctx *ctx);
