@@ -165,6 +165,18 @@ int64_t vxm_stream_read_sink_words(int32_t n, const int64_t *bytes);
 int vxm_mul_mat_q8_0_noalloc(vxm_ctx *ctx, const vxm_weight *w, const float *x_dev, int64_t M,
                              float *y_dev);
 size_t vxm_noalloc_scratch_bytes(void);
+/* Test hook, host only: the kernel that vxm_mul_mat_q8_0 (fp32_rows != 0) or
+ * vxm_mul_mat_q8_0_q8_0 runs for an n x k weight and m rows in 16-byte aligned buffers
+ * apart from each other, on a device of n_cu CUs, and its K splits. */
+#define VXM_KERNEL_NONE 0      /* refused: operands of 2 GiB and more */
+#define VXM_KERNEL_GEMV 1      /* weight-streaming GEMV */
+#define VXM_KERNEL_GEMV_F32 2  /* ... that quantizes its rows itself */
+#define VXM_KERNEL_SMALL 3     /* register-fed small-M GEMM */
+#define VXM_KERNEL_SMALL_F32 4 /* ... that quantizes its rows itself */
+#define VXM_KERNEL_TILE 5      /* DMA-fed tile GEMM */
+#define VXM_KERNEL_STAGED 6    /* register-staged tile GEMM (k % 256 != 0) */
+int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t fp32_rows,
+                          int32_t *kernel, int32_t *splits);
 /* Debug: int32 per-block sums of vec_dot_q8_0_q8_0, out[(m*N + n)*(K/32) + b]. */
 int vxm_block_dots_q8_0(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq_dev,
                         const uint16_t *xd_dev, int64_t M, int32_t *out_dev);

@@ -87,3 +87,39 @@ def test_graft_entry_has_build_and_smoke():
     m = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(m)
     assert callable(m.build) and callable(m.smoke)
+
+
+def test_mul_mat_plans():
+    """The kernel and K splits of the dispatch at the lines between its kernels."""
+    import vxm
+
+    plan = vxm.host_mul_mat_plan
+    for n, k, m, fp32, want in [
+            (6144, 2048, 7, 0, ("gemv", 1)), (6144, 2048, 8, 0, ("small", 4)), (12288, 2048, 16, 0, ("small", 2)),
+            # above one row tile: the tile GEMM where it needs no K split
+            (12288, 2048, 17, 0, ("tile", 1)), (2048, 2048, 17, 0, ("small", 8)), (2048, 2048, 64, 0, ("small", 8)),
+            (2048, 2048, 65, 0, ("small", 4)), (2048, 2048, 128, 0, ("small", 4)), (2048, 2048, 129, 0, ("tile", 2)),
+            (2560, 2048, 64, 0, ("small", 8)), (2560, 2048, 65, 0, ("tile", 3)),
+            (2048, 2080, 100, 0, ("staged", 4)), (96, 2048, 16, 0, ("tile", 4)),
+            # fp32 rows
+            (6144, 2048, 1, 1, ("gemv_f32", 1)), (6144, 2048, 3, 1, ("gemv_f32", 1)), (6144, 2048, 4, 1, ("gemv", 1)),
+            (1024, 1024, 5, 1, ("gemv_f32", 1)), (1024, 1024, 6, 1, ("gemv", 1)),
+            (6144, 2048, 16, 1, ("small_f32", 4)), (6144, 2048, 32, 1, ("small", 4)), (12288, 2048, 8, 1, ("small", 2)),
+            (2048, 2048, 32, 1, ("small_f32", 8)), (2048, 2048, 33, 1, ("small", 8))]:
+        assert plan(n, k, m, fp32_rows=fp32) == want, (n, k, m, fp32, plan(n, k, m, fp32_rows=fp32))
+    for path, want in ((vxm.PATH_GEMV, "gemv"), (vxm.PATH_MFMA, "small"), (vxm.PATH_MFMA_TILED, "tile")):
+        assert plan(2048, 2048, 16, path, fp32_rows=False)[0] == want
+
+
+def test_mul_mat_plan_takes_operands_up_to_2_gib():
+    """Up to 64 rows every weight below 2 GiB of quants runs: the small-M GEMM takes those that
+    the tile GEMM, which addresses whole tiles past the last row, refuses."""
+    import vxm
+
+    for k in (256, 2048, 6144):
+        n = ((1 << 31) // k - 1) // 64 * 64
+        assert n * k < 1 << 31 and (n + 128) * k >= 1 << 31
+        for m in (8, 16, 17, 24, 33, 64):
+            assert vxm.host_mul_mat_plan(n, k, m)[0] == "small", (n, k, m)
+        assert vxm.host_mul_mat_plan(n, k, 65)[0] == "none"
+        assert vxm.host_mul_mat_plan(n - 192, k, 17)[0] != "none"

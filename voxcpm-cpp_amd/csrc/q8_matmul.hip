@@ -1969,12 +1969,14 @@ constexpr int kSmallAlwaysRows = 16;
 // 320 workgroups, 16.6 against 15.7 us at M = 100.  With three row tiles (M > 128) it
 // loses: 2048 x 6144 30.1 against 23.4 us at M = 150.  K is bounded there so that the
 // slices and the quantized rows of any such product fit the allocation-free entry's
-// scratch together.
+// scratch together.  Up to 64 rows it also takes what it can address and the tile GEMM
+// cannot (N K just below 2^31).
 static bool small_wins(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                        int max_parts, bool fixup, SmallPlan &p) {
     if (!small_plan(ctx, M, w->n, w->k, max_parts, p)) return false;
     if (M <= kSmallAlwaysRows) return true;
     if (M > VXM_SMALL_TILE_ROWS && fixup && (int64_t)p.groups * p.mtiles * p.splits > ctx->n_cu) return false;
+    if (M <= VXM_SMALL_TILE_ROWS && !gemm_fits(M, w->n, w->k)) return true;
     GemmPlan t;
     return (M <= VXM_SMALL_TILE_ROWS || w->k <= 16384) && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
 }
@@ -2077,7 +2079,7 @@ bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *
     const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
     if (!mfma || M <= 0 || N % 64) return false;
     SmallPlan sp;
-    if (M <= kSmallGateUpRows && small_plan(ctx, M, N, K, 1, sp)) {
+    if ((M <= kSmallGateUpRows || !gemm_fits(M, N, K)) && small_plan(ctx, M, N, K, 1, sp)) {
         // unsplit: each workgroup holds whole 32-pair blocks over all of K
         launch_small(ctx, w, xq, xd, M, nullptr, sp, sq, sd, variant);
     } else {
@@ -2181,18 +2183,26 @@ static void launch_gemv_f32_c(vxm_ctx *ctx, const vxm_weight *w, const float *x,
                            (int)w->n, (int)M, e);
 }
 
+static int64_t gemv_f32_lds(const vxm_weight *w, int64_t M) { return M * w->k + M * (w->k / VXM_QK) * 2; }
+
+static bool gemv_f32_takes(const vxm_ctx *ctx, const vxm_weight *w, int64_t M) {
+    const int64_t K = w->k;
+    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || gemv_f32_lds(w, M) > kGemvF32MaxLds) return false;
+    const int c = w->dg ? (int)(K / 1024) : 0;
+    const int64_t wg_rows = c == 1 ? 16 : c == 2 ? 8 : 4;   // rows of a workgroup: 4 waves of R
+    return M == 1 || M * K * ((w->n + wg_rows - 1) / wg_rows) <= kGemvF32MaxValues;
+}
+
 bool vxm_launch_gemv_f32(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant,
                          const vxm_gemv_epi &e, int *rc) {
     *rc = VXM_OK;
-    const int64_t K = w->k, lds = M * K + M * (K / VXM_QK) * 2;
-    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || lds > kGemvF32MaxLds) return false;
+    if (!gemv_f32_takes(ctx, w, M)) return false;
+    const int64_t K = w->k, lds = gemv_f32_lds(w, M);
     // an output over the input: workgroups would still read rows that others have written
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)M * K * sizeof(float);
     for (const float *o : {e.y, e.y2, e.y3})
         if (o && (uintptr_t)o < x1 && (uintptr_t)o + (size_t)M * w->n * sizeof(float) > x0) return false;
     const int c = w->dg ? (int)(K / 1024) : 0;
-    const int64_t wg_rows = c == 1 ? 16 : c == 2 ? 8 : 4;   // rows of a workgroup: 4 waves of R
-    if (M > 1 && M * K * ((w->n + wg_rows - 1) / wg_rows) > kGemvF32MaxValues) return false;
     if (c == 1) launch_gemv_f32_c<1, 4>(ctx, w, x, M, variant, (unsigned)lds, e);
     else if (c == 2) launch_gemv_f32_c<2, 2>(ctx, w, x, M, variant, (unsigned)lds, e);
     else if (c == 4) launch_gemv_f32_c<4, 1>(ctx, w, x, M, variant, (unsigned)lds, e);
@@ -2210,13 +2220,24 @@ bool vxm_launch_gemv_f32(vxm_ctx *ctx, const vxm_weight *w, const float *x, int6
     return true;
 }
 
+// The public entries' small-M products: quantized operands, and fp32 rows.
+static bool small_takes(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
+                        SmallPlan &sp) {
+    return use_mfma(ctx, M) && ctx->path != VXM_PATH_MFMA_TILED &&
+           small_wins(ctx, w, xq, xd, M, VXM_MAX_PARTS, true, sp);
+}
+
+static bool small_f32_takes(vxm_ctx *ctx, const vxm_weight *w, int64_t M, SmallPlan &sp) {
+    return M <= kSmallF32MaxRows && small_takes(ctx, w, nullptr, nullptr, M, sp) &&
+           (int64_t)16 * sp.mt * w->k * sp.groups <= kSmallF32MaxValues;
+}
+
 static int launch_mul_mat(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                           float *y, const MmWork *wk) {
     if (M <= 0) return VXM_OK;
     if (use_mfma(ctx, M)) {
         SmallPlan sp;
-        if (ctx->path != VXM_PATH_MFMA_TILED && small_wins(ctx, w, xq, xd, M, VXM_MAX_PARTS, true, sp))
-            return launch_gemm_small(ctx, w, xq, xd, M, y, sp, wk);
+        if (small_takes(ctx, w, xq, xd, M, sp)) return launch_gemm_small(ctx, w, xq, xd, M, y, sp, wk);
         return launch_gemm(ctx, w, xq, xd, M, y, wk);
     }
     launch_gemv(ctx, w, xq, xd, M, y, nullptr);
@@ -2235,7 +2256,7 @@ static int launch_block_dots(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
                              int32_t *out) {
     if (use_mfma(ctx, M)) {
         SmallPlan sp;
-        if (ctx->path != VXM_PATH_MFMA_TILED && small_wins(ctx, w, xq, xd, M, VXM_MAX_PARTS, true, sp)) {
+        if (small_takes(ctx, w, xq, xd, M, sp)) {
             launch_small(ctx, w, xq, xd, M, nullptr, sp, nullptr, nullptr, 0, out);
         } else {
             const int N = (int)w->n, K = (int)w->k;
@@ -2261,6 +2282,42 @@ static int launch_block_dots(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 }
 
 // ---- C ABI -----------------------------------------------------------------
+
+extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t fp32_rows,
+                                     int32_t *kernel, int32_t *splits) {
+    if (!kernel || !splits || n_cu <= 0 || n <= 0 || n > INT32_MAX || k <= 0 || k % VXM_QK || m <= 0 ||
+        path < VXM_PATH_AUTO || path > VXM_PATH_MFMA_TILED)
+        return VXM_ERR_INVALID_ARG;
+    vxm_ctx ctx;
+    ctx.n_cu = n_cu;
+    ctx.path = path;
+    vxm_weight w;   // which scale layouts an upload makes (never read here)
+    w.n = n;
+    w.k = k;
+    w.dg = k % 1024 == 0 ? (uint16_t *)256 : nullptr;
+    w.dt = k % 256 == 0 ? (uint16_t *)256 : nullptr;
+    SmallPlan sp;
+    *splits = 1;
+    if (fp32_rows && gemv_f32_takes(&ctx, &w, m)) {
+        *kernel = VXM_KERNEL_GEMV_F32;
+    } else if (!use_mfma(&ctx, m)) {
+        *kernel = VXM_KERNEL_GEMV;
+    } else if (fp32_rows && small_f32_takes(&ctx, &w, m, sp)) {
+        *kernel = VXM_KERNEL_SMALL_F32;
+        *splits = sp.splits;
+    } else if (small_takes(&ctx, &w, nullptr, nullptr, m, sp)) {
+        *kernel = VXM_KERNEL_SMALL;
+        *splits = sp.splits;
+    } else if (!gemm_fits(m, n, k)) {
+        *kernel = VXM_KERNEL_NONE;
+    } else {
+        GemmPlan p;
+        *kernel = tile_plan(&ctx, &w, nullptr, nullptr, m, SIZE_MAX, p) ? VXM_KERNEL_TILE : VXM_KERNEL_STAGED;
+        if (*kernel == VXM_KERNEL_STAGED) p = gemm_plan(&ctx, m, (int)n, (int)(k / VXM_QK));
+        *splits = p.splits;
+    }
+    return VXM_OK;
+}
 
 extern "C" int vxm_quantize_q8_0(vxm_ctx *ctx, const float *x_dev, int64_t M, int64_t K, int variant,
                                  int8_t *xq_dev, uint16_t *xd_dev) {
@@ -2301,9 +2358,7 @@ extern "C" int vxm_mul_mat_q8_0(vxm_ctx *ctx, const vxm_weight *w, const float *
     SmallPlan sp;
     const bool over = (uintptr_t)y_dev < (uintptr_t)x_dev + (size_t)M * K * 4 &&
                       (uintptr_t)y_dev + (size_t)M * w->n * 4 > (uintptr_t)x_dev;
-    if (M <= kSmallF32MaxRows && use_mfma(ctx, M) && ctx->path != VXM_PATH_MFMA_TILED &&
-        small_wins(ctx, w, nullptr, nullptr, M, VXM_MAX_PARTS, true, sp) &&
-        (int64_t)16 * sp.mt * K * sp.groups <= kSmallF32MaxValues && !(over && sp.splits == 1))
+    if (small_f32_takes(ctx, w, M, sp) && !(over && sp.splits == 1))
         return launch_gemm_small(ctx, w, nullptr, nullptr, M, y_dev, sp, nullptr, x_dev);
     const size_t qbytes = ((size_t)M * K + 255) & ~(size_t)255;
     rc = vxm_ensure_act(ctx, qbytes + (size_t)M * (K / VXM_QK) * 2);

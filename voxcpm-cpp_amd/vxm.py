@@ -85,6 +85,7 @@ _SIGS = {
     "vxm_mul_mat_q8_0_q8_0_multi": (_I, [_P, C.c_int32, _P, _P, _P, _I64, _P]),
     "vxm_stream_read": (_I, [_P, C.c_int32, _P, _P, _P]),
     "vxm_stream_read_sink_words": (_I64, [C.c_int32, _P]),
+    "vxm_host_mul_mat_plan": (_I, [C.c_int32, C.c_int32, _I64, _I64, _I64, C.c_int32, _P, _P]),
     "vxm_block_dots_q8_0": (_I, [_P, _P, _P, _P, _I64, _P]),
     "vxm_rms_norm": (_I, [_P, _P, _P, _I64, _I64, _F, _P, _P, _P]),
     "vxm_minicpm4_create": (_I, [_P, _P, _P, _P, C.POINTER(_P)]),
@@ -650,6 +651,19 @@ def host_quantize_q8_0(x):
     if rc:
         raise VxmError(rc, "vxm_host_quantize_q8_0")
     return out
+
+
+# kernels of vxm_host_mul_mat_plan
+KERNELS = ("none", "gemv", "gemv_f32", "small", "small_f32", "tile", "staged")
+
+
+def host_mul_mat_plan(n, k, m, path=PATH_AUTO, fp32_rows=True, n_cu=256):
+    """(kernel, K splits) that a product of an n x k weight and m rows runs."""
+    kernel, splits = C.c_int32(), C.c_int32()
+    rc = lib().vxm_host_mul_mat_plan(n_cu, path, n, k, m, int(fp32_rows), C.byref(kernel), C.byref(splits))
+    if rc:
+        raise VxmError(rc, "vxm_host_mul_mat_plan")
+    return KERNELS[kernel.value], splits.value
 
 
 def host_sinusoid_embed(t, dim):
