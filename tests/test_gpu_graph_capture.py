@@ -5,10 +5,11 @@ The tiled GEMM's K splits hand partial tiles to the tile's last workgroup as
 tagged words.  The tag is a device word advanced before every split launch, so a
 graph replay reads a tag no earlier launch used.  With a host-side tag, a
 captured launch would replay one fixed tag, and the last workgroup of a tile
-could take a partial word that the previous replay left behind.
+could take a partial word that the previous replay left behind.  The small-M
+GEMM's K splits are slices that a second launch adds.
 
 Each test records vxm_mul_mat_q8_0 and vxm_mul_mat_q8_0_noalloc on a shape whose
-plan splits K (2048 x 6144 from 96 rows: 4 splits), then replays the graph three
+plan splits K (the tiled GEMM 2 and 4 ways, the small-M GEMM 4), then replays the graph three
 times with new activations written into the same device buffer, with eager work
 between the replays.  Every replay must equal an eager call on the same inputs
 bit for bit, and the oracle's fp64 product to the matmul bar.
@@ -33,10 +34,13 @@ def _bar(orc, wq, x, N, K, y):
     assert np.all(err <= ATOL + RTOL * np.abs(ref)), f"max err {err.max()}"
 
 
-@pytest.mark.parametrize("N,K,M", [(2048, 6144, 96), (2048, 2048, 130)])
-def test_captured_split_matmul_replays_match_eager(vxm_ctx, orc, N, K, M):
+@pytest.mark.parametrize("N,K,M,plan", [(2048, 6144, 96, ("small", 4)), (2048, 2048, 130, ("tile", 2)),
+                                        (1024, 4096, 130, ("tile", 4))])
+def test_captured_split_matmul_replays_match_eager(vxm_ctx, orc, N, K, M, plan):
     import torch
+    import vxm
 
+    assert vxm.host_mul_mat_plan(N, K, M) == plan
     print(f"graph capture of split matmuls {N}x{K} M={M}", flush=True)
     wq = _wq(orc, N, K, 7)
     w = vxm_ctx.upload_q8_0(wq, N, K)

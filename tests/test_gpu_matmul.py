@@ -136,14 +136,17 @@ _PRODUCTION_DOTS = [
     (0, 1024, 4096, 5),     # LocEnc down at 5 rows: GEMV <4, 1>
     (0, 256, 1024, 2),      # GEMV <1, 4>
     (0, 7, 96, 2),          # generic GEMV
-    (0, 8192, 1024, 48),    # CFM gate/up at 2 x 24 rows: small-M
-    (0, 3072, 1024, 48),    # CFM QKV: small-M
+    (0, 8192, 1024, 48),    # CFM gate/up at 2 x 24 rows: tile GEMM
+    (0, 3072, 1024, 48),    # CFM QKV: tile GEMM
     (0, 1024, 4096, 48),    # CFM down: small-M, K split
+    (0, 8192, 1024, 16),    # small-M, unsplit
+    (0, 2048, 6144, 97),    # small-M, two row tiles, the last one ragged
     (2, 1024, 4096, 5),     # small-M at 5 rows (the block pipeline's choice)
     (0, 2048, 2048, 512),   # prefill O: tile GEMM, 64 x 64 tiles
     (0, 2560, 1024, 512),   # tile GEMM, 64 x 128 tiles (the prefill QKV choice)
     (0, 8192, 256, 512),    # tile GEMM, 128 x 128 tiles (one full round of 256; long-prompt gate/up, O)
-    (0, 256, 8192, 128),    # tile GEMM, four K splits (more blocks than one activation scale panel holds)
+    (0, 256, 8192, 128),    # small-M, eight K splits
+    (0, 256, 8192, 130),    # tile GEMM, four K splits (more blocks than one activation scale panel holds)
     (0, 1001, 512, 100),    # tile GEMM, ragged M and N (N % 4 != 0: no 16-byte stores)
     (3, 2048, 2048, 33),    # tiled, 16-block stages, K split
     (0, 2560, 2048, 100),   # tile GEMM, ragged M tile
@@ -177,7 +180,7 @@ def test_block_dots_of_the_kernel_that_runs(vxm_ctx, orc, path, N, K, M):
 
 
 @pytest.mark.parametrize("N,K,M", [(2048, 2048, 512), (2560, 1024, 512), (8192, 256, 512), (256, 8192, 128),
-                                   (1001, 512, 100), (8192, 1024, 48)])
+                                   (1001, 512, 100), (8192, 1024, 48), (256, 8192, 130), (8192, 1024, 16)])
 def test_gemm_subnormal_scales(vxm_ctx, orc, N, K, M):
     """Every third weight row and every other activation row are scaled so far down that
     each of their Q8_0 scales is an fp16 subnormal (block maxima near 3e-5, d near 2e-7).
@@ -277,15 +280,23 @@ def test_mfma_gemm_split_k(mfma_path, orc, N, K, M):
     w.free()
 
 
-# Shapes of the register-fed small-M MFMA kernel (M <= 64, N % 64 == 0, K % 512 == 0):
-# the LocDiT projections at M = 2 x 24, a single 64-row group, partial m-tiles, one
-# 16-block stage, several stages per split (long K) and 2 to 8 K splits.  The tiled GEMM (forced) must meet the same bar on the same inputs.
+# Shapes of the register-fed small-M MFMA kernel (N % 64 == 0, K % 256 == 0): the LocDiT
+# projections at one row tile, a single 64-row group, partial m-tiles, one stage, several
+# stages per split (long K) and 1 to 8 K splits; and four that it hands to the tile GEMM
+# (unsplit above 16 rows).  The tiled GEMM (forced) must meet the same bar on the same inputs.
+_SMALL_TO_TILE = [(8192, 1024, 48), (3072, 1024, 48), (1024, 1024, 48), (4096, 1024, 64)]
+
+
 @pytest.mark.parametrize("N,K,M", [(8192, 1024, 48), (3072, 1024, 48), (1024, 1024, 48), (1024, 4096, 48),
                                    (2048, 6144, 48), (64, 512, 5), (64, 32768, 64), (2560, 2048, 16),
-                                   (6144, 2048, 8), (128, 1536, 33), (1024, 512, 1), (4096, 1024, 64)])
+                                   (6144, 2048, 8), (128, 1536, 33), (1024, 512, 1), (4096, 1024, 64),
+                                   (8192, 1024, 16), (12288, 1024, 11), (1024, 1024, 16), (4096, 1536, 64),
+                                   (64, 256, 16), (3072, 2048, 48)])
 def test_mfma_small_m(vxm_ctx, orc, N, K, M):
     import vxm
 
+    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, fp32_rows=False)[0]
+    assert kernel == ("tile" if (N, K, M) in _SMALL_TO_TILE else "small")
     _, x, wq = _case(orc, N, K, M, 19 * N + K + M)
     w = vxm_ctx.upload_q8_0(wq, N, K)
     xq_d, xd_d = vxm_ctx.quantize_q8_0(_dev(x), 1)
@@ -304,10 +315,11 @@ def test_mfma_small_m(vxm_ctx, orc, N, K, M):
 
 
 def test_mfma_small_m_back_to_back_shapes(vxm_ctx, orc):
-    """Consecutive split launches of different shapes share the tagged partial buffer:
-    each must read only its own launch's words."""
+    """Consecutive split launches of different shapes share the slices of the small-M GEMM and
+    the tagged partial buffer of the tile GEMM: each must read only its own launch's."""
     cases = []
-    for (N, K, M) in ((1024, 4096, 48), (1024, 1024, 40), (1024, 4096, 48), (3072, 1024, 24)):
+    for (N, K, M) in ((1024, 4096, 48), (1024, 1024, 40), (1024, 4096, 48), (3072, 1024, 24), (2048, 6144, 96),
+                      (1024, 4096, 200), (1024, 4096, 130)):
         _, x, wq = _case(orc, N, K, M, 7 * N + 3 * K + M)
         w = vxm_ctx.upload_q8_0(wq, N, K)
         xq_d, xd_d = vxm_ctx.quantize_q8_0(_dev(x), 1)

@@ -11,12 +11,17 @@ pytestmark = pytest.mark.gpu
 
 # K = 6144 over 8 splits: three stages per split, three wave groups.  65 to 128 rows: two row
 # tiles (of 48 or 64 rows, the last one ragged), K splits (the tile GEMM would split K there).
+# 64 x 256 at 65 rows and 2560 x 2048 at 77 go to the tile GEMM: the tile's plan is unsplit, and
+# the small-M grid more than one round.
 @pytest.mark.parametrize("N,K,M", [(64, 6144, 1), (64, 6144, 16), (2048, 6144, 17), (2048, 6144, 32), (2048, 6144, 33),
                                    (64, 256, 65), (2048, 2048, 65), (2048, 2048, 96), (2048, 2048, 97),
-                                   (1024, 4096, 127), (512, 2048, 128), (2048, 6144, 128), (2560, 2048, 77)])
+                                   (1024, 4096, 127), (512, 2048, 128), (2048, 6144, 128), (2560, 2048, 77),
+                                   (64, 1536, 65), (192, 4864, 77)])
 def test_small_gemm_row_tiles_and_wave_groups(vxm_ctx, orc, N, K, M):
     import vxm
 
+    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, fp32_rows=False)[0]
+    assert kernel == ("tile" if (N, K, M) in ((64, 256, 65), (2560, 2048, 77)) else "small")
     rng = np.random.default_rng(N + 3 * K + 7 * M)
     x = rng.normal(0, 1, (M, K)).astype(np.float32)
     wq = orc.quantize_rows(rng.normal(0, 0.02, (N, K)).astype(np.float32), orc.QUANT_REF)

@@ -35,23 +35,29 @@ def _check(orc, vxm_ctx, wq, x, N, K, y_na, y_ref):
     assert np.all(err <= ATOL + RTOL * np.abs(ref)), f"max err {err.max()}"
 
 
-# (N, K, M) pairs: the kernel the first call takes, then a smaller input
+# (N, K, M) pairs, then a smaller input, and the kernels that quantized rows of each take
 PAIRS = [
-    # tiled MFMA GEMM with K split 4 ways, then the small-M GEMM with 8 K slices
-    ((2048, 6144, 96), (1024, 4096, 24)),
+    # small-M GEMM with 4 K slices of two row tiles, then with 8 of one
+    ((2048, 6144, 96), (1024, 4096, 24), "small", "small"),
     # small-M GEMM with K slices, then the GEMV
-    ((1024, 4096, 48), (6144, 2048, 1)),
-    # the same tiled product twice, fewer rows the second time (new split tags)
-    ((2048, 2048, 130), (2048, 2048, 70)),
+    ((1024, 4096, 48), (6144, 2048, 1), "small", "gemv"),
+    # tiled MFMA GEMM with K split 2 ways, then the small-M GEMM of the same weight shape
+    ((2048, 2048, 130), (2048, 2048, 70), "tile", "small"),
+    # tiled MFMA GEMM with K split 4 ways, twice, fewer rows the second time (new split tags)
+    ((1024, 4096, 200), (1024, 4096, 130), "tile", "tile"),
+    # ... then the small-M GEMM with 8 K slices
+    ((1024, 4096, 130), (1024, 4096, 24), "tile", "small"),
     # GEMV over two rows, then one
-    ((2048, 6144, 3), (2048, 6144, 1)),
+    ((2048, 6144, 3), (2048, 6144, 1), "gemv", "gemv"),
 ]
 
 
-@pytest.mark.parametrize("first,second", PAIRS)
-def test_noalloc_matches_allocating_entry(vxm_ctx, orc, first, second):
+@pytest.mark.parametrize("first,second,kernel1,kernel2", PAIRS)
+def test_noalloc_matches_allocating_entry(vxm_ctx, orc, first, second, kernel1, kernel2):
     import torch
+    import vxm
 
+    assert [vxm.host_mul_mat_plan(*s, fp32_rows=False)[0] for s in (first, second)] == [kernel1, kernel2]
     print(f"noalloc pair {first} -> {second}", flush=True)
     runs = []
     for i, (N, K, M) in enumerate((first, second)):
@@ -72,12 +78,12 @@ def test_noalloc_matches_allocating_entry(vxm_ctx, orc, first, second):
         w.free()
 
 
-def test_noalloc_repeat_after_allocating_calls(vxm_ctx, orc):
+@pytest.mark.parametrize("N,K,M", [(2048, 6144, 96), (1024, 4096, 130)])
+def test_noalloc_repeat_after_allocating_calls(vxm_ctx, orc, N, K, M):
     """The scratch keeps the last call's contents: a later call with new data and
-    the same shape (same split tags region) still matches."""
+    the same shape (same slices, or same split tags region) still matches."""
     import torch
 
-    N, K, M = 2048, 6144, 96
     for seed in (1, 2):
         x, wq = _case(orc, N, K, M, seed)
         w = vxm_ctx.upload_q8_0(wq, N, K)
