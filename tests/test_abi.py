@@ -105,7 +105,9 @@ def test_mul_mat_plans():
             (6144, 2048, 1, 1, ("gemv_f32", 1)), (6144, 2048, 3, 1, ("gemv_f32", 1)), (6144, 2048, 4, 1, ("gemv", 1)),
             (1024, 1024, 5, 1, ("gemv_f32", 1)), (1024, 1024, 6, 1, ("gemv", 1)),
             (6144, 2048, 16, 1, ("small_f32", 4)), (6144, 2048, 32, 1, ("small", 4)), (12288, 2048, 8, 1, ("small", 2)),
-            (2048, 2048, 32, 1, ("small_f32", 8)), (2048, 2048, 33, 1, ("small", 8))]:
+            (2048, 2048, 32, 1, ("small_f32", 8)), (2048, 2048, 33, 1, ("small", 8)),
+            # two row tiles in three wave groups quantize in a launch of their own
+            (1344, 6144, 16, 1, ("small_f32", 8)), (1344, 6144, 17, 1, ("small", 8)), (64, 768, 20, 1, ("tile", 1))]:
         assert plan(n, k, m, fp32_rows=fp32) == want, (n, k, m, fp32, plan(n, k, m, fp32_rows=fp32))
     for path, want in ((vxm.PATH_GEMV, "gemv"), (vxm.PATH_MFMA, "small"), (vxm.PATH_MFMA_TILED, "tile")):
         assert plan(2048, 2048, 16, path, fp32_rows=False)[0] == want

@@ -1925,8 +1925,9 @@ struct SmallPlan {
     int mt, bps, splits, groups, mtiles, kg;
 };
 
-// Most wave groups whose registers hold a tile of mt 16-row tiles.
-constexpr int small_kg_max(int mt) { return mt <= 2 ? 3 : 2; }
+// Most wave groups whose registers hold a tile of mt 16-row tiles (with xf, the fp32
+// pieces of the next stage beside it: two tiles in three groups spilled 8 bytes a lane).
+constexpr int small_kg_max(int mt, bool xf) { return mt <= (xf ? 1 : 2) ? 3 : 2; }
 
 static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_parts, SmallPlan &p) {
     if (M < 1 || M > VXM_SMALL_MAX_ROWS || N % (16 * kSmallRG) || K % (32 * kSmallStage)) return false;
@@ -1949,7 +1950,7 @@ static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_pa
     // registers of 12 waves hold the tile; four gained nothing over two at K = 2048
     // unsplit (11.5 against 11.9 us at 5 rows, 16.4 against 13.5 at 24).
     p.kg = 1;
-    for (int kg = 2; kg <= small_kg_max(p.mt); kg++)
+    for (int kg = 2; kg <= small_kg_max(p.mt, false); kg++)
         if (per % kg == 0 && stages % kg == 0) p.kg = kg;
     return true;
 }
@@ -1981,7 +1982,8 @@ static bool small_wins(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, cons
     return (M <= VXM_SMALL_TILE_ROWS || w->k <= 16384) && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
 }
 
-// xf != nullptr: fp32 activations, quantized by the kernel with `variant` (p.mt <= 2, no dots).
+// xf != nullptr: fp32 activations, quantized by the kernel with `variant` (p.mt <= 2,
+// p.kg <= small_kg_max(p.mt, true), no dots).
 static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                          float *y, const SmallPlan &p, int8_t *sq = nullptr, uint16_t *sd = nullptr,
                          int variant = 0, int32_t *dots = nullptr, const float *xf = nullptr) {
@@ -1991,7 +1993,7 @@ static void launch_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, co
 #define VXM_SMALL_KG(MT, D, X)                                                                                \
     do {                                                                                                      \
         if (p.kg == 3)                                                                                        \
-            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, small_kg_max(MT), D, X>), grid, block, 0, ctx->stream,  \
+            hipLaunchKernelGGL((k_gemm_q8_0_small<MT, small_kg_max(MT, X), D, X>), grid, block, 0, ctx->stream, \
                                VXM_SMALL_ARGS);                                                               \
         else if (p.kg == 2)                                                                                   \
             hipLaunchKernelGGL((k_gemm_q8_0_small<MT, 2, D, X>), grid, block, 0, ctx->stream, VXM_SMALL_ARGS); \
@@ -2228,7 +2230,7 @@ static bool small_takes(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, con
 }
 
 static bool small_f32_takes(vxm_ctx *ctx, const vxm_weight *w, int64_t M, SmallPlan &sp) {
-    return M <= kSmallF32MaxRows && small_takes(ctx, w, nullptr, nullptr, M, sp) &&
+    return M <= kSmallF32MaxRows && small_takes(ctx, w, nullptr, nullptr, M, sp) && sp.kg <= small_kg_max(sp.mt, true) &&
            (int64_t)16 * sp.mt * w->k * sp.groups <= kSmallF32MaxValues;
 }
 
