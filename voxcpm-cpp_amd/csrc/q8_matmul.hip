@@ -2164,14 +2164,19 @@ static bool use_mfma(const vxm_ctx *ctx, int64_t M) {
            (ctx->path == VXM_PATH_AUTO && M >= kMfmaMinRows);
 }
 
-// The fused GEMV's range: one row, or up to five while the values that all workgroups
-// quantize together (each of them the M rows) cost less than the launch saved.
-// Measured (us a call, fused against two launches): one row 4.0 / 7.3 (6144 x 2048), 4.5 /
-// 7.0 (2048 x 6144), 5.5 / 7.0 (12288 x 2048); 3 rows of 6144 x 2048 (4.7 M values) 6.2 /
-// 7.4, 4 rows (6.3 M) 7.6 / 7.2; 2 rows of 12288 x 2048 (6.3 M) 7.8 / 7.2; 5 rows of 1024 x
-// 1024 7.2 / 7.3, 7 rows 9.2 / 8.2.
-constexpr int kGemvF32MaxRows = 5, kGemvF32MaxLds = 48 * 1024;
-constexpr int64_t kGemvF32MaxValues = 5 << 20;
+// The fused GEMV's range, while quantizing costs less than the launch saved.  A workgroup
+// quantizes M K values one after another (0.15 us per 1024, before its products): at most
+// 12288, whatever the grid (us a call, fused against two launches: 64 x 6144 at 2 rows 5.1 / 6.4,
+// at 3 rows 6.7 / 6.2; 512 x 4096 at 3 rows 5.5 / 6.4, at 4 rows 6.6 / 6.3; one row of 320 x 12288
+// 7.6 / 7.9, of 256 x 16384 9.3 / 9.1, of 512 x 40960 20.5 / 17.6).  All workgroups together: up
+// to 5 M values for one row (20480 x 2048 8.0 / 8.6, 3072 x 6144 4.7 M 5.9 / 6.3; 4096 x 6144 6.3
+// M 6.9 / 6.8, 5120 x 5120 6.6 M 8.1 / 6.5, 4096 x 11008 14.1 / 10.8), 4 M for more (4096 x 2048
+// at 4 rows 6.4 / 6.5, 6144 x 2048 at 2 rows 3.1 M 5.1 / 6.2, at 3 rows 4.7 M 6.4 / 6.3), 2.5 M
+// where a workgroup has 16 weight rows (K = 1024: 8192 at 5 rows 7.5 / 7.9, 12288 at 4 rows 3.1 M
+// 8.1 / 7.7).  And 16 workgroups per CU, past which each adds its start (32768 x 256, 32 per CU,
+// 8.3 / 7.9; 16384 x 256 5.1 / 6.9).
+constexpr int kGemvF32MaxRows = 5, kGemvF32MaxWgValues = 12288, kGemvF32MaxWgsPerCu = 16;
+constexpr int64_t kGemvF32MaxValues1 = 5 << 20, kGemvF32MaxValues = 4 << 20, kGemvF32MaxValuesK1024 = 5 << 19;
 
 template <int C, int R>
 static void launch_gemv_f32_c(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant, unsigned lds,
@@ -2185,21 +2190,21 @@ static void launch_gemv_f32_c(vxm_ctx *ctx, const vxm_weight *w, const float *x,
                            (int)w->n, (int)M, e);
 }
 
-static int64_t gemv_f32_lds(const vxm_weight *w, int64_t M) { return M * w->k + M * (w->k / VXM_QK) * 2; }
-
 static bool gemv_f32_takes(const vxm_ctx *ctx, const vxm_weight *w, int64_t M) {
     const int64_t K = w->k;
-    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || gemv_f32_lds(w, M) > kGemvF32MaxLds) return false;
+    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || M * K > kGemvF32MaxWgValues) return false;
     const int c = w->dg ? (int)(K / 1024) : 0;
     const int64_t wg_rows = c == 1 ? 16 : c == 2 ? 8 : 4;   // rows of a workgroup: 4 waves of R
-    return M == 1 || M * K * ((w->n + wg_rows - 1) / wg_rows) <= kGemvF32MaxValues;
+    const int64_t wgs = (w->n + wg_rows - 1) / wg_rows;
+    return wgs <= (int64_t)kGemvF32MaxWgsPerCu * ctx->n_cu &&
+           M * K * wgs <= (M == 1 ? kGemvF32MaxValues1 : c == 1 ? kGemvF32MaxValuesK1024 : kGemvF32MaxValues);
 }
 
 bool vxm_launch_gemv_f32(vxm_ctx *ctx, const vxm_weight *w, const float *x, int64_t M, int variant,
                          const vxm_gemv_epi &e, int *rc) {
     *rc = VXM_OK;
     if (!gemv_f32_takes(ctx, w, M)) return false;
-    const int64_t K = w->k, lds = gemv_f32_lds(w, M);
+    const int64_t K = w->k, lds = M * K + M * (K / VXM_QK) * 2;
     // an output over the input: workgroups would still read rows that others have written
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)M * K * sizeof(float);
     for (const float *o : {e.y, e.y2, e.y3})
