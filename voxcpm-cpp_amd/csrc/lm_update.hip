@@ -18,9 +18,11 @@
 
 #include "vxm_model.h"
 
-// Patches whose in_proj k_locenc_assemble forms itself: its row of x in LDS, and few
-// rows, since every row's workgroup reads the whole weight.
-constexpr int kLocEncFuseFeat = 256, kLocEncFuseRows = 64;
+// Patches whose in_proj k_locenc_assemble forms itself: its row of x in LDS, few rows and a
+// small weight, since every row's workgroup reads all of it.  Encoder without blocks, 4 and 64
+// rows, against launches of their own: 1024 x 64 6.4 / 11.0 and 6.4 / 12.8 us, 2048 x 64 8.5 /
+// 11.3, 1024 x 128 8.9 / 11.0; with 256 K values 1024 x 256 13.0 / 10.9, 2048 x 128 13.7 / 11.6.
+constexpr int kLocEncFuseFeat = 256, kLocEncFuseRows = 64, kLocEncFuseValues = 128 * 1024;
 
 struct vxm_locenc {
     vxm_ctx *ctx = nullptr;
@@ -308,7 +310,8 @@ extern "C" int vxm_locenc_forward(vxm_locenc *m, const float *x_dev, int32_t P, 
     if ((rc = vxm_ws_ensure(ctx, m->ws, S, H, qd, kvd, d.F, (int64_t)d.nkv * S * d.hd))) return rc;
     if ((rc = vxm_rope_ensure(ctx, m->dims, S))) return rc;
     if ((rc = locenc_bufs(m, S, P))) return rc;
-    const bool fuse_in = m->cfg.feat_dim <= kLocEncFuseFeat && P <= kLocEncFuseRows && ctx->path == VXM_PATH_AUTO;
+    const bool fuse_in = m->cfg.feat_dim <= kLocEncFuseFeat && P <= kLocEncFuseRows &&
+                         H * m->cfg.feat_dim <= kLocEncFuseValues && ctx->path == VXM_PATH_AUTO;
     if (!fuse_in) {
         if ((rc = vxm_launch_quantize(ctx, x_dev, P, m->cfg.feat_dim, var, m->aq, m->ad))) return rc;
         if ((rc = vxm_launch_mul_mat(ctx, m->in_proj, m->aq, m->ad, P, m->xh))) return rc;
