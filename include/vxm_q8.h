@@ -55,8 +55,8 @@ typedef enum vxm_status {
 #define VXM_PATH_AUTO 0
 #define VXM_PATH_GEMV 1   /* weight-streaming GEMV, any M (loops over rows of x) */
 #define VXM_PATH_MFMA 2   /* int8 MFMA: register-fed small-M kernel up to 16 rows, and up to
-                           * 128 where the tiled GEMM would split K (N % 64 == 0,
-                           * K % 256 == 0), else the LDS-tiled GEMM */
+                           * 128 where it is the faster one (N % 64 == 0, K % 256 == 0),
+                           * else the LDS-tiled GEMM */
 #define VXM_PATH_MFMA_TILED 3 /* the LDS-tiled MFMA GEMM for every M            */
 
 typedef struct vxm_ctx vxm_ctx;
@@ -165,9 +165,13 @@ int64_t vxm_stream_read_sink_words(int32_t n, const int64_t *bytes);
 int vxm_mul_mat_q8_0_noalloc(vxm_ctx *ctx, const vxm_weight *w, const float *x_dev, int64_t M,
                              float *y_dev);
 size_t vxm_noalloc_scratch_bytes(void);
-/* Test hook, host only: the kernel that vxm_mul_mat_q8_0 (fp32_rows != 0) or
- * vxm_mul_mat_q8_0_q8_0 runs for an n x k weight and m rows in 16-byte aligned buffers
- * apart from each other, on a device of n_cu CUs, and its K splits. */
+/* Test hook, host only: the kernel that a product of an n x k weight and m rows in
+ * 16-byte aligned buffers apart from each other runs on a device of n_cu CUs, and its
+ * K splits: vxm_mul_mat_q8_0_q8_0's, vxm_mul_mat_q8_0's, or a model block's, whose
+ * next kernel adds the small-M GEMM's slices. */
+#define VXM_ROWS_Q8 0
+#define VXM_ROWS_F32 1
+#define VXM_ROWS_BLOCK 2
 #define VXM_KERNEL_NONE 0      /* refused: operands of 2 GiB and more */
 #define VXM_KERNEL_GEMV 1      /* weight-streaming GEMV */
 #define VXM_KERNEL_GEMV_F32 2  /* ... that quantizes its rows itself */
@@ -175,7 +179,7 @@ size_t vxm_noalloc_scratch_bytes(void);
 #define VXM_KERNEL_SMALL_F32 4 /* ... that quantizes its rows itself */
 #define VXM_KERNEL_TILE 5      /* DMA-fed tile GEMM */
 #define VXM_KERNEL_STAGED 6    /* register-staged tile GEMM (k % 256 != 0) */
-int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t fp32_rows,
+int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t rows,
                           int32_t *kernel, int32_t *splits);
 /* Debug: int32 per-block sums of vec_dot_q8_0_q8_0, out[(m*N + n)*(K/32) + b]. */
 int vxm_block_dots_q8_0(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq_dev,

@@ -94,7 +94,7 @@ def test_mul_mat_plans():
     import vxm
 
     plan = vxm.host_mul_mat_plan
-    for n, k, m, fp32, want in [
+    for n, k, m, rows, want in [
             (6144, 2048, 7, 0, ("gemv", 1)), (6144, 2048, 8, 0, ("small", 4)), (12288, 2048, 16, 0, ("small", 2)),
             # above one row tile: the tile GEMM where it needs no K split
             (12288, 2048, 17, 0, ("tile", 1)), (2048, 2048, 17, 0, ("small", 8)), (2048, 2048, 64, 0, ("small", 8)),
@@ -111,11 +111,24 @@ def test_mul_mat_plans():
             (32000, 4096, 1, 1, ("gemv", 1)), (4096, 11008, 1, 1, ("gemv", 1)), (73448, 2048, 1, 1, ("gemv", 1)),
             (6144, 2048, 16, 1, ("small_f32", 4)), (6144, 2048, 32, 1, ("small", 4)), (12288, 2048, 8, 1, ("small", 2)),
             (2048, 2048, 32, 1, ("small_f32", 8)), (2048, 2048, 33, 1, ("small", 8)),
+            # whose stages are not too many in a row
+            (512, 5632, 16, 1, ("small_f32", 8)), (512, 11008, 16, 1, ("small", 8)), (1024, 8192, 17, 1, ("small", 8)),
+            # short K unsplit by the tile GEMM: while the launches cost less than its stages
+            (2048, 256, 24, 0, ("small", 1)), (2048, 256, 49, 0, ("tile", 1)), (2048, 512, 24, 0, ("tile", 1)),
+            (1024, 1024, 48, 0, ("small", 4)), (1024, 1024, 49, 0, ("tile", 1)),
+            # two row tiles, by the stages in a row
+            (2048, 4096, 128, 0, ("small", 4)), (2048, 5120, 77, 0, ("small", 4)), (2048, 5120, 100, 0, ("tile", 4)),
+            (2048, 11008, 77, 0, ("tile", 4)),
+            # a block's products, whose slices the next kernel adds
+            (3072, 1024, 48, 2, ("small", 4)), (8192, 1024, 24, 2, ("small", 2)), (8192, 768, 48, 2, ("small", 2)),
+            (8192, 768, 49, 2, ("tile", 1)), (12288, 2048, 24, 2, ("tile", 1)), (2048, 6144, 77, 2, ("small", 4)),
+            (2560, 2048, 128, 2, ("small", 4)), (2560, 4096, 96, 2, ("small", 4)), (2560, 4096, 97, 2, ("tile", 3)),
+            (2048, 11008, 77, 2, ("tile", 4)), (4096, 11008, 128, 2, ("tile", 2)),
             # two row tiles in three wave groups quantize in a launch of their own
             (1344, 6144, 16, 1, ("small_f32", 8)), (1344, 6144, 17, 1, ("small", 8)), (64, 768, 20, 1, ("tile", 1))]:
-        assert plan(n, k, m, fp32_rows=fp32) == want, (n, k, m, fp32, plan(n, k, m, fp32_rows=fp32))
+        assert plan(n, k, m, rows=rows) == want, (n, k, m, rows, plan(n, k, m, rows=rows))
     for path, want in ((vxm.PATH_GEMV, "gemv"), (vxm.PATH_MFMA, "small"), (vxm.PATH_MFMA_TILED, "tile")):
-        assert plan(2048, 2048, 16, path, fp32_rows=False)[0] == want
+        assert plan(2048, 2048, 16, path, rows=vxm.ROWS_Q8)[0] == want
 
 
 def test_mul_mat_plan_takes_operands_up_to_2_gib():

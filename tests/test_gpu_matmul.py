@@ -137,7 +137,7 @@ _PRODUCTION_DOTS = [
     (0, 256, 1024, 2),      # GEMV <1, 4>
     (0, 7, 96, 2),          # generic GEMV
     (0, 8192, 1024, 48),    # CFM gate/up at 2 x 24 rows: tile GEMM
-    (0, 3072, 1024, 48),    # CFM QKV: tile GEMM
+    (0, 3072, 1024, 48),    # CFM QKV: small-M, K split
     (0, 1024, 4096, 48),    # CFM down: small-M, K split
     (0, 8192, 1024, 16),    # small-M, unsplit
     (0, 2048, 6144, 97),    # small-M, two row tiles, the last one ragged
@@ -282,9 +282,9 @@ def test_mfma_gemm_split_k(mfma_path, orc, N, K, M):
 
 # Shapes of the register-fed small-M MFMA kernel (N % 64 == 0, K % 256 == 0): the LocDiT
 # projections at one row tile, a single 64-row group, partial m-tiles, one stage, several
-# stages per split (long K) and 1 to 8 K splits; and four that it hands to the tile GEMM
-# (unsplit above 16 rows).  The tiled GEMM (forced) must meet the same bar on the same inputs.
-_SMALL_TO_TILE = [(8192, 1024, 48), (3072, 1024, 48), (1024, 1024, 48), (4096, 1024, 64)]
+# stages per split (long K) and 1 to 8 K splits; and two that it hands to the tile GEMM
+# (unsplit, above 48 rows or with too many values for the fix-up).  The tiled GEMM (forced) must meet the same bar on the same inputs.
+_SMALL_TO_TILE = [(8192, 1024, 48), (4096, 1024, 64)]
 
 
 @pytest.mark.parametrize("N,K,M", [(8192, 1024, 48), (3072, 1024, 48), (1024, 1024, 48), (1024, 4096, 48),
@@ -295,7 +295,7 @@ _SMALL_TO_TILE = [(8192, 1024, 48), (3072, 1024, 48), (1024, 1024, 48), (4096, 1
 def test_mfma_small_m(vxm_ctx, orc, N, K, M):
     import vxm
 
-    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, fp32_rows=False)[0]
+    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, rows=vxm.ROWS_Q8)[0]
     assert kernel == ("tile" if (N, K, M) in _SMALL_TO_TILE else "small")
     _, x, wq = _case(orc, N, K, M, 19 * N + K + M)
     w = vxm_ctx.upload_q8_0(wq, N, K)

@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 def test_small_gemm_row_tiles_and_wave_groups(vxm_ctx, orc, N, K, M):
     import vxm
 
-    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, fp32_rows=False)[0]
+    kernel = vxm.host_mul_mat_plan(N, K, M, vxm.PATH_MFMA, rows=vxm.ROWS_Q8)[0]
     assert kernel == ("tile" if (N, K, M) in ((64, 256, 65), (2560, 2048, 77)) else "small")
     rng = np.random.default_rng(N + 3 * K + 7 * M)
     x = rng.normal(0, 1, (M, K)).astype(np.float32)

@@ -57,7 +57,7 @@ def test_noalloc_matches_allocating_entry(vxm_ctx, orc, first, second, kernel1, 
     import torch
     import vxm
 
-    assert [vxm.host_mul_mat_plan(*s, fp32_rows=False)[0] for s in (first, second)] == [kernel1, kernel2]
+    assert [vxm.host_mul_mat_plan(*s, rows=vxm.ROWS_Q8)[0] for s in (first, second)] == [kernel1, kernel2]
     print(f"noalloc pair {first} -> {second}", flush=True)
     runs = []
     for i, (N, K, M) in enumerate((first, second)):

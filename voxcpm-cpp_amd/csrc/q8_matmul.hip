@@ -1908,8 +1908,10 @@ static int launch_gemm(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, cons
 // workgroups quantize together (padding rows included) costs less than the launch saved.
 // Measured (us a call, 8 rows unless said, against three launches): 2048 x 2048 7.3 / 10.2,
 // 2048 x 6144 (3.1 M values) 9.2 / 11.4, 6144 x 2048 (3.1 M) 8.8 / 12.0, 1024 x 4096 at 32 rows (2.1 M)
-// 10.4 / 11.0; 12288 x 2048 (6.3 M) 12.6 / 12.1, 6144 x 2048 at 24 rows (6.3 M) 14.8 / 12.9.
-constexpr int kSmallF32MaxRows = 32;
+// 10.4 / 11.0; 12288 x 2048 (6.3 M) 12.6 / 12.1, 6144 x 2048 at 24 rows (6.3 M) 14.8 / 12.9.  The
+// conversion also lengthens each stage of a wave group's chain: up to three stages in one
+// row tile (512 x 11008 with six 15.9 / 14.5), one in two (1024 x 8192 with two at 24 rows 14.3 / 12.9).
+constexpr int kSmallF32MaxRows = 32, kSmallF32MaxChain = 3;
 constexpr int64_t kSmallF32MaxValues = 4 << 20;
 // Rows of activations from which the MFMA GEMM replaces the weight-streaming
 // GEMV (which re-reads each activation row per weight row group).
@@ -1923,6 +1925,8 @@ constexpr int kSmallPartsMinRows = 2;
 // K % 256, M > 128, operands of 2 GiB) take the tiled GEMM.
 struct SmallPlan {
     int mt, bps, splits, groups, mtiles, kg;
+    int chain() const { return bps / kSmallStage / kg; }   // stages in a row of one wave group
+    int64_t wgs() const { return (int64_t)groups * mtiles * splits; }
 };
 
 // Most wave groups whose registers hold a tile of mt 16-row tiles (with xf, the fp32
@@ -1959,27 +1963,43 @@ static bool small_plan(vxm_ctx *ctx, int64_t M, int64_t N, int64_t K, int max_pa
 // where it is level with the tile GEMM at worst (12288 x 2048, 16 rows: 13.1 / 12.9 us).
 constexpr int kSmallAlwaysRows = 16;
 
-// The small-M kernel's plan for the product, where it is the one to run: any M it
-// takes up to kSmallAlwaysRows; above that (each row tile of its waves repeats the
-// scaling work, and past 64 rows the read of the weights) where the tile GEMM would
-// split K, whose tag launch, partial words and last-workgroup fix-up cost more (M = 77,
-// public entry: 2048 x 2048 15.6 -> 11.5 us, 2048 x 6144 19.7 -> 16.9, 1024 x 4096 17.0 ->
-// 13.1 at M = 100).  12288 x 2048, which the tile GEMM takes unsplit, goes there: 24.3 ->
-// 13.0 us at M = 64, 17.4 -> 12.9 at 24, 28.2 / 19.0 at 77.  Past 64 rows and with a fix-up
-// launch of its own (the public entries) only where its grid is one round: 2560 x 2048,
-// 320 workgroups, 16.6 against 15.7 us at M = 100.  With three row tiles (M > 128) it
-// loses: 2048 x 6144 30.1 against 23.4 us at M = 150.  K is bounded there so that the
-// slices and the quantized rows of any such product fit the allocation-free entry's
-// scratch together.  Up to 64 rows it also takes what it can address and the tile GEMM
-// cannot (N K just below 2^31).
+// The small-M kernel's plan for the product, where it is the one to run: any M it takes up to
+// kSmallAlwaysRows, and above that against the tile GEMM's plan, whose time grows by a stage of
+// K after another (0.95 us each, unsplit) and by about 5 us for a K split's tag launch, partial
+// words and last-workgroup fix-up.  fixup: the slices are added by a launch of its own (the
+// public entries; 1.9 us), else by the consumer.  Device us, small-M / tile:
+// - up to 64 rows, where the tile GEMM splits K: always.  Where it does not and the consumer
+//   adds: while the grid is one round (one workgroup of two wave groups per CU, or two of one:
+//   3072 x 1024 at 48 rows 4.5 / 7.4, 8192 x 1024 at 17 4.8 / 7.4; two rounds: 12288 x 2048 at
+//   24 13.0 / 10.8), above 32 rows of a full device with few stages in a row of one wave group
+//   (8192 x 768, two, at 48 6.1 / 6.8; 16384 x 2048, four, 13.9 / 11.1; 12288 x 1280, three, at 64
+//   10.4 / 8.5).  With a fix-up up to 48 rows of K = 256, which has none (2048 x 256 at 24, with
+//   the quantization, 5.4 / 6.3), and of K = 1024 (1024 x 1024 at 24 7.7 / 9.1; from 49 rows the
+//   launch saved is worth more to the host, and K = 512 is level).  It also takes what it can
+//   address and the tile GEMM cannot (N K just below 2^31).
+// - 65 to 128 rows (two row tiles, each reading the weights), where the tile GEMM splits K, by
+//   the stages in a row.  Consumer adds: six in one round (2048 x 6144 at 77 rows, three, 9.9 /
+//   17.4; 4096 x 6144, six, at 128 24.3 / 24.2; 2048 x 11008, eleven, at 77 24.7 / 21.2), in two
+//   rounds two of 48-row tiles, one of 64-row ones (2560 x 2048, one, at 77 8.9 / 13.5; 2560 x
+//   4096, two, at 77 14.4 / 15.7, at 100 17.0 / 16.2).  With a fix-up at most one workgroup per CU
+//   and five stages, four of 64-row tiles (2048 x 5120 at 100, five, 20.6 / 19.6).  With three row
+//   tiles (M > 128) it loses: 2048 x 6144 30.1 / 23.4 at M = 150.
 static bool small_wins(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                        int max_parts, bool fixup, SmallPlan &p) {
     if (!small_plan(ctx, M, w->n, w->k, max_parts, p)) return false;
     if (M <= kSmallAlwaysRows) return true;
-    if (M > VXM_SMALL_TILE_ROWS && fixup && (int64_t)p.groups * p.mtiles * p.splits > ctx->n_cu) return false;
-    if (M <= VXM_SMALL_TILE_ROWS && !gemm_fits(M, w->n, w->k)) return true;
+    const bool one_round = p.wgs() <= (p.kg == 1 ? 2 : 1) * ctx->n_cu;
     GemmPlan t;
-    return (M <= VXM_SMALL_TILE_ROWS || w->k <= 16384) && (!tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) || t.splits > 1);
+    const bool unsplit = tile_plan(ctx, w, xq, xd, M, SIZE_MAX, t) && t.splits == 1;
+    if (M <= VXM_SMALL_TILE_ROWS) {
+        if (!unsplit || !gemm_fits(M, w->n, w->k)) return true;
+        if (!one_round) return false;
+        if (fixup) return M <= 48 && p.chain() == 1 && (p.splits == 1 || p.splits >= 4);
+        return M <= 32 || p.chain() <= (M <= 48 ? 3 : 1) || p.wgs() < ctx->n_cu;
+    }
+    if (unsplit) return false;
+    if (fixup) return p.wgs() <= ctx->n_cu && p.chain() <= (p.mt == 4 ? 4 : 5);
+    return p.chain() <= (one_round ? 6 : p.mt == 3 ? 2 : 1);
 }
 
 // xf != nullptr: fp32 activations, quantized by the kernel with `variant` (p.mt <= 2,
@@ -2050,14 +2070,18 @@ static int launch_gemm_small(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
     return VXM_OK;
 }
 
+static bool parts_takes(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
+                        int max_parts, SmallPlan &sp) {
+    return (ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows)) &&
+           small_wins(ctx, w, xq, xd, M, max_parts < VXM_MAX_PARTS ? max_parts : VXM_MAX_PARTS, false, sp);
+}
+
 int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                              float *y, int max_parts, int *parts) {
     *parts = 1;
     if (M <= 0) return VXM_OK;
     SmallPlan sp;
-    const bool small = (ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows)) &&
-                       small_wins(ctx, w, xq, xd, M, max_parts < VXM_MAX_PARTS ? max_parts : VXM_MAX_PARTS, false, sp);
-    if (!small) return vxm_launch_mul_mat(ctx, w, xq, xd, M, y);
+    if (!parts_takes(ctx, w, xq, xd, M, max_parts, sp)) return vxm_launch_mul_mat(ctx, w, xq, xd, M, y);
     launch_small(ctx, w, xq, xd, M, y, sp);
     VXM_CHECK_LAUNCH(ctx);
     *parts = sp.splits;
@@ -2067,12 +2091,12 @@ int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 // The gate/up projection with SwiGLU and the Q8_0 of its output fused into the
 // GEMM's epilogue (rows of w interleave gate n = row 2n and up n = row 2n+1): sq
 // [M][N/2] and sd [M][N/64] are the down projection's input.  The small-M kernel
-// takes M <= 32, the tile GEMM larger M when its plan needs no K split.  Returns
+// takes M <= 32 (48 where K < 768), the tile GEMM larger M when its plan needs no K split.  Returns
 // false without launching otherwise (and under PATH_MFMA_TILED, which keeps the
 // unfused GEMM + k_swiglu_quant as the reference of the fused epilogue).
-// (up to two of the small-M kernel's row tiles it is level with the tile GEMM; one layer at
-// 64 rows 64.7 -> 58.7 us on the tile GEMM, at 33 rows 54.5)
-constexpr int kSmallGateUpRows = 32;
+// (us, small-M / tile: 12288 x 2048 at 24 rows 11.4 / 11.4, at 33 rows 14.4 / 11.5; 8192 x 1024 at
+// 48 rows 9.1 / 8.4, 4096 x 768 8.4 / 7.6, 4096 x 512 6.0 / 6.4)
+constexpr int kSmallGateUpRows = 32, kSmallGateUpRowsShortK = 48, kSmallGateUpShortK = 768;
 
 bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                                int8_t *sq, uint16_t *sd, int variant, int *rc) {
@@ -2081,7 +2105,8 @@ bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *
     const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
     if (!mfma || M <= 0 || N % 64) return false;
     SmallPlan sp;
-    if ((M <= kSmallGateUpRows || !gemm_fits(M, N, K)) && small_plan(ctx, M, N, K, 1, sp)) {
+    const int small_rows = K < kSmallGateUpShortK ? kSmallGateUpRowsShortK : kSmallGateUpRows;
+    if ((M <= small_rows || !gemm_fits(M, N, K)) && small_plan(ctx, M, N, K, 1, sp)) {
         // unsplit: each workgroup holds whole 32-pair blocks over all of K
         launch_small(ctx, w, xq, xd, M, nullptr, sp, sq, sd, variant);
     } else {
@@ -2095,9 +2120,9 @@ bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *
     return true;
 }
 
-// The QKV projection with k_rope_kv's work in the tile GEMM's epilogue (qe):
-// taken where vxm_launch_mul_mat_parts would run the tile GEMM without a K
-// split (M > 64 and a plan of one split), so the products are the same.
+// The QKV projection with k_rope_kv's work in the tile GEMM's epilogue (qe): taken
+// above 64 rows where vxm_launch_mul_mat_parts would run the tile GEMM without a K
+// split, so the products are the same (up to 64 rows that GEMM writes its products).
 // Returns false without launching otherwise, and under PATH_MFMA_TILED (which
 // keeps the GEMM + k_rope_kv pair as the reference of the fused epilogue).
 static bool use_mfma(const vxm_ctx *ctx, int64_t M);
@@ -2235,7 +2260,8 @@ static bool small_takes(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, con
 }
 
 static bool small_f32_takes(vxm_ctx *ctx, const vxm_weight *w, int64_t M, SmallPlan &sp) {
-    return M <= kSmallF32MaxRows && small_takes(ctx, w, nullptr, nullptr, M, sp) && sp.kg <= small_kg_max(sp.mt, true) &&
+    return M <= kSmallF32MaxRows && small_takes(ctx, w, nullptr, nullptr, M, sp) &&
+           sp.kg <= small_kg_max(sp.mt, true) && sp.chain() <= (sp.mt == 1 ? kSmallF32MaxChain : 1) &&
            (int64_t)16 * sp.mt * w->k * sp.groups <= kSmallF32MaxValues;
 }
 
@@ -2290,10 +2316,10 @@ static int launch_block_dots(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 
 // ---- C ABI -----------------------------------------------------------------
 
-extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t fp32_rows,
+extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t rows,
                                      int32_t *kernel, int32_t *splits) {
     if (!kernel || !splits || n_cu <= 0 || n <= 0 || n > INT32_MAX || k <= 0 || k % VXM_QK || m <= 0 ||
-        path < VXM_PATH_AUTO || path > VXM_PATH_MFMA_TILED)
+        path < VXM_PATH_AUTO || path > VXM_PATH_MFMA_TILED || rows < VXM_ROWS_Q8 || rows > VXM_ROWS_BLOCK)
         return VXM_ERR_INVALID_ARG;
     vxm_ctx ctx;
     ctx.n_cu = n_cu;
@@ -2305,11 +2331,14 @@ extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int6
     w.dt = k % 256 == 0 ? (uint16_t *)256 : nullptr;
     SmallPlan sp;
     *splits = 1;
-    if (fp32_rows && gemv_f32_takes(&ctx, &w, m)) {
+    if (rows == VXM_ROWS_F32 && gemv_f32_takes(&ctx, &w, m)) {
         *kernel = VXM_KERNEL_GEMV_F32;
+    } else if (rows == VXM_ROWS_BLOCK && parts_takes(&ctx, &w, nullptr, nullptr, m, VXM_MAX_PARTS, sp)) {
+        *kernel = VXM_KERNEL_SMALL;
+        *splits = sp.splits;
     } else if (!use_mfma(&ctx, m)) {
         *kernel = VXM_KERNEL_GEMV;
-    } else if (fp32_rows && small_f32_takes(&ctx, &w, m, sp)) {
+    } else if (rows == VXM_ROWS_F32 && small_f32_takes(&ctx, &w, m, sp)) {
         *kernel = VXM_KERNEL_SMALL_F32;
         *splits = sp.splits;
     } else if (small_takes(&ctx, &w, nullptr, nullptr, m, sp)) {

@@ -657,10 +657,13 @@ def host_quantize_q8_0(x):
 KERNELS = ("none", "gemv", "gemv_f32", "small", "small_f32", "tile", "staged")
 
 
-def host_mul_mat_plan(n, k, m, path=PATH_AUTO, fp32_rows=True, n_cu=256):
+ROWS_Q8, ROWS_F32, ROWS_BLOCK = 0, 1, 2
+
+
+def host_mul_mat_plan(n, k, m, path=PATH_AUTO, rows=ROWS_F32, n_cu=256):
     """(kernel, K splits) that a product of an n x k weight and m rows runs."""
     kernel, splits = C.c_int32(), C.c_int32()
-    rc = lib().vxm_host_mul_mat_plan(n_cu, path, n, k, m, int(fp32_rows), C.byref(kernel), C.byref(splits))
+    rc = lib().vxm_host_mul_mat_plan(n_cu, path, n, k, m, rows, C.byref(kernel), C.byref(splits))
     if rc:
         raise VxmError(rc, "vxm_host_mul_mat_plan")
     return KERNELS[kernel.value], splits.value
