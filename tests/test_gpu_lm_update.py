@@ -208,6 +208,27 @@ def test_lm_update_small_three_steps(vxm_ctx, orc, with_fsq):
         o.free()
 
 
+@pytest.mark.parametrize("path", ["PATH_GEMV", "PATH_MFMA", "PATH_MFMA_TILED"])
+def test_lm_update_forced_matmul_path(vxm_ctx, orc, path):
+    """The chain's projections with their quantization, bias, FSQ and copies in launches of their
+    own (a forced MFMA path), and in one (the GEMV)."""
+    import vxm
+
+    enc, tsl, ral, pw, u = _build_update(vxm, vxm_ctx, orc, 92, True, SMALL)
+
+    def stack_bar(y, ref, what):
+        assert_layer_close(y, ref, what=f"{path} {what}")
+
+    try:
+        vxm_ctx.set_path(getattr(vxm, path))
+        _check_update(orc, vxm_ctx, enc, tsl, ral, pw, u, 2, 93, stack_bar)
+    finally:
+        vxm_ctx.set_path(vxm.PATH_AUTO)
+    u.free()
+    for o in (enc[0], tsl[0], ral[0], tsl[1], ral[1]):
+        o.free()
+
+
 def test_lm_update_full_width_persistent(vxm_ctx, orc):
     """TSLM and RALM at the decode shape (hidden 2048, 16 / 2 heads x 128, FFN 6144; 2 layers each, the
     RALM without rope) run on the single-launch decode kernel inside the update; LocEnc at full width
@@ -307,4 +328,11 @@ def test_embed_rows_q8_0_bit_exact(vxm_ctx, orc):
     ids = np.array([5, 999, 0, -3, 1000, 123, 123, 77] + list(rng.integers(0, rows, 56)), np.int32)
     out = _np(vxm_ctx.embed_rows_q8_0(w, torch.from_numpy(ids).to("cuda:0")))
     assert np.array_equal(out, orc.embed_rows_q8_0(table, rows, k, ids))
+    # an output that is not 16-byte aligned
+    buf = torch.full((ids.size * k + 2,), float("nan"), dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
+    vxm_ctx.embed_rows_q8_0(w, torch.from_numpy(ids).to("cuda:0"), buf[1:-1].view(ids.size, k))
+    vxm_ctx.sync()
+    got = _np(buf)
+    assert np.isnan(got[[0, -1]]).all() and np.array_equal(got[1:-1].reshape(out.shape), out)
     w.free()

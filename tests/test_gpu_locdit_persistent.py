@@ -113,6 +113,38 @@ def test_persistent_locenc_one_block(vxm_ctx, orc, special):
     enc.free()
 
 
+@pytest.mark.parametrize("nkv,hd", [(2, 128), (16, 64)])
+@pytest.mark.parametrize("special", [True, False])
+@pytest.mark.parametrize("P", [1, 15, 16, 17])
+def test_persistent_locenc_final_norm(vxm_ctx, orc, nkv, hd, special, P):
+    """Up to 16 rows the single launch writes the returned rows' final norm itself; an output that
+    is not 8-byte aligned, and more rows, take a launch of their own for it: the same bits, and
+    the oracle's block."""
+    import torch
+    import vxm
+    from test_gpu_locdit import assert_sensitivity_close
+    from test_lm_update_host import make_locenc
+
+    cfg, w, ow, ocfg = make_locenc(orc, 160 + P, H=1024, L=1, nh=16, nkv=nkv, hd=hd, F=4096, special=special)
+    enc = vxm.LocEnc(vxm_ctx, cfg, w)
+    enc.set_block_mode(vxm.DECODE_PERSISTENT)
+    x = np.random.default_rng(170 + P).normal(0, 1, (P, 64)).astype(np.float32)
+    n = 1024 if special else 1024 * P
+    outs = []
+    for off in (0, 1):
+        buf = torch.full((n + 2,), float("nan"), dtype=torch.float32, device="cuda:0")
+        torch.cuda.synchronize()
+        enc.forward(_dev(x), buf[off:off + n])
+        enc.check()
+        got = buf.cpu().numpy()
+        assert np.isnan(got[:off]).all() and np.isnan(got[off + n:]).all()
+        outs.append(got[off:off + n])
+    assert np.array_equal(outs[0], outs[1])
+    assert_sensitivity_close(outs[0].reshape(-1, 1024), orc.locenc_forward(ocfg, ow, x).reshape(-1, 1024),
+                             what=f"persistent locenc {nkv}x{hd} P={P} special={special}")
+    enc.free()
+
+
 def test_persistent_locenc_full_size(vxm_ctx, orc):
     """The 12-block encoder (5 rows): within the deep-stack bar of the oracle, and no farther
     from the launch-based path than that path is from the oracle (plus the same bar)."""
