@@ -105,8 +105,8 @@ def test_mul_mat_plans():
             (6144, 2048, 1, 1, ("gemv_f32", 1)), (6144, 2048, 2, 1, ("gemv_f32", 1)), (6144, 2048, 3, 1, ("gemv", 1)),
             (1024, 1024, 5, 1, ("gemv_f32", 1)), (1024, 1024, 6, 1, ("gemv", 1)),
             (8192, 1024, 5, 1, ("gemv_f32", 1)), (12288, 1024, 4, 1, ("gemv", 1)),
-            (5, 6144, 2, 1, ("gemv_f32", 1)), (5, 6144, 3, 1, ("gemv", 1)), (5, 12288, 1, 1, ("gemv_f32", 1)),
-            (5, 12320, 1, 1, ("gemv", 1)), (512, 40960, 1, 1, ("gemv", 1)), (16384, 256, 1, 1, ("gemv_f32", 1)),
+            (5, 6144, 2, 1, ("gemv_f32", 1)), (5, 6144, 3, 1, ("gemv", 1)), (5, 9216, 1, 1, ("gemv_f32", 1)),
+            (5, 9248, 1, 1, ("gemv", 1)), (512, 40960, 1, 1, ("gemv", 1)), (16384, 256, 1, 1, ("gemv_f32", 1)),
             (16388, 256, 1, 1, ("gemv", 1)), (3072, 6144, 1, 1, ("gemv_f32", 1)), (4096, 6144, 1, 1, ("gemv", 1)),
             (32000, 4096, 1, 1, ("gemv", 1)), (4096, 11008, 1, 1, ("gemv", 1)), (73448, 2048, 1, 1, ("gemv", 1)),
             (6144, 2048, 16, 1, ("small_f32", 4)), (6144, 2048, 32, 1, ("small", 4)), (12288, 2048, 8, 1, ("small", 2)),

@@ -31,12 +31,12 @@ def _same(a, b, wild):
 
 
 # the last three are past the fused kernel's range
-_TWO_LAUNCHES = [(3, 6144, 5), (7, 3072, 5), (5, 12320, 1)]
+_TWO_LAUNCHES = [(3, 6144, 5), (7, 3072, 5), (5, 9248, 1)]
 
 
 @pytest.mark.parametrize("N,K,M", [(64, 1024, 1), (1001, 1024, 5), (512, 2048, 1), (2051, 2048, 3), (2048, 4096, 2),
                                    (1023, 6144, 1), (2048, 512, 5), (1024, 64, 4), (5, 32, 1), (7, 6144, 2),
-                                   (9, 4096, 3), (7, 3072, 4), (5, 12288, 1)] + _TWO_LAUNCHES)
+                                   (9, 4096, 3), (7, 3072, 4), (5, 9216, 1)] + _TWO_LAUNCHES)
 @pytest.mark.parametrize("variant", [0, 1])
 @pytest.mark.parametrize("wild", [False, True])
 def test_fused_gemv_equals_two_launches(vxm_ctx, orc, N, K, M, variant, wild):

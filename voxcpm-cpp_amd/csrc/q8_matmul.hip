@@ -2190,17 +2190,17 @@ static bool use_mfma(const vxm_ctx *ctx, int64_t M) {
 }
 
 // The fused GEMV's range, while quantizing costs less than the launch saved.  A workgroup
-// quantizes M K values one after another (0.15 us per 1024, before its products): at most
-// 12288, whatever the grid (us a call, fused against two launches: 64 x 6144 at 2 rows 5.1 / 6.4,
-// at 3 rows 6.7 / 6.2; 512 x 4096 at 3 rows 5.5 / 6.4, at 4 rows 6.6 / 6.3; one row of 320 x 12288
-// 7.6 / 7.9, of 256 x 16384 9.3 / 9.1, of 512 x 40960 20.5 / 17.6).  All workgroups together: up
-// to 5 M values for one row (20480 x 2048 8.0 / 8.6, 3072 x 6144 4.7 M 5.9 / 6.3; 4096 x 6144 6.3
-// M 6.9 / 6.8, 5120 x 5120 6.6 M 8.1 / 6.5, 4096 x 11008 14.1 / 10.8), 4 M for more (4096 x 2048
-// at 4 rows 6.4 / 6.5, 6144 x 2048 at 2 rows 3.1 M 5.1 / 6.2, at 3 rows 4.7 M 6.4 / 6.3), 2.5 M
-// where a workgroup has 16 weight rows (K = 1024: 8192 at 5 rows 7.5 / 7.9, 12288 at 4 rows 3.1 M
-// 8.1 / 7.7).  And 16 workgroups per CU, past which each adds its start (32768 x 256, 32 per CU,
-// 8.3 / 7.9; 16384 x 256 5.1 / 6.9).
-constexpr int kGemvF32MaxRows = 5, kGemvF32MaxWgValues = 12288, kGemvF32MaxWgsPerCu = 16;
+// quantizes M K values one after another (0.15 us per 1024, before its products): rows of at
+// most 9216 and 12288 in all, whatever the grid (us a call, fused against two launches: 64 x
+// 6144 at 2 rows 5.1 / 6.4, at 3 rows 6.7 / 6.2; 512 x 4096 at 3 rows 5.5 / 6.4, at 4 rows 6.6 /
+// 6.3; one row of 2048 x 9216 6.6 / 7.0, of 2048 x 10240 8.0 / 7.3, of 512 x 40960 20.5 / 17.6).
+// All workgroups together: up to 5 M values for one row (20480 x 2048 8.0 / 8.6, 3072 x 6144
+// 4.7 M 5.9 / 6.3; 4096 x 6144 6.3 M 6.9 / 6.8, 5120 x 5120 6.6 M 8.1 / 6.5), 4 M for more (4096 x
+// 2048 at 4 rows 6.4 / 6.5, 6144 x 2048 at 2 rows 3.1 M 5.1 / 6.2, at 3 rows 4.7 M 6.4 / 6.3),
+// 2.5 M where a workgroup has 16 weight rows (K = 1024: 8192 at 5 rows 7.5 / 7.9, 12288 at 4 rows
+// 3.1 M 8.1 / 7.7).  And 16 workgroups per CU, past which each adds its start (32768 x 256, 32
+// per CU, 8.3 / 7.9; 16384 x 256 5.1 / 6.9).
+constexpr int kGemvF32MaxRows = 5, kGemvF32MaxK = 9216, kGemvF32MaxWgValues = 12288, kGemvF32MaxWgsPerCu = 16;
 constexpr int64_t kGemvF32MaxValues1 = 5 << 20, kGemvF32MaxValues = 4 << 20, kGemvF32MaxValuesK1024 = 5 << 19;
 
 template <int C, int R>
@@ -2217,7 +2217,8 @@ static void launch_gemv_f32_c(vxm_ctx *ctx, const vxm_weight *w, const float *x,
 
 static bool gemv_f32_takes(const vxm_ctx *ctx, const vxm_weight *w, int64_t M) {
     const int64_t K = w->k;
-    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || M * K > kGemvF32MaxWgValues) return false;
+    if (M <= 0 || M > kGemvF32MaxRows || use_mfma(ctx, M) || K > kGemvF32MaxK || M * K > kGemvF32MaxWgValues)
+        return false;
     const int c = w->dg ? (int)(K / 1024) : 0;
     const int64_t wg_rows = c == 1 ? 16 : c == 2 ? 8 : 4;   // rows of a workgroup: 4 waves of R
     const int64_t wgs = (w->n + wg_rows - 1) / wg_rows;
