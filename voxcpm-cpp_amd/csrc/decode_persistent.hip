@@ -206,19 +206,12 @@ struct Shape {
     static_assert(kAttSplitMax * (HD + 2) <= BIG && HD + 2 <= kAttpWords, "chunk partials fit the score space");
 };
 
-// workgroup that runs the attention of query head h: the heads of one kv
-// group land on workgroups of one XCD (dispatch is round-robin over the 8
-// XCDs), so the group's K/V rows are shared through that XCD's L2.
-template <class S>
-__device__ __forceinline__ int attn_wg(int h) { return (h % S::QPK) * 8 + h / S::QPK; }
-
 // Workgroup of chunk c of query head h: (kv group g, chunk c) is combination
-// k = c * NKV + g, whose QPK heads share one XCD (x = k % 8) and so read the
-// chunk's K/V rows through one L2; chunk 0 is attn_wg(h).  Injective over
-// h < NH, c < kAttSplitMax: workgroup (sb * QPK + h % QPK) * 8 + x with
-// sb = k / 8.
+// k = c * NKV + g, whose QPK heads share one XCD (x = k % 8; dispatch is round-robin
+// over the 8 XCDs) and so read the chunk's K/V rows through one L2.  Injective over
+// h < NH, c < kAttSplitMax: workgroup (sb * QPK + h % QPK) * 8 + x with sb = k / 8.
 template <class S>
-__device__ __forceinline__ int attn_wg_chunk(int h, int c) {
+__host__ __device__ constexpr int attn_wg(int h, int c) {
     const int k = c * S::NKV + h / S::QPK;
     return ((k / 8) * S::QPK + h % S::QPK) * 8 + k % 8;
 }
@@ -226,10 +219,27 @@ __device__ __forceinline__ int attn_wg_chunk(int h, int c) {
 // Its inverse: the query head that workgroup wg attends for with n chunks per head, and
 // the chunk; -1 for a workgroup without one.
 template <class S>
-__device__ __forceinline__ int attn_head_of(int wg, int n, int &chunk) {
+__host__ __device__ constexpr int attn_head_of(int wg, int n, int &chunk) {
     const int sb = wg / 8 / S::QPK, k = sb * 8 + wg % 8;
     chunk = k / S::NKV;
     return chunk < n ? (k % S::NKV) * S::QPK + wg / 8 % S::QPK : -1;
+}
+
+// Every workgroup with a head has one that maps to it, and every head and chunk its own.
+template <class S>
+constexpr bool attn_maps_invert() {
+    for (int n = 1; n <= kAttSplitMax; n++) {
+        int found = 0;
+        for (int wg = 0; wg < kG; wg++) {
+            int c = 0;
+            const int h = attn_head_of<S>(wg, n, c);
+            if (h < 0) continue;
+            if (h >= S::NH || attn_wg<S>(h, c) != wg) return false;
+            found++;
+        }
+        if (found != n * S::NH) return false;
+    }
+    return true;
 }
 
 __device__ __forceinline__ uint32_t make_tag(uint32_t epoch, int layer, int phase) {
@@ -1661,6 +1671,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_decode_persistent(vxm_pparams p
 // host side
 // ---------------------------------------------------------------------------
 using ShapeTslm = Shape<2048, 16, 2, 128, 6144>;
+static_assert(attn_maps_invert<ShapeTslm>(), "a workgroup's head and the head's workgroup");
 
 struct vxm_persistent_state {
     void *base = nullptr;
