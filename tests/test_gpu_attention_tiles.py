@@ -1,7 +1,7 @@
 """The MFMA attention at the edges of its query tiles (32), key blocks (32), rounds (128 keys) and
 head pairs, through a block: causal behind an existing context, and scores whose row max keeps
 rising over the keys.  Fewer queries than a tile take the scalar kernel, here with long contexts
-and with a value row that overflows the f16 cache."""
+and caches and with value rows of infinities and NaN."""
 import numpy as np
 import pytest
 
@@ -98,5 +98,32 @@ def test_overflowing_value_row_reaches_no_earlier_token(vxm_ctx, orc, M, pos, hd
     assert np.isfinite(ys[0]).all()
     assert np.isinf(kv.download(0)[1].view(np.float16)[:, pos + M - 1, 0]).all()
     assert np.array_equal(ys[0][:-1], ys[1][:-1])
+    kv.free()
+    model.free()
+
+
+# past 40624 rows (64 dims) the scalar kernel's score buffer holds no more than the call's own
+# keys; a call with more of them takes the MFMA kernel
+@pytest.mark.parametrize("M,pos,cap", [(5, 300, 20000), (1, 98, 40624), (31, 98, 40624), (31, 98, 40625), (2, 127, 45000),
+                                       (31, 1000, 45000), (5, 40800, 45000)])
+def test_few_queries_in_a_long_cache(vxm_ctx, orc, M, pos, cap):
+    import vxm
+
+    rng = np.random.default_rng(M + pos + cap)
+    H, nh, nkv, hd, F = 256, 4, 2, 64, 256
+    lw = rand_layer(orc, rng, H, nh, nkv, hd, F)
+    c = cfg_dict(H, 1, nh, nkv, hd, F)
+    k = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    v = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    x = rng.normal(0, 1, (M, H)).astype(np.float32)
+    model = vxm.MiniCPM4(vxm_ctx, c, [lw])
+    kv = vxm.KVCache(vxm_ctx, 1, nkv, hd, cap)
+    kv.upload(0, k, v)
+    xd = _dev(x)
+    model.block(kv, 0, xd, pos)
+    vxm_ctx.sync()
+    y = xd.cpu().numpy().astype(np.float64)
+    ref = orc.minicpm4_block(orc_cfg(orc, c), to_orc(orc, lw), x, k.reshape(-1).copy(), v.reshape(-1).copy(), cap, pos, 0)
+    assert np.linalg.norm(y - ref) <= 5e-3 * np.linalg.norm(ref)
     kv.free()
     model.free()

@@ -664,6 +664,9 @@ static void launch_attention_mfma(vxm_ctx *ctx, const float *q, const uint16_t *
                            (int)M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
 }
 
+// k_attention's dynamic LDS: a workgroup's 160 KB less its static arrays.
+constexpr size_t kAttnMaxLds = 160 * 1024 - 64;
+
 int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t *vc, float *out,
                          int64_t M, int nh, int nkv, int hd, int cap, int64_t seg_stride, int S, int kv_base,
                          int causal, int8_t *xq, uint16_t *xd, int variant) {
@@ -672,11 +675,16 @@ int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "attention: head_dim %d / heads %d,%d unsupported", hd, nh, nkv);
     // the MFMA kernel: the queries of a single segment, from a tile of them.  Fewer keep
     // k_attention although it is slower over a long context (16 heads of 128, 24 queries over
-    // 474 keys: 23.5 against 14.7 us): it reads only the keys that a query sees, so a cache row
+    // 474 keys: 18.6 against 13.0 us): it reads only the keys that a query sees, so a cache row
     // of infinities or NaN reaches no query before it, and its queries and probabilities stay
-    // fp32 (a BF16 query past f16's range stays finite).
+    // fp32 (a BF16 query past f16's range stays finite).  Its score buffer holds the capacity;
+    // in a cache past that limit, the keys of the call, and past those the MFMA kernel runs.
     const int64_t span = causal ? kv_base + M : M;
-    if (S == M && M >= AQ && span <= cap && (hd == 128 || hd == 64)) {
+    const bool tiles = S == M && span <= cap && (hd == 128 || hd == 64);
+    const bool few = tiles && M >= 2 && M < AQ && span > 128;
+    size_t lds = (size_t)(hd + cap + 256) * sizeof(float);
+    if (few && lds > kAttnMaxLds) lds = (size_t)(hd + span + 256) * sizeof(float);
+    if (tiles && (M >= AQ || (few && lds > kAttnMaxLds))) {
         if (hd == 128)
             launch_attention_mfma<128>(ctx, q, kc, vc, out, M, nh, nkv, cap, kv_base, causal, xq, xd, variant);
         else
@@ -684,8 +692,7 @@ int vxm_launch_attention(vxm_ctx *ctx, const float *q, const uint16_t *kc, const
         VXM_CHECK_LAUNCH(ctx);
         return VXM_OK;
     }
-    const size_t lds = (size_t)(hd + cap + 256) * sizeof(float);
-    if (lds > 160 * 1024)
+    if (lds > kAttnMaxLds)
         return vxm_fail(ctx, VXM_ERR_INVALID_ARG, "attention: capacity %d exceeds the LDS score buffer", cap);
     // 16-byte key loads need whole 16-byte rows and bases (the caches and the workspace
     // are 16-byte aligned, their heads and segments whole rows apart)
