@@ -127,3 +127,38 @@ def test_few_queries_in_a_long_cache(vxm_ctx, orc, M, pos, cap):
     assert np.linalg.norm(y - ref) <= 5e-3 * np.linalg.norm(ref)
     kv.free()
     model.free()
+
+
+def test_nan_output_quantizes_as_by_itself(vxm_ctx, orc):
+    """Under the reference's rounding rule a NaN value quantizes to 0 in k_quantize_q8_0; so it does
+    where the attention of few queries writes the Q8_0 rows: a value dim that holds a NaN gives what
+    one of zeros gives."""
+    import vxm
+
+    rng = np.random.default_rng(17)
+    H, nh, nkv, hd, F, cap, M, pos, dim = 256, 4, 2, 128, 256, 128, 5, 60, 37
+    lw = rand_layer(orc, rng, H, nh, nkv, hd, F)
+    wv = rng.normal(0, 0.02, (nkv * hd, H)).astype(np.float32)
+    wv[dim] = 0
+    lw["v_proj"] = orc.quantize_rows(wv, orc.QUANT_REF)
+    k = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    v = orc.fp32_to_fp16_bits(orc.bf16_round(rng.normal(0, 1, (nkv, cap, hd)).astype(np.float32)))
+    v[0, :, dim] = 0
+    x = rng.normal(0, 1, (M, H)).astype(np.float32)
+    model = vxm.MiniCPM4(vxm_ctx, cfg_dict(H, 1, nh, nkv, hd, F), [lw])
+    kv = vxm.KVCache(vxm_ctx, 1, nkv, hd, cap)
+    ys = []
+    try:
+        vxm_ctx.set_quant_variant(vxm.QUANT_REF)
+        for bits in (0, 0x7E00):
+            v[0, 3, dim] = bits
+            kv.upload(0, k, v)
+            xd = _dev(x)
+            model.block(kv, 0, xd, pos)
+            vxm_ctx.sync()
+            ys.append(xd.cpu().numpy())
+    finally:
+        vxm_ctx.set_quant_variant(vxm.QUANT_X86)
+    assert np.isfinite(ys[0]).all() and np.array_equal(ys[0], ys[1])
+    kv.free()
+    model.free()

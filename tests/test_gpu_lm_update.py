@@ -135,6 +135,26 @@ def _sync_caches(kv, lm):
         lm["v"][l][...] = v
 
 
+def test_locenc_nan_in_the_patch(vxm_ctx, orc):
+    """Under the reference's rounding rule a NaN quantizes to 0, also where the sequence's assembly
+    quantizes the patch itself: a NaN in it gives what a zero gives."""
+    import vxm
+
+    cfg, w, _, _ = make_locenc(orc, 47)
+    enc = vxm.LocEnc(vxm_ctx, cfg, w)
+    x = np.random.default_rng(57).normal(0, 1, (4, 64)).astype(np.float32)
+    outs = []
+    try:
+        vxm_ctx.set_quant_variant(vxm.QUANT_REF)
+        for v in (0.0, np.nan):
+            x[1, 40] = v
+            outs.append(_np(enc.forward(_dev(x))).copy())
+    finally:
+        vxm_ctx.set_quant_variant(vxm.QUANT_X86)
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
+    enc.free()
+
+
 def _build_update(vxm, vxm_ctx, orc, seed, with_fsq, dims):
     enc, tslm, ralm, pw = make_lm_update(orc, seed, with_fsq=with_fsq, **dims["sizes"])
     ecfg, ew, eow, eocfg = enc

@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void k_locenc_assemble(float *__restrict__ seq
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; e++) v[e] = x[(int64_t)(row - off) * feat + 8 * threadIdx.x + e];
-            quant_block_4lanes(v, variant, q + 8 * threadIdx.x, qd + threadIdx.x / 4, (threadIdx.x & 3) == 0);
+            quant_block_4lanes(v, variant, q + 8 * threadIdx.x, qd + threadIdx.x / 4, (threadIdx.x & 3) == 0, true, true);
         }
         __syncthreads();
     }

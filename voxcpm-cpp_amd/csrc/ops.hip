@@ -369,7 +369,7 @@ __global__ __launch_bounds__(256) void k_attention(const float *__restrict__ q, 
         const float4 a = *(const float4 *)(sq + 8 * threadIdx.x), b = *(const float4 *)(sq + 8 * threadIdx.x + 4);
         const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         const int64_t e = (int64_t)t * nh * hd + h * hd + 8 * threadIdx.x;
-        quant_block_4lanes(v, variant, xq + e, xd + e / 32, (threadIdx.x & 3) == 0);
+        quant_block_4lanes(v, variant, xq + e, xd + e / 32, (threadIdx.x & 3) == 0, true, true);
     }
 }
 

@@ -125,9 +125,11 @@ __device__ __forceinline__ float vxm_quad_max(float v) {
 // Q8_0 of one 32-value block held 8 per lane by four consecutive lanes (lane & 3
 // = part) with the x86 rule (id = 127/amax, round half even) or the _ref rule;
 // the lane with write_d set stores d.  write = false: compute (every lane of the
-// four takes part in the amax exchange) but store nothing.
-__device__ __forceinline__ void quant_block_4lanes(const float v[8], int variant, int8_t *q8,
-                                                   uint16_t *dout, bool write_d, bool write = true) {
+// four takes part in the amax exchange) but store nothing.  nan_zero: in the place of
+// k_quantize_q8_0, which does not clamp under the _ref rule: a NaN is 0 there, not -128
+// (no finite quotient leaves the range).
+__device__ __forceinline__ void quant_block_4lanes(const float v[8], int variant, int8_t *q8, uint16_t *dout,
+                                                   bool write_d, bool write = true, bool nan_zero = false) {
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
@@ -140,7 +142,7 @@ __device__ __forceinline__ void quant_block_4lanes(const float v[8], int variant
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         float q = variant == VXM_QUANT_X86 ? rintf(v[i] * id) : roundf(v[i] * id);
-        q = fminf(fmaxf(q, -128.0f), 127.0f);
+        if (variant == VXM_QUANT_X86 || !nan_zero) q = fminf(fmaxf(q, -128.0f), 127.0f);
         const uint32_t b = (uint32_t)(uint8_t)(int8_t)(int)q;
         if (i < 4) lo |= b << (8 * i);
         else hi |= b << (8 * (i - 4));
