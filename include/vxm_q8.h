@@ -168,10 +168,12 @@ size_t vxm_noalloc_scratch_bytes(void);
 /* Test hook, host only: the kernel that a product of an n x k weight and m rows in
  * 16-byte aligned buffers apart from each other runs on a device of n_cu CUs, and its
  * K splits: vxm_mul_mat_q8_0_q8_0's, vxm_mul_mat_q8_0's, or a model block's, whose
- * next kernel adds the small-M GEMM's slices. */
+ * next kernel adds the small-M GEMM's slices; or a block's gate/up with SwiGLU and
+ * Q8_0 in its epilogue (NONE: the block runs them apart). */
 #define VXM_ROWS_Q8 0
 #define VXM_ROWS_F32 1
 #define VXM_ROWS_BLOCK 2
+#define VXM_ROWS_GATE_UP 3
 #define VXM_KERNEL_NONE 0      /* refused: operands of 2 GiB and more */
 #define VXM_KERNEL_GEMV 1      /* weight-streaming GEMV */
 #define VXM_KERNEL_GEMV_F32 2  /* ... that quantizes its rows itself */

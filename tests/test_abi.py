@@ -124,6 +124,11 @@ def test_mul_mat_plans():
             (8192, 768, 49, 2, ("tile", 1)), (12288, 2048, 24, 2, ("tile", 1)), (2048, 6144, 77, 2, ("small", 4)),
             (2560, 2048, 128, 2, ("small", 4)), (2560, 4096, 96, 2, ("small", 4)), (2560, 4096, 97, 2, ("tile", 3)),
             (2048, 11008, 77, 2, ("tile", 4)), (4096, 11008, 128, 2, ("tile", 2)),
+            # a block's gate/up with SwiGLU in the epilogue; past 32-bit offsets the small-M GEMM up to one
+            # row tile of its waves, above it refused as every tiled product of that size
+            (12288, 2048, 32, 3, ("small", 1)), (12288, 2048, 33, 3, ("tile", 1)), (4096, 512, 48, 3, ("small", 1)),
+            (4096, 512, 49, 3, ("tile", 1)), (1048512, 2048, 33, 3, ("small", 1)), (1048512, 2048, 64, 3, ("small", 1)),
+            (1048512, 2048, 65, 3, ("none", 1)), (1048512, 2048, 128, 3, ("none", 1)),
             # two row tiles in three wave groups quantize in a launch of their own
             (1344, 6144, 16, 1, ("small_f32", 8)), (1344, 6144, 17, 1, ("small", 8)), (64, 768, 20, 1, ("tile", 1))]:
         assert plan(n, k, m, rows=rows) == want, (n, k, m, rows, plan(n, k, m, rows=rows))

@@ -2091,31 +2091,39 @@ int vxm_launch_mul_mat_parts(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 // The gate/up projection with SwiGLU and the Q8_0 of its output fused into the
 // GEMM's epilogue (rows of w interleave gate n = row 2n and up n = row 2n+1): sq
 // [M][N/2] and sd [M][N/64] are the down projection's input.  The small-M kernel
-// takes M <= 32 (48 where K < 768), the tile GEMM larger M when its plan needs no K split.  Returns
-// false without launching otherwise (and under PATH_MFMA_TILED, which keeps the
-// unfused GEMM + k_swiglu_quant as the reference of the fused epilogue).
+// takes M <= 32 (48 where K < 768; 64 of a product past the tile GEMM's offsets), the tile
+// GEMM larger M when its plan needs no K split.  Returns false without launching
+// otherwise (and under PATH_MFMA_TILED, which keeps the unfused GEMM + k_swiglu_quant as
+// the reference of the fused epilogue).
 // (us, small-M / tile: 12288 x 2048 at 24 rows 11.4 / 11.4, at 33 rows 14.4 / 11.5; 8192 x 1024 at
 // 48 rows 9.1 / 8.4, 4096 x 768 8.4 / 7.6, 4096 x 512 6.0 / 6.4)
 constexpr int kSmallGateUpRows = 32, kSmallGateUpRowsShortK = 48, kSmallGateUpShortK = 768;
 
+// The kernel of the fused form, with its plan, or VXM_KERNEL_NONE.
+static int gate_up_kernel(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
+                          SmallPlan &sp, GemmPlan &p) {
+    const int64_t N = w->n, K = w->k;
+    const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
+    if (!mfma || M <= 0 || N % 64) return VXM_KERNEL_NONE;
+    const int small_rows = K < kSmallGateUpShortK ? kSmallGateUpRowsShortK : kSmallGateUpRows;
+    const bool fits = gemm_fits(M, N, K);
+    // unsplit: each workgroup holds whole 32-pair blocks over all of K
+    if (M <= (fits ? small_rows : VXM_SMALL_TILE_ROWS) && small_plan(ctx, M, N, K, 1, sp)) return VXM_KERNEL_SMALL;
+    return fits && tile_plan(ctx, w, xq, xd, M, 0, p) && p.splits == 1 ? VXM_KERNEL_TILE : VXM_KERNEL_NONE;
+}
+
 bool vxm_launch_gate_up_swiglu(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq, const uint16_t *xd, int64_t M,
                                int8_t *sq, uint16_t *sd, int variant, int *rc) {
     *rc = VXM_OK;
-    const int64_t N = w->n, K = w->k;
-    const bool mfma = ctx->path == VXM_PATH_MFMA || (ctx->path == VXM_PATH_AUTO && M >= kSmallPartsMinRows);
-    if (!mfma || M <= 0 || N % 64) return false;
     SmallPlan sp;
-    const int small_rows = K < kSmallGateUpShortK ? kSmallGateUpRowsShortK : kSmallGateUpRows;
-    if ((M <= small_rows || !gemm_fits(M, N, K)) && small_plan(ctx, M, N, K, 1, sp)) {
-        // unsplit: each workgroup holds whole 32-pair blocks over all of K
+    GemmPlan p;
+    const int kernel = gate_up_kernel(ctx, w, xq, xd, M, sp, p);
+    if (kernel == VXM_KERNEL_NONE) return false;
+    if (kernel == VXM_KERNEL_SMALL)
         launch_small(ctx, w, xq, xd, M, nullptr, sp, sq, sd, variant);
-    } else {
-        GemmPlan p;
-        if (!tile_plan(ctx, w, xq, xd, M, 0, p) || p.splits != 1) return false;
-        if ((*rc = launch_gemm_tile<false>(ctx, w, xq, xd, M, nullptr, nullptr, p, nullptr, nullptr, nullptr, sq, sd,
-                                           variant)))
-            return true;
-    }
+    else if ((*rc = launch_gemm_tile<false>(ctx, w, xq, xd, M, nullptr, nullptr, p, nullptr, nullptr, nullptr, sq, sd,
+                                            variant)))
+        return true;
     if (hipGetLastError() != hipSuccess) *rc = vxm_fail(ctx, VXM_ERR_BACKEND, "gate/up + SwiGLU launch failed");
     return true;
 }
@@ -2320,7 +2328,7 @@ static int launch_block_dots(vxm_ctx *ctx, const vxm_weight *w, const int8_t *xq
 extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int64_t k, int64_t m, int32_t rows,
                                      int32_t *kernel, int32_t *splits) {
     if (!kernel || !splits || n_cu <= 0 || n <= 0 || n > INT32_MAX || k <= 0 || k % VXM_QK || m <= 0 ||
-        path < VXM_PATH_AUTO || path > VXM_PATH_MFMA_TILED || rows < VXM_ROWS_Q8 || rows > VXM_ROWS_BLOCK)
+        path < VXM_PATH_AUTO || path > VXM_PATH_MFMA_TILED || rows < VXM_ROWS_Q8 || rows > VXM_ROWS_GATE_UP)
         return VXM_ERR_INVALID_ARG;
     vxm_ctx ctx;
     ctx.n_cu = n_cu;
@@ -2332,7 +2340,10 @@ extern "C" int vxm_host_mul_mat_plan(int32_t n_cu, int32_t path, int64_t n, int6
     w.dt = k % 256 == 0 ? (uint16_t *)256 : nullptr;
     SmallPlan sp;
     *splits = 1;
-    if (rows == VXM_ROWS_F32 && gemv_f32_takes(&ctx, &w, m)) {
+    if (rows == VXM_ROWS_GATE_UP) {
+        GemmPlan p;
+        *kernel = gate_up_kernel(&ctx, &w, nullptr, nullptr, m, sp, p);
+    } else if (rows == VXM_ROWS_F32 && gemv_f32_takes(&ctx, &w, m)) {
         *kernel = VXM_KERNEL_GEMV_F32;
     } else if (rows == VXM_ROWS_BLOCK && parts_takes(&ctx, &w, nullptr, nullptr, m, VXM_MAX_PARTS, sp)) {
         *kernel = VXM_KERNEL_SMALL;

@@ -657,7 +657,7 @@ def host_quantize_q8_0(x):
 KERNELS = ("none", "gemv", "gemv_f32", "small", "small_f32", "tile", "staged")
 
 
-ROWS_Q8, ROWS_F32, ROWS_BLOCK = 0, 1, 2
+ROWS_Q8, ROWS_F32, ROWS_BLOCK, ROWS_GATE_UP = 0, 1, 2, 3
 
 
 def host_mul_mat_plan(n, k, m, path=PATH_AUTO, rows=ROWS_F32, n_cu=256):
