@@ -152,9 +152,11 @@ int vxm_stream_read(vxm_ctx *ctx, int32_t n, const void *const *ranges_dev, cons
 int64_t vxm_stream_read_sink_words(int32_t n, const int64_t *bytes);
 /* vxm_mul_mat_q8_0 without any allocation: no counterpart in the reference.
  * For callers that cannot allocate device memory (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * kernels, plans and results as vxm_mul_mat_q8_0; the quantized activation
- * and the K-split partials live in a fixed device array of
+ * capture, tight serving loops, harnesses that forbid hipMalloc).  The results
+ * of vxm_mul_mat_q8_0 bit for bit, with its K splits, always from a quantization
+ * launch and the kernel that vxm_mul_mat_q8_0_q8_0 picks (vxm_mul_mat_q8_0
+ * quantizes up to 32 rows inside its GEMV or small-M GEMM); the quantized
+ * activation and the K-split partials live in a fixed device array of
  * vxm_noalloc_scratch_bytes() per device (48 MiB 64 KiB), held until the
  * process ends.  A product whose quantized activation exceeds 32 MiB, or whose
  * K-split plan needs more than the array's 16 MiB of partial words (for

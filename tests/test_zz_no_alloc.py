@@ -1,8 +1,9 @@
 """The allocation-free matmul (vxm_mul_mat_q8_0_noalloc) against the allocating
 one (vxm_mul_mat_q8_0) through the C ABI.
 
-Both run the same kernels with the same plans, so the outputs must be equal bit
-for bit; each is also held to the matmul bar (1e-3 rel / 1e-4 abs of the
+The first always quantizes in a launch of its own, the second inside the product's
+launch for a few rows; the products and K splits are the same, so the outputs must
+be equal bit for bit; each is also held to the matmul bar (1e-3 rel / 1e-4 abs of the
 oracle's fp64 sum).  Every case makes two calls in a row on the shared scratch
 array, the second with a smaller input, with no synchronisation in between.
 """

@@ -2428,9 +2428,11 @@ extern "C" int vxm_block_dots_q8_0(vxm_ctx *ctx, const vxm_weight *w, const int8
 }
 
 // ---- the allocation-free matmul ---------------------------------------------
-// vxm_mul_mat_q8_0_noalloc runs the kernels of vxm_mul_mat_q8_0, with the same
-// plans, but takes every buffer beyond x and y from `scratch`, a file-scope
-// device array that the code object carries: no call allocates.  Layout:
+// vxm_mul_mat_q8_0_noalloc quantizes in a launch of its own and runs the kernel and
+// K splits of vxm_mul_mat_q8_0_q8_0, which give vxm_mul_mat_q8_0's bits also where that
+// entry quantizes inside the product's launch.  Every buffer beyond x and y is in
+// `scratch`, a file-scope device array that the code object carries: no call
+// allocates.  Layout:
 //   [0, kScrCnt - 256)           per-tile arrival counters of the tiled GEMM's
 //                                K splits (zeroed by each call that splits)
 //   [kScrCnt - 256, kScrCnt)     the split tag word (advanced on the device
