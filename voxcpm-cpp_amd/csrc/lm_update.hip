@@ -71,7 +71,7 @@ struct vxm_lm_update {
 // xh != nullptr: the projection's rows, formed by launches of their own.  Else the
 // workgroup of a row quantizes its x (feat values) and forms the projection itself:
 // for a patch's few rows of 64 values three dependent launches (quantization,
-// product, this one) are mostly gaps (an encoder call of 5 rows 303 -> 300 us, of 13 rows 354 -> 349).
+// product, this one) are mostly gaps (an encoder call of 5 rows 293.5 -> 290.7 us, of 13 rows 350.5 -> 345.8).
 __global__ __launch_bounds__(256) void k_locenc_assemble(float *__restrict__ seq, const float *__restrict__ special,
                                                          const float *__restrict__ xh, const float *__restrict__ x,
                                                          const int8_t *__restrict__ wq,
@@ -330,7 +330,7 @@ extern "C" int vxm_locenc_forward(vxm_locenc *m, const float *x_dev, int32_t P, 
     const int64_t rows = off ? 1 : S;
     if (persistent) {
         // all blocks in one launch, the returned rows' final norm included (a launch of its own
-        // for it took an encoder call of 5 rows from 289.7 to 295.5 us); seq then holds the last
+        // for it takes an encoder call of 5 rows from 290.7 to 294.9 us); seq then holds the last
         // block's output.  One row tile only, the form built for it; the norm writes pairs, so an
         // output that is not 8-byte aligned keeps its launch too.
         vxm_lfinal fin{};
